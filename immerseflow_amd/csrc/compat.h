@@ -22,6 +22,8 @@ struct CompatCase {
     double *uf = nullptr, *vf = nullptr, *vx = nullptr, *vy = nullptr;
     double *part = nullptr, *scal = nullptr;
     double *h_out = nullptr;
+    bool one_ad = false, one_ppe = false;  // the one-workgroup forms fit (compat.hip)
+    size_t lds_ad = 0, lds_ppe = 0;
 
     ~CompatCase();
     if_status create(const if_case_desc &d);

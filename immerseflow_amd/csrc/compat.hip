@@ -251,6 +251,432 @@ __global__ void kc_pbc(int nx, int ny, double *p)
 }
 
 // ---------------------------------------------------------------------------
+// One-workgroup forms of ADsolver and PPESolver for grids whose fields fit in
+// the LDS of one CU (the reference's own deck: 52 x 52 cells with ghosts).
+// At this size a pass is waits, not work: launched kernel by kernel, one
+// Poisson iteration took 21 us (four launches, a copy and a host wait for
+// 2,704 cells).  Here the whole call is one launch; an iteration costs its
+// LDS reads, its FP64 arithmetic and one (Poisson) or four (AD) barriers.
+//
+// Wave w owns the cells id = 512 w + lane + 64 q, q = 0..7: exactly the cells
+// of block w of reduce6's first pass, so that pass's fold needs no LDS and no
+// barrier (h = 128 and 64 fall on a lane's own cells, h = 32..1 are lane
+// exchanges), and every sum has the bits of the launch-by-launch form.
+//
+// LDS is indexed from its array by integer offsets, never through pointers
+// chosen at run time: those become flat accesses, whose base the compiler may
+// place below the array (the south neighbour of a first-row cell, 64 q cells
+// on in the immediate offset), outside the LDS aperture the hardware tests.
+// ---------------------------------------------------------------------------
+constexpr int kOneCells = 8192;       // 16 waves x 512 cells
+constexpr int kOneQ = 8;              // cells per lane
+constexpr int kOneIters = 16384;      // Poisson iterations per launch: bounds a launch to about 10 ms
+constexpr size_t kOneLds = 160 * 1024;
+
+// Lane l's value plus that of lane l ^ h for h = 32, 16, ..: in lane 0 the
+// order of the fold s[t] += s[t + h] (each step adds the same two numbers).
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v)
+{
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, true);
+    return v + __hiloint2double(hi, lo);
+}
+// h = 8, 4, 2, 1 within rows of 16 lanes (row rotations)
+__device__ __forceinline__ double fold16(double v)
+{
+    v = dpp_add<0x128>(v);
+    v = dpp_add<0x124>(v);
+    v = dpp_add<0x122>(v);
+    return dpp_add<0x121>(v);
+}
+__device__ __forceinline__ double fold64(double v)
+{
+    v += __shfl_xor(v, 32, 64);
+    v += __shfl_xor(v, 16, 64);
+    return fold16(v);
+}
+__device__ __forceinline__ double lane0(double v)
+{
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
+// Pass 1 of Reduction over a wave's 512 values: thread t of the reference's
+// block adds val(t) + val(t + 256) (val(t) alone past the end), which are
+// this lane's values q and q + 4.
+__device__ __forceinline__ double fold512(const double (&val)[kOneQ], int id0, int n)
+{
+    double a[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int id = id0 + 64 * q;
+        a[q] = id + 256 < n ? 0.0 + (val[q] + val[q + 4]) : (id < n ? 0.0 + val[q] : 0.0);
+    }
+    return fold64((a[0] + a[2]) + (a[1] + a[3]));
+}
+
+// Pass 2 over at most 16 block sums (the others are zero), in every wave.
+__device__ __forceinline__ double fold_parts(const double *lds, int part, int lane)
+{
+    return lane0(fold16(lane < 16 ? 0.0 + lds[part + lane] : 0.0));
+}
+
+// x / b, correctly rounded, from y = RN(1 / b): q = x y is within one ulp, the
+// remainder x - q b is exact in an FMA, and RN(q + remainder y) is the
+// correctly rounded quotient (P. Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", IBM J. Res. Dev. 34, 1990,
+// theorem 7.2), unless b's mantissa is all ones or an operation leaves the
+// normal range: those take the division (div_special, and the range test).
+// Three operations where the division takes about 25, in a loop that is made
+// of one division per cell.
+__device__ __forceinline__ bool div_special(double b)
+{
+    const unsigned long long m = (unsigned long long)__double_as_longlong(b) & 0xfffffffffffffull;
+    const double a = fabs(b);
+    return m == 0xfffffffffffffull || !(a > 1e-60 && a < 1e60);
+}
+__device__ __forceinline__ double div_by(double x, double b, double y, bool special)
+{
+    const double a = fabs(x);
+    if (special || !((a > 1e-200 && a < 1e200) || a == 0.0)) return x / b;
+    const double q = x * y;
+    return __builtin_fma(__builtin_fma(-q, b, x), y, q);
+}
+
+// Per-lane coefficients of its cells: held in registers (REG, at most 8 waves,
+// 256 registers a lane) or read from the LDS copies of the axis vectors.
+template <bool REG>
+struct OneCoef {
+    double xp[REG ? kOneQ : 1], xm[REG ? kOneQ : 1], yp[REG ? kOneQ : 1], ym[REG ? kOneQ : 1];
+};
+
+// PPESolver's loop (PPESolver.cu:164-195).  Iteration k reads p_k once: the
+// same four products give its residual (the stop test of iteration k) and
+// p_{k+1}, which goes to the other LDS buffer.  The test's sum is complete
+// after the iteration's one barrier; a stop at k stores p_k from registers.
+template <bool REG>
+__global__ __launch_bounds__(REG ? 512 : 1024) void kc_ppe_one(int nx, int ny, const double *vx, const double *vy,
+                                                               double *p, int iter0, int itermax, int most, double tol,
+                                                               double *out)
+{
+    extern __shared__ __align__(16) double lds[];
+    const int n = nx * ny;
+    // offsets in lds: the two iterates from 0 and n; the block sums, [2][16];
+    // !REG: cxp, cxm and cyp, cym
+    const int part = 2 * n, lx = part + 32, ly = lx + 2 * nx;
+    const double *cxp = vx + 5 * nx, *cxm = vx + 6 * nx, *cyp = vy + 5 * ny, *cym = vy + 6 * ny;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int id0 = 512 * w + lane;
+    OneCoef<REG> C;
+    double own[kOneQ], y[kOneQ], ap[REG ? kOneQ : 1];
+    int ij[kOneQ];  // i in the low half, j in the high half
+    unsigned in = 0;
+    bool special = false;
+    if (!REG) {
+        for (int k = threadIdx.x; k < 2 * nx; k += blockDim.x) lds[lx + k] = cxp[k];  // cxp, cxm are adjacent
+        for (int k = threadIdx.x; k < 2 * ny; k += blockDim.x) lds[ly + k] = cyp[k];
+    }
+    if (threadIdx.x < 32) lds[part + threadIdx.x] = 0.0;
+#pragma unroll
+    for (int q = 0; q < kOneQ; q++) {
+        const int id = id0 + 64 * q;
+        own[q] = y[q] = 0.0;
+        ij[q] = 0;
+        if constexpr (REG) C.xp[q] = C.xm[q] = C.yp[q] = C.ym[q] = ap[q] = 0.0;
+        if (id < n) {
+            const int j = id / nx, i = id - j * nx;
+            ij[q] = i | (j << 16);
+            double v = p[id];
+            if (i == 0 || j == 0) v = 100.0;  // set_pressure_BC
+            own[q] = v;
+            lds[id] = v;
+            lds[n + id] = v;
+            if (i > 0 && i < nx - 1 && j > 0 && j < ny - 1) {
+                in |= 1u << q;
+                const double a = -1 * ((cxp[i] + cxm[i]) + (cyp[j] + cym[j]));
+                special = special || div_special(a);
+                y[q] = 1.0 / a;
+                if constexpr (REG) {
+                    C.xp[q] = cxp[i];
+                    C.xm[q] = cxm[i];
+                    C.yp[q] = cyp[j];
+                    C.ym[q] = cym[j];
+                    ap[q] = a;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    double res = 1.0;
+    int k = iter0;
+    bool stopped = k >= itermax;
+    // k - iter0 iterations done; p_k is iterate (k - iter0) & 1
+    while (!stopped) {
+        const int b = ((k - iter0) & 1) * n, nb = n - b;
+        double r[kOneQ], nv[kOneQ];
+#pragma unroll
+        for (int q = 0; q < kOneQ; q++) {
+            r[q] = 0.0;
+            nv[q] = own[q];
+            if (in & (1u << q)) {
+                const int id = b + id0 + 64 * q;
+                double xp, xm, yp, ym, a;
+                if constexpr (REG) {
+                    xp = C.xp[q];
+                    xm = C.xm[q];
+                    yp = C.yp[q];
+                    ym = C.ym[q];
+                    a = ap[q];
+                } else {
+                    const int i = ij[q] & 0xffff, j = ij[q] >> 16;
+                    xp = lds[lx + i];
+                    xm = lds[lx + nx + i];
+                    yp = lds[ly + j];
+                    ym = lds[ly + ny + j];
+                    a = -1 * ((xp + xm) + (yp + ym));
+                }
+                const double e = lds[id + 1] * xp, ww = lds[id - 1] * xm, nn = lds[id + nx] * yp, s = lds[id - nx] * ym;
+                r[q] = own[q] * a + e + ww + nn + s;
+                nv[q] = div_by(-(e + ww + nn + s), a, y[q], special);
+            }
+        }
+        // the next iterate, before the test is known: a stop keeps p_k, which
+        // is in own; the buffer's former contents were last read before the
+        // previous barrier
+#pragma unroll
+        for (int q = 0; q < kOneQ; q++)
+            if (in & (1u << q)) lds[nb + id0 + 64 * q] = nv[q];
+        const double f = fold512(r, id0, n);
+        if (lane == 0) lds[part + 16 * (k & 1) + w] = f;
+        __syncthreads();
+        if (k > iter0) {  // (iter0: nothing done yet, or decided by the launch before)
+            res = fold_parts(lds, part + 16 * (k & 1), lane);
+            if (!(res > tol) || k >= itermax) stopped = true;
+        }
+        if (stopped || k - iter0 >= most) break;
+#pragma unroll
+        for (int q = 0; q < kOneQ; q++) own[q] = nv[q];
+        k++;
+    }
+#pragma unroll
+    for (int q = 0; q < kOneQ; q++)
+        if (id0 + 64 * q < n) p[id0 + 64 * q] = own[q];
+    if (threadIdx.x == 0) {
+        out[0] = res;
+        out[1] = (double)k;
+        out[2] = stopped ? 1.0 : 0.0;
+    }
+}
+
+// ADsolver (ADSolver.cu:268-395) on one workgroup.  u and v live in LDS, in
+// place: a sweep holds its new values in registers until every cell has been
+// read.  The reference's second buffer matters only through its ring, which
+// keeps the values of two iterations ago: those are kept apart (alt) and
+// change places with the ring after each sweep.
+template <bool REG>
+__global__ __launch_bounds__(REG ? 512 : 1024) void kc_ad_one(int nx, int ny, const double *vx, const double *vy,
+                                                              double *u, double *v, double *uf, double *vf, double dt,
+                                                              double w_ad, double tol, int itermax, double *out)
+{
+    extern __shared__ __align__(16) double lds[];
+    const int n = nx * ny, nr = 2 * (nx + ny);
+    // offsets in lds: u and v from 0 and n; the other buffers' rings, [2][nr];
+    // the block sums, [2 fields][16]
+    const int alt = 2 * n, part = alt + 2 * nr;
+    const double *dx = vx, *dy = vy;
+    const double *axp = vx + 2 * nx, *axm = vx + 3 * nx, *px = vx + 4 * nx;
+    const double *ayp = vy + 2 * ny, *aym = vy + 3 * ny, *py = vy + 4 * ny;
+    const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, w = tid >> 6;
+    const int id0 = 512 * w + lane;
+    const int nuf = (nx - 1) * (ny - 2), nvf = (nx - 2) * (ny - 1);
+
+    // Compute_velf (kc_velf's expressions)
+    auto velf = [&]() {
+        for (int id = tid; id < (nuf > nvf ? nuf : nvf); id += nt) {
+            if (id < nuf) {
+                const int j = id / (nx - 1), i = id - j * (nx - 1);
+                const int idc = j * nx + i;
+                uf[id] = 1.0 / (dx[i] + dx[i + 1]) * (lds[idc + nx + 1] * dx[i] + lds[idc + nx] * dx[i + 1]);
+            } else {
+                const int j = id / (nx - 2), i = id - j * (nx - 2);
+                const int idc = j * nx + i;
+                vf[id] = 1.0 / (dy[j + 1] + dy[j]) * (lds[n + idc + nx + 1] * dy[j] + lds[n + idc + 1] * dy[j + 1]);
+            }
+        }
+    };
+    // set_velocity_BC (kc_bc) on both fields
+    auto bc = [&]() {
+        for (int k = tid; k < 2 * (nx + ny - 4); k += nt) {
+            const int c = k >= nx + ny - 4, kk = k - c * (nx + ny - 4);
+            const int o = c * n;
+            const double two = (c ? 0.0 : 1.0) * 2.0;
+            if (kk < ny - 2) {
+                const int j = 1 + kk;
+                const int ww = j * nx, e = nx - 1 + j * nx;
+                const double old_w = lds[o + ww];
+                const double nw = -lds[o + ww + 1] + two, ne = -lds[o + e - 1] + two;
+                lds[o + ww] = nw;
+                lds[o + e] = ne;
+                if (j == 1) lds[o + 0] = -old_w + two;
+                if (j == ny - 2) lds[o + (ny - 1) * nx] = -nw + two;
+                if (j == ny - 2) lds[o + nx - 1 + (ny - 1) * nx] = -ne + two;
+            } else {
+                const int i = 1 + (kk - (ny - 2));
+                const double ns = -lds[o + i + nx] + two;
+                lds[o + i] = ns;
+                lds[o + i + (ny - 1) * nx] = -lds[o + i + (ny - 2) * nx] + two;
+                if (i == nx - 2) lds[o + nx - 1] = -ns + two;
+            }
+        }
+    };
+    // ring index -> cell: south row, north row, west and east columns
+    auto ring = [&](int k) {
+        if (k < nx) return k;
+        if (k < 2 * nx) return (ny - 1) * nx + (k - nx);
+        if (k < 2 * nx + ny - 2) return (k - 2 * nx + 1) * nx;
+        return (k - 2 * nx - (ny - 2) + 1) * nx + nx - 1;
+    };
+    const int nring = 2 * nx + 2 * (ny - 2);
+
+    for (int k = tid; k < n; k += nt) {
+        lds[k] = u[k];
+        lds[n + k] = v[k];
+    }
+    for (int k = tid; k < 2 * nr; k += nt) lds[alt + k] = 0.0;  // fresh scratch (:275-287)
+    if (tid < 32) lds[part + tid] = 0.0;
+    __syncthreads();
+    velf();  // :298, before the BC (stale ghosts)
+    __syncthreads();
+    bc();  // :304
+    __syncthreads();
+
+    // ADSource (kc_source's expressions) of the owned cells, coefficients
+    OneCoef<REG> C;
+    double s[2][kOneQ], y[kOneQ], ap[REG ? kOneQ : 1];
+    int ij[kOneQ];
+    unsigned in = 0;
+    bool special = false;
+#pragma unroll
+    for (int q = 0; q < kOneQ; q++) {
+        const int id = id0 + 64 * q;
+        s[0][q] = s[1][q] = y[q] = 0.0;
+        ij[q] = 0;
+        if constexpr (REG) C.xp[q] = C.xm[q] = C.yp[q] = C.ym[q] = ap[q] = 0.0;
+        if (id >= n) continue;
+        const int j = id / nx, i = id - j * nx;
+        ij[q] = i | (j << 16);
+        if (!(i > 0 && i < nx - 1 && j > 0 && j < ny - 1)) continue;
+        in |= 1u << q;
+        const double dx_i = dx[i], dx_ip1 = dx[i + 1], dx_im1 = dx[i - 1];
+        const double dy_j = dy[j], dy_jp1 = dy[j + 1], dy_jm1 = dy[j - 1];
+        const double ufe = uf[i + (j - 1) * (nx - 1)], ufw = uf[i - 1 + (j - 1) * (nx - 1)];
+        const double vfn = vf[i - 1 + j * (nx - 2)], vfs = vf[i - 1 + (j - 1) * (nx - 2)];
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const int a = c * n;
+            s[c][q] =
+                (lds[a + id] - (dt / dx_i) * 0.5 * (((1 / (dx_i + dx_ip1)) * (lds[a + id + 1] * dx_i + lds[a + id] * dx_ip1) * ufe)
+                                              - ((1 / (dx_i + dx_im1)) * (lds[a + id] * dx_im1 + lds[a + id - 1] * dx_i) * ufw)))
+                - (dt / dy_j) * 0.5 * (((1 / (dy_j + dy_jp1)) * (lds[a + id + nx] * dy_j + lds[a + id] * dy_jp1) * vfn)
+                                       - ((1 / (dy_j + dy_jm1)) * (lds[a + id] * dy_jm1 + lds[a + id - nx] * dy_j) * vfs));
+        }
+        const double d = px[i] + py[j];
+        special = special || div_special(d);
+        y[q] = 1.0 / d;
+        if constexpr (REG) {
+            C.xp[q] = axp[i];
+            C.xm[q] = axm[i];
+            C.yp[q] = ayp[j];
+            C.ym[q] = aym[j];
+            ap[q] = d;
+        }
+    }
+    __syncthreads();  // uf, vf read before the loop rewrites them
+
+    double ures = 1.0, vres = 1.0;
+    int iter = 0;
+    while (ures + vres > tol && iter < itermax) {  // :315
+        bc();                                       // :317
+        __syncthreads();
+        velf();  // :321
+        double nv[2][kOneQ], r[2][kOneQ];
+#pragma unroll
+        for (int q = 0; q < kOneQ; q++) {
+            r[0][q] = r[1][q] = nv[0][q] = nv[1][q] = 0.0;
+            if (!(in & (1u << q))) continue;
+            const int id = id0 + 64 * q;
+            double xp, xm, yp, ym, d;
+            if constexpr (REG) {
+                xp = C.xp[q];
+                xm = C.xm[q];
+                yp = C.yp[q];
+                ym = C.ym[q];
+                d = ap[q];
+            } else {
+                const int i = ij[q] & 0xffff, j = ij[q] >> 16;
+                xp = axp[i];
+                xm = axm[i];
+                yp = ayp[j];
+                ym = aym[j];
+                d = px[i] + py[j];
+            }
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                const int a = c * n;
+                const double t = s[c][q] + xp * lds[a + id + 1] + xm * lds[a + id - 1] + yp * lds[a + id + nx] + ym * lds[a + id - nx];
+                double x = div_by(t, d, y[q], special);
+                if (w_ad != 1.0) x = (1.0 - w_ad) * lds[a + id] + w_ad * x;
+                nv[c][q] = x;
+                r[c][q] = fabs(x - lds[a + id]);
+            }
+        }
+        const double fu = fold512(r[0], id0, n), fv = fold512(r[1], id0, n);
+        if (lane == 0) {
+            lds[part + w] = fu;
+            lds[part + 16 + w] = fv;
+        }
+        __syncthreads();
+        ures = fold_parts(lds, part, lane);  // :350-366
+        vres = fold_parts(lds, part + 16, lane);
+        // the new interior, and the ring of the other buffer (:337 changed
+        // only the old buffer's corner (0,0), from its ghost (0,1))
+#pragma unroll
+        for (int q = 0; q < kOneQ; q++)
+            if (in & (1u << q)) {
+                lds[id0 + 64 * q] = nv[0][q];
+                lds[n + id0 + 64 * q] = nv[1][q];
+            }
+        for (int k = tid; k < 2 * nring; k += nt) {
+            const int c = k >= nring, kk = k - c * nring;
+            const int id = ring(kk);
+            double old = lds[c * n + id];
+            const double a = lds[alt + c * nr + kk];
+            if (kk == 0) old = -lds[c * n + nx] + (c ? 0.0 : 1.0) * 2.0;
+            if (kk != 2 * nx) lds[c * n + id] = a;  // (0,1) is written below, after the corner has read it
+            lds[alt + c * nr + kk] = kk == 2 * nx ? lds[alt + c * nr + kk] : old;
+        }
+        __syncthreads();
+        if (tid < 2) {  // ghost (0,1)
+            const double a = lds[alt + tid * nr + 2 * nx];
+            lds[alt + tid * nr + 2 * nx] = lds[tid * n + nx];
+            lds[tid * n + nx] = a;
+        }
+        iter++;
+        __syncthreads();
+    }
+    for (int k = tid; k < n; k += nt) {
+        u[k] = lds[k];
+        v[k] = lds[n + k];
+    }
+    if (tid == 0) {
+        out[0] = ures;
+        out[1] = vres;
+        out[2] = (double)iter;
+    }
+}
+
+// ---------------------------------------------------------------------------
 CompatCase::~CompatCase()
 {
     if (st) hipStreamSynchronize(st);
@@ -321,6 +747,17 @@ if_status CompatCase::create(const if_case_desc &d)
     IFF_HIP(hipMemcpyAsync(vx, ax.data(), ax.size() * 8, hipMemcpyHostToDevice, st));
     IFF_HIP(hipMemcpyAsync(vy, ay.data(), ay.size() * 8, hipMemcpyHostToDevice, st));
     IFF_HIP(hipHostMalloc((void **)&h_out, 4 * sizeof(double), hipHostMallocDefault));
+    // the one-workgroup forms, where the fields fit in one CU's LDS
+    if (N <= (size_t)kOneCells && nx < 32768 && ny < 32768) {
+        lds_ad = sizeof(double) * (2 * N + 4 * (size_t)(nx + ny) + 32);
+        lds_ppe = sizeof(double) * (2 * N + 32 + 2 * (size_t)(nx + ny));
+        one_ad = lds_ad <= kOneLds && ad_itermax <= kOneIters;
+        one_ppe = lds_ppe <= kOneLds;
+        const int most = (int)kOneLds;
+        for (const void *k : {(const void *)kc_ad_one<true>, (const void *)kc_ad_one<false>,
+                              (const void *)kc_ppe_one<true>, (const void *)kc_ppe_one<false>})
+            IFF_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, most));
+    }
     hipLaunchKernelGGL(kc_init, dim3(nblk), dim3(256), 0, st, nx, ny, vx + nx, vy + ny, u[0], v[0],
                        p[0], iblank);
     IFF_HIP(hipGetLastError());
@@ -346,6 +783,23 @@ if_status CompatCase::ad_step(if_step_stats *stt)
 {
     const double *xp = vx + 2 * nx, *xm = vx + 3 * nx, *px = vx + 4 * nx;
     const double *yp = vy + 2 * ny, *ym = vy + 3 * ny, *py = vy + 4 * ny;
+    if (one_ad) {
+        const int waves = (nx * ny + 511) / 512;
+        auto *k = waves <= 8 ? kc_ad_one<true> : kc_ad_one<false>;
+        hipLaunchKernelGGL(k, dim3(1), dim3(64 * waves), lds_ad, st, nx, ny, vx, vy, u[cur], v[cur], uf, vf, dt, w_ad,
+                           std::pow(10.0, -6.0), ad_itermax, h_out);
+        IFF_HIP(hipGetLastError());
+        IFF_HIP(hipStreamSynchronize(st));
+        steps++;
+        if (stt) {
+            std::memset(stt, 0, sizeof(*stt));
+            stt->steps = 1;
+            stt->ad_iters = (int)h_out[2];
+            stt->ad_res = h_out[0] + h_out[1];
+            stt->total_ad_iters = stt->ad_iters;
+        }
+        return IF_OK;
+    }
     // fresh per-call scratch (cudaMalloc'd in the reference, :275-287)
     IFF_HIP(hipMemsetAsync(u[1 - cur], 0, sizeof(double) * nx * ny, st));
     IFF_HIP(hipMemsetAsync(v[1 - cur], 0, sizeof(double) * nx * ny, st));
@@ -387,6 +841,25 @@ if_status CompatCase::ad_step(if_step_stats *stt)
 if_status CompatCase::ppe_solve(if_step_stats *stt)
 {
     const double *cxp = vx + 5 * nx, *cxm = vx + 6 * nx, *cyp = vy + 5 * ny, *cym = vy + 6 * ny;
+    if (one_ppe) {
+        const int waves = (nx * ny + 511) / 512;
+        auto *k = waves <= 8 ? kc_ppe_one<true> : kc_ppe_one<false>;
+        h_out[0] = 1.0;
+        h_out[1] = h_out[2] = 0.0;
+        do {  // a launch runs at most kOneIters iterations
+            hipLaunchKernelGGL(k, dim3(1), dim3(64 * waves), lds_ppe, st, nx, ny, vx, vy, p[pcur], (int)h_out[1],
+                               ppe_itermax, kOneIters, std::pow(10.0, -6.0), h_out);
+            IFF_HIP(hipGetLastError());
+            IFF_HIP(hipStreamSynchronize(st));
+        } while (h_out[2] == 0.0);
+        if (stt) {
+            std::memset(stt, 0, sizeof(*stt));
+            stt->ppe_sweeps = (int)h_out[1];
+            stt->ppe_res = h_out[0];
+            stt->total_ppe_sweeps = stt->ppe_sweeps;
+        }
+        return IF_OK;
+    }
     IFF_HIP(hipMemsetAsync(p[1 - pcur], 0, sizeof(double) * nx * ny, st));
     hipLaunchKernelGGL(kc_pbc, dim3(nblk), dim3(256), 0, st, nx, ny, p[pcur]);
     double residual = 1.0;

@@ -269,6 +269,7 @@ __global__ void kc_pbc(int nx, int ny, double *p)
 // on in the immediate offset), outside the LDS aperture the hardware tests.
 // ---------------------------------------------------------------------------
 constexpr int kOneCells = 8192;       // 16 waves x 512 cells
+constexpr int kOneReg = 4096;         // 8 waves, 256 registers a lane
 constexpr int kOneQ = 8;              // cells per lane
 constexpr int kOneIters = 16384;      // Poisson iterations per launch: bounds a launch to about 10 ms
 constexpr size_t kOneLds = 160 * 1024;
@@ -302,24 +303,18 @@ __device__ __forceinline__ double lane0(double v)
                             __builtin_amdgcn_readfirstlane(__double2loint(v)));
 }
 
-// Pass 1 of Reduction over a wave's 512 values: thread t of the reference's
-// block adds val(t) + val(t + 256) (val(t) alone past the end), which are
-// this lane's values q and q + 4.
-__device__ __forceinline__ double fold512(const double (&val)[kOneQ], int id0, int n)
+// Pass 1 of Reduction over a wave's 512 values (zero past the end): thread t
+// of the reference's block adds val(t) + val(t + 256), which are this lane's
+// values q and q + 4.
+__device__ __forceinline__ double fold512(const double (&val)[kOneQ])
 {
-    double a[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int id = id0 + 64 * q;
-        a[q] = id + 256 < n ? 0.0 + (val[q] + val[q + 4]) : (id < n ? 0.0 + val[q] : 0.0);
-    }
-    return fold64((a[0] + a[2]) + (a[1] + a[3]));
+    return fold64(((val[0] + val[4]) + (val[2] + val[6])) + ((val[1] + val[5]) + (val[3] + val[7])));
 }
 
 // Pass 2 over at most 16 block sums (the others are zero), in every wave.
 __device__ __forceinline__ double fold_parts(const double *lds, int part, int lane)
 {
-    return lane0(fold16(lane < 16 ? 0.0 + lds[part + lane] : 0.0));
+    return lane0(fold16(lane < 16 ? lds[part + lane] : 0.0));
 }
 
 // x / b, correctly rounded, from y = RN(1 / b): q = x y is within one ulp, the
@@ -327,7 +322,7 @@ __device__ __forceinline__ double fold_parts(const double *lds, int part, int la
 // correctly rounded quotient (P. Markstein, "Computation of elementary
 // functions on the IBM RISC System/6000 processor", IBM J. Res. Dev. 34, 1990,
 // theorem 7.2), unless b's mantissa is all ones or an operation leaves the
-// normal range: those take the division (div_special, and the range test).
+// normal range: those take the division.
 // Three operations where the division takes about 25, in a loop that is made
 // of one division per cell.
 __device__ __forceinline__ bool div_special(double b)
@@ -336,44 +331,154 @@ __device__ __forceinline__ bool div_special(double b)
     const double a = fabs(b);
     return m == 0xfffffffffffffull || !(a > 1e-60 && a < 1e60);
 }
-__device__ __forceinline__ double div_by(double x, double b, double y, bool special)
+__device__ __forceinline__ double div_by(double x, double b, double y)
 {
-    const double a = fabs(x);
-    if (special || !((a > 1e-200 && a < 1e200) || a == 0.0)) return x / b;
     const double q = x * y;
     return __builtin_fma(__builtin_fma(-q, b, x), y, q);
 }
+__device__ __forceinline__ double div_by(double x, double b, double y, bool special)
+{
+    const double a = fabs(x);
+    return (special || !((a > 1e-200 && a < 1e200) || a == 0.0)) ? x / b : div_by(x, b, y);
+}
 
-// Per-lane coefficients of its cells: held in registers (REG, at most 8 waves,
-// 256 registers a lane) or read from the LDS copies of the axis vectors.
-template <bool REG>
-struct OneCoef {
-    double xp[REG ? kOneQ : 1], xm[REG ? kOneQ : 1], yp[REG ? kOneQ : 1], ym[REG ? kOneQ : 1];
-};
+// A compile-time distance between the LDS buffers puts a buffer's offset into
+// the instructions.
+constexpr int kOneStride = kOneReg + 1;
 
-// PPESolver's loop (PPESolver.cu:164-195).  Iteration k reads p_k once: the
-// same four products give its residual (the stop test of iteration k) and
-// p_{k+1}, which goes to the other LDS buffer.  The test's sum is complete
-// after the iteration's one barrier; a stop at k stores p_k from registers.
-template <bool REG>
-__global__ __launch_bounds__(REG ? 512 : 1024) void kc_ppe_one(int nx, int ny, const double *vx, const double *vy,
+// PPESolver's loop (PPESolver.cu:164-195), at most kOneReg cells.  Iteration
+// k reads p_k once: the same four products give its residual (the stop test
+// of iteration k) and p_{k+1}, which goes to the other LDS buffer.  The
+// test's sum is complete after the iteration's one barrier; a stop at k
+// stores p_k from registers.  Everything a cell needs is in registers (8
+// waves, 256 registers a lane) and the loop has no branch per cell: a ring
+// cell, or one past the end, has zero coefficients, reads an interior cell's
+// neighbours and stores to a spare cell.  Bound by its FP64 instructions (17
+// per cell): the deck's 14,755 iterations on 52 x 52 cells take 16.0 ms (312
+// launch by launch, 27.8 with a branch per cell).
+__global__ __launch_bounds__(512) void kc_ppe_one(int nx, int ny, const double *vx, const double *vy, double *p,
+                                                  int iter0, int itermax, int most, double tol, double *out)
+{
+    __shared__ __align__(16) double lds[2 * kOneStride + 32];
+    constexpr int part = 2 * kOneStride;  // [2][16]
+    const int n = nx * ny;
+    const double *cxp = vx + 5 * nx, *cxm = vx + 6 * nx, *cyp = vy + 5 * ny, *cym = vy + 6 * ny;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int id0 = 512 * w + lane;
+    double xp[kOneQ], xm[kOneQ], yp[kOneQ], ym[kOneQ], own[kOneQ], y[kOneQ], ap[kOneQ];
+    int cs[kOneQ], cw[kOneQ], cn[kOneQ], to[kOneQ];  // south, west, north neighbour; where the cell is stored
+    bool special = false;
+    if (threadIdx.x < 32) lds[part + threadIdx.x] = 0.0;
+#pragma unroll
+    for (int q = 0; q < kOneQ; q++) {
+        const int id = id0 + 64 * q;
+        own[q] = 0.0;
+        int j = 0, i = 0;
+        if (id < n) {
+            j = id / nx;
+            i = id - j * nx;
+            double v = p[id];
+            if (i == 0 || j == 0) {  // set_pressure_BC
+                v = 100.0;
+                p[id] = v;
+            }
+            own[q] = v;
+            lds[id] = v;
+            lds[kOneStride + id] = v;
+        }
+        const bool in = i > 0 && i < nx - 1 && j > 0 && j < ny - 1;
+        const int c = in ? id : nx + 1;
+        cs[q] = c - nx;
+        cw[q] = c - 1;
+        cn[q] = c + nx;
+        to[q] = in ? id : kOneReg;
+        if (!in) own[q] = 0.0;
+        xp[q] = in ? cxp[i] : 0.0;
+        xm[q] = in ? cxm[i] : 0.0;
+        yp[q] = in ? cyp[j] : 0.0;
+        ym[q] = in ? cym[j] : 0.0;
+        ap[q] = in ? -1 * ((xp[q] + xm[q]) + (yp[q] + ym[q])) : 1.0;
+        special = special || div_special(ap[q]);
+        y[q] = 1.0 / ap[q];
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+    double res = 1.0;
+    int k = iter0;
+    bool stopped = k >= itermax;
+    // iteration k, p_k in buffer B; true: no further one
+    auto iteration = [&]<int B>() -> bool {
+        constexpr int b = B * kOneStride, nb = kOneStride - b;
+        double r[kOneQ], nv[kOneQ], small = 1.0, large = 1.0;
+#pragma unroll
+        for (int q = 0; q < kOneQ; q++) {
+            const double e = lds[b + cw[q] + 2] * xp[q], ww = lds[b + cw[q]] * xm[q];
+            const double nn = lds[b + cn[q]] * yp[q], s = lds[b + cs[q]] * ym[q];
+            r[q] = own[q] * ap[q] + e + ww + nn + s;
+            const double t = -(e + ww + nn + s);
+            nv[q] = div_by(t, ap[q], y[q]);
+            // (a cell without coefficients has t = 0 and is left out)
+            small = fmin(small, to[q] == kOneReg ? 1.0 : fabs(t));
+            large = fmax(large, fabs(t));
+        }
+        if (__any(special || !(small > 1e-200 && large < 1e200))) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int q = 0; q < kOneQ; q++) {
+                const double e = lds[b + cw[q] + 2] * xp[q], ww = lds[b + cw[q]] * xm[q];
+                const double nn = lds[b + cn[q]] * yp[q], s = lds[b + cs[q]] * ym[q];
+                nv[q] = -(e + ww + nn + s) / ap[q];
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        // the next iterate, before the test is known; the buffer's former
+        // contents were last read before the previous barrier
+#pragma unroll
+        for (int q = 0; q < kOneQ; q++) lds[nb + to[q]] = nv[q];
+        const double f = fold512(r);
+        if (lane == 0) lds[part + 16 * B + w] = f;
+        __syncthreads();
+        if (k > iter0) {  // (iter0: nothing done yet, or decided by the launch before)
+            res = fold_parts(lds, part + 16 * B, lane);
+            stopped = !(res > tol) || k >= itermax;
+        }
+        if (stopped || k - iter0 >= most) return true;
+#pragma unroll
+        for (int q = 0; q < kOneQ; q++) own[q] = nv[q];
+        k++;
+        return false;
+    };
+    while (!stopped)
+        if (iteration.template operator()<0>() || iteration.template operator()<1>()) break;
+#pragma unroll
+    for (int q = 0; q < kOneQ; q++)
+        if (to[q] != kOneReg) p[to[q]] = own[q];
+    if (threadIdx.x == 0) {
+        out[0] = res;
+        out[1] = (double)k;
+        out[2] = stopped ? 1.0 : 0.0;
+    }
+}
+
+// The same for up to kOneCells cells (16 waves, 128 registers a lane), with
+// the coefficients read from LDS.
+__global__ __launch_bounds__(1024) void kc_ppe_wide(int nx, int ny, const double *vx, const double *vy,
                                                                double *p, int iter0, int itermax, int most, double tol,
                                                                double *out)
 {
     extern __shared__ __align__(16) double lds[];
     const int n = nx * ny;
     // offsets in lds: the two iterates from 0 and n; the block sums, [2][16];
-    // !REG: cxp, cxm and cyp, cym
+    // cxp, cxm and cyp, cym
     const int part = 2 * n, lx = part + 32, ly = lx + 2 * nx;
     const double *cxp = vx + 5 * nx, *cxm = vx + 6 * nx, *cyp = vy + 5 * ny, *cym = vy + 6 * ny;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int id0 = 512 * w + lane;
-    OneCoef<REG> C;
-    double own[kOneQ], y[kOneQ], ap[REG ? kOneQ : 1];
+    double own[kOneQ], y[kOneQ];
     int ij[kOneQ];  // i in the low half, j in the high half
     unsigned in = 0;
     bool special = false;
-    if (!REG) {
+    {
         for (int k = threadIdx.x; k < 2 * nx; k += blockDim.x) lds[lx + k] = cxp[k];  // cxp, cxm are adjacent
         for (int k = threadIdx.x; k < 2 * ny; k += blockDim.x) lds[ly + k] = cyp[k];
     }
@@ -383,7 +488,6 @@ __global__ __launch_bounds__(REG ? 512 : 1024) void kc_ppe_one(int nx, int ny, c
         const int id = id0 + 64 * q;
         own[q] = y[q] = 0.0;
         ij[q] = 0;
-        if constexpr (REG) C.xp[q] = C.xm[q] = C.yp[q] = C.ym[q] = ap[q] = 0.0;
         if (id < n) {
             const int j = id / nx, i = id - j * nx;
             ij[q] = i | (j << 16);
@@ -397,13 +501,6 @@ __global__ __launch_bounds__(REG ? 512 : 1024) void kc_ppe_one(int nx, int ny, c
                 const double a = -1 * ((cxp[i] + cxm[i]) + (cyp[j] + cym[j]));
                 special = special || div_special(a);
                 y[q] = 1.0 / a;
-                if constexpr (REG) {
-                    C.xp[q] = cxp[i];
-                    C.xm[q] = cxm[i];
-                    C.yp[q] = cyp[j];
-                    C.ym[q] = cym[j];
-                    ap[q] = a;
-                }
             }
         }
     }
@@ -422,20 +519,12 @@ __global__ __launch_bounds__(REG ? 512 : 1024) void kc_ppe_one(int nx, int ny, c
             if (in & (1u << q)) {
                 const int id = b + id0 + 64 * q;
                 double xp, xm, yp, ym, a;
-                if constexpr (REG) {
-                    xp = C.xp[q];
-                    xm = C.xm[q];
-                    yp = C.yp[q];
-                    ym = C.ym[q];
-                    a = ap[q];
-                } else {
-                    const int i = ij[q] & 0xffff, j = ij[q] >> 16;
-                    xp = lds[lx + i];
-                    xm = lds[lx + nx + i];
-                    yp = lds[ly + j];
-                    ym = lds[ly + ny + j];
-                    a = -1 * ((xp + xm) + (yp + ym));
-                }
+                const int i = ij[q] & 0xffff, j = ij[q] >> 16;
+                xp = lds[lx + i];
+                xm = lds[lx + nx + i];
+                yp = lds[ly + j];
+                ym = lds[ly + ny + j];
+                a = -1 * ((xp + xm) + (yp + ym));
                 const double e = lds[id + 1] * xp, ww = lds[id - 1] * xm, nn = lds[id + nx] * yp, s = lds[id - nx] * ym;
                 r[q] = own[q] * a + e + ww + nn + s;
                 nv[q] = div_by(-(e + ww + nn + s), a, y[q], special);
@@ -447,7 +536,7 @@ __global__ __launch_bounds__(REG ? 512 : 1024) void kc_ppe_one(int nx, int ny, c
 #pragma unroll
         for (int q = 0; q < kOneQ; q++)
             if (in & (1u << q)) lds[nb + id0 + 64 * q] = nv[q];
-        const double f = fold512(r, id0, n);
+        const double f = fold512(r);
         if (lane == 0) lds[part + 16 * (k & 1) + w] = f;
         __syncthreads();
         if (k > iter0) {  // (iter0: nothing done yet, or decided by the launch before)
@@ -469,11 +558,19 @@ __global__ __launch_bounds__(REG ? 512 : 1024) void kc_ppe_one(int nx, int ny, c
     }
 }
 
+// Per-lane coefficients of its cells: held in registers (REG, at most
+// kOneReg cells) or read from the axis vectors.
+template <bool REG>
+struct OneCoef {
+    double xp[REG ? kOneQ : 1], xm[REG ? kOneQ : 1], yp[REG ? kOneQ : 1], ym[REG ? kOneQ : 1];
+};
+
 // ADsolver (ADSolver.cu:268-395) on one workgroup.  u and v live in LDS, in
 // place: a sweep holds its new values in registers until every cell has been
 // read.  The reference's second buffer matters only through its ring, which
 // keeps the values of two iterations ago: those are kept apart (alt) and
-// change places with the ring after each sweep.
+// change places with the ring after each sweep.  The deck's ten calls of five
+// iterations: 0.65 ms (3.5 launch by launch); 88 x 88 cells 2.7 ms (5.5).
 template <bool REG>
 __global__ __launch_bounds__(REG ? 512 : 1024) void kc_ad_one(int nx, int ny, const double *vx, const double *vy,
                                                               double *u, double *v, double *uf, double *vf, double dt,
@@ -631,7 +728,7 @@ __global__ __launch_bounds__(REG ? 512 : 1024) void kc_ad_one(int nx, int ny, co
                 r[c][q] = fabs(x - lds[a + id]);
             }
         }
-        const double fu = fold512(r[0], id0, n), fv = fold512(r[1], id0, n);
+        const double fu = fold512(r[0]), fv = fold512(r[1]);
         if (lane == 0) {
             lds[part + w] = fu;
             lds[part + 16 + w] = fv;
@@ -748,15 +845,14 @@ if_status CompatCase::create(const if_case_desc &d)
     IFF_HIP(hipMemcpyAsync(vy, ay.data(), ay.size() * 8, hipMemcpyHostToDevice, st));
     IFF_HIP(hipHostMalloc((void **)&h_out, 4 * sizeof(double), hipHostMallocDefault));
     // the one-workgroup forms, where the fields fit in one CU's LDS
-    if (N <= (size_t)kOneCells && nx < 32768 && ny < 32768) {
+    if (N <= (size_t)kOneCells) {
         lds_ad = sizeof(double) * (2 * N + 4 * (size_t)(nx + ny) + 32);
-        lds_ppe = sizeof(double) * (2 * N + 32 + 2 * (size_t)(nx + ny));
+        lds_ppe = N <= (size_t)kOneReg ? 0 : sizeof(double) * (2 * N + 32 + 2 * (size_t)(nx + ny));
         one_ad = lds_ad <= kOneLds && ad_itermax <= kOneIters;
         one_ppe = lds_ppe <= kOneLds;
-        const int most = (int)kOneLds;
         for (const void *k : {(const void *)kc_ad_one<true>, (const void *)kc_ad_one<false>,
-                              (const void *)kc_ppe_one<true>, (const void *)kc_ppe_one<false>})
-            IFF_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, most));
+                              (const void *)kc_ppe_wide})
+            IFF_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kOneLds));
     }
     hipLaunchKernelGGL(kc_init, dim3(nblk), dim3(256), 0, st, nx, ny, vx + nx, vy + ny, u[0], v[0],
                        p[0], iblank);
@@ -784,10 +880,11 @@ if_status CompatCase::ad_step(if_step_stats *stt)
     const double *xp = vx + 2 * nx, *xm = vx + 3 * nx, *px = vx + 4 * nx;
     const double *yp = vy + 2 * ny, *ym = vy + 3 * ny, *py = vy + 4 * ny;
     if (one_ad) {
-        const int waves = (nx * ny + 511) / 512;
-        auto *k = waves <= 8 ? kc_ad_one<true> : kc_ad_one<false>;
-        hipLaunchKernelGGL(k, dim3(1), dim3(64 * waves), lds_ad, st, nx, ny, vx, vy, u[cur], v[cur], uf, vf, dt, w_ad,
-                           std::pow(10.0, -6.0), ad_itermax, h_out);
+        const dim3 wg(64 * ((nx * ny + 511) / 512));
+        const double tol = std::pow(10.0, -6.0);
+        auto *k = nx * ny <= kOneReg ? kc_ad_one<true> : kc_ad_one<false>;
+        hipLaunchKernelGGL(k, dim3(1), wg, lds_ad, st, nx, ny, vx, vy, u[cur], v[cur], uf, vf, dt, w_ad, tol,
+                           ad_itermax, h_out);
         IFF_HIP(hipGetLastError());
         IFF_HIP(hipStreamSynchronize(st));
         steps++;
@@ -842,12 +939,12 @@ if_status CompatCase::ppe_solve(if_step_stats *stt)
 {
     const double *cxp = vx + 5 * nx, *cxm = vx + 6 * nx, *cyp = vy + 5 * ny, *cym = vy + 6 * ny;
     if (one_ppe) {
-        const int waves = (nx * ny + 511) / 512;
-        auto *k = waves <= 8 ? kc_ppe_one<true> : kc_ppe_one<false>;
+        const dim3 wg(64 * ((nx * ny + 511) / 512));
+        auto *k = nx * ny <= kOneReg ? kc_ppe_one : kc_ppe_wide;
         h_out[0] = 1.0;
         h_out[1] = h_out[2] = 0.0;
         do {  // a launch runs at most kOneIters iterations
-            hipLaunchKernelGGL(k, dim3(1), dim3(64 * waves), lds_ppe, st, nx, ny, vx, vy, p[pcur], (int)h_out[1],
+            hipLaunchKernelGGL(k, dim3(1), wg, lds_ppe, st, nx, ny, vx, vy, p[pcur], (int)h_out[1],
                                ppe_itermax, kOneIters, std::pow(10.0, -6.0), h_out);
             IFF_HIP(hipGetLastError());
             IFF_HIP(hipStreamSynchronize(st));

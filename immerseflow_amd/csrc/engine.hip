@@ -771,7 +771,7 @@ if_status Engine::refresh()
         int ty = 32;
         if (use_persistent)
             for (int cand : {48, 64, 80})
-                if (pers_fits(IF_FP64, 16, cand, 4, tiles_at(cand))) {
+                if (pers_fits(IF_FP64, 16, cand, 4, tiles_at(cand), wmode_)) {
                     ty = cand;
                     break;
                 }
@@ -958,7 +958,7 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         // persistent chunk: a register-tile shape with a persistent form in
         // this precision, and the grid fits on the device
         bool pers = any_rb && use_persistent && sweep_kind >= 2 &&
-                    pers_fits(pprec_, reg_waves(sweep_kind), tiles_sweep_ty_, M, nt_sweep_);
+                    pers_fits(pprec_, reg_waves(sweep_kind), tiles_sweep_ty_, M, nt_sweep_, wmode_);
         ran_pers = ran_pers || pers;
         if (any_rb) launch_sweeps = pers ? K : M;
         if (use_graphs) {
@@ -1193,7 +1193,7 @@ if_status Engine::autotune(if_tune_result *out)
         // FP64 shapes are timed per stage: an FP64 persistent launch's
         // second stage would overwrite the solve's current pressure.
         const bool pc = pprec_ != IF_FP64 && c.kind >= 2 && use_persistent &&
-                        pers_fits(pprec_, reg_waves(c.kind), c.ty, c.m, nt_sweep_);
+                        pers_fits(pprec_, reg_waves(c.kind), c.ty, c.m, nt_sweep_, wmode_);
         const int kp = 32 * c.m;
         const int s0 = pprec_ == IF_FP64 ? 0 : c.m;
         auto timed = [&]() {

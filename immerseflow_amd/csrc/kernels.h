@@ -33,8 +33,8 @@ void launch_ppe_sweep_reg(hipStream_t st, int prec, int waves, int ty, int m, co
 // resident on the device at once (a host query; call it outside stream
 // capture).  flags: one stage counter per tile, zeroed whenever the tile
 // table changes.
-bool pers_fits(int prec, int waves, int ty, int m, int nt);
-int pers_blocks(int prec, int waves, int ty, int m);  // 0: no persistent form
+bool pers_fits(int prec, int waves, int ty, int m, int nt, int wt);
+int pers_blocks(int prec, int waves, int ty, int m, int wt);  // 0: no persistent form
 void launch_ppe_sweep_pers(hipStream_t st, int prec, int waves, int ty, int m, const CaseDev *cs,
                            const int2 *tiles, int nt, int K, GridBar *bar, unsigned *flags, int wt);
 void launch_ppe_check(hipStream_t st, int prec, const CaseDev *cs, int ncase, const int2 *tiles,

@@ -317,7 +317,8 @@ __global__ __launch_bounds__(256) void k_ghost_p(const CaseDev *cs)
 // ---------------------------------------------------------------------------
 // P3: intermediate face velocities (Compute_velf interpolation,
 // ADSolver.cu:173-174,184-185, on open faces; body velocity on blanked
-// faces; the BC on domain faces) and the divergence RHS, in one pass.
+// faces; the BC on domain faces) and the divergence RHS, in one pass; with
+// them the kept cells' pressures for FP64 red-black solves.
 // ---------------------------------------------------------------------------
 template <typename TS>
 __global__ __launch_bounds__(256) void k_faces_rhs(const CaseDev *cs, const int2 *tiles,
@@ -336,6 +337,9 @@ __global__ __launch_bounds__(256) void k_faces_rhs(const CaseDev *cs, const int2
     double *uf = c.uf[out_buf], *vf = c.vf[out_buf];
     const AxisD &ax = c.x, &ay = c.y;
     const double dxi = ax.d[i], dxp = ax.d[i + 1], dxm = ax.d[i - 1];
+    const bool keep = with_rhs && c.ppe_solver == IF_PPE_RBSOR && !c.e[0];
+    const double *pb = c.p[c.ctrl->ppe_base];
+    double *pn = c.p[1 - c.ctrl->ppe_base];
     for (int r = threadIdx.x >> 6; r < c.tile_y; r += 4) {
         const int j = 1 + tc.ty * c.tile_y + r;
         if (j > ny - 2) break;
@@ -363,6 +367,10 @@ __global__ __launch_bounds__(256) void k_faces_rhs(const CaseDev *cs, const int2
         if (with_rhs)
             c.rhs[id] = (f & F_FLUID) ? ((ufe - ufw) * ax.rd[i] + (vfn - vfs) * ay.rd[j]) * c.rdt
                                       : 0.0;
+        // FP64 red-black solves: the register-tile sweeps do not write the
+        // cells they keep (not fluid, or without an open face), so both
+        // pressure buffers hold their values from here on
+        if (keep && (!(f & F_FLUID) || !(f & (F_OPEN_E | F_OPEN_W | F_OPEN_N | F_OPEN_S)))) pn[id] = pb[id];
     }
 }
 

@@ -12,13 +12,11 @@
 //   * north/south neighbours: the lane's own registers, except at the
 //     wave's first and last row, whose neighbours come from the adjacent
 //     waves through a small LDS exchange (one barrier per half-sweep).
-// FP64 (the oracle's update, bit for bit): rows whose cells are all fluid
-// with four open faces (nearly all of them) take a fast path whose
-// coefficients are the metric itself (x: per lane, y: per row); a row
-// holding any other cell evaluates every lane with its face flags.  FP32
-// (the mixed path's error sweeps): every cell takes one branch-free form,
-// the general one or, on a grid with one coefficient value per axis, the
-// five-operation one.  Every kernel computes the same expression per case
+// Every cell takes one branch-free form, with the metric itself as its
+// coefficients (x: per lane, y: per row) and 0 held in every cell the sweep
+// keeps.  FP64: the oracle's update, bit for bit.  FP32 (the mixed path's
+// error sweeps): the general form or, on a grid with one coefficient value
+// per axis, the five-operation one.  Every kernel computes the same expression per case
 // (sor.h), so the result does not depend on the path, the tile shape, the
 // kernel or the batch a case is in.  The cells' weights come from a table
 // indexed by the flag byte (uniform grids) or per cell (FP32: loaded once
@@ -104,34 +102,25 @@ __device__ __forceinline__ float reg_cell_w(float pc, float wr, float a1, float 
 }
 
 // One cell of a half-sweep, FP64, with the cell's weight w = om / sa formed
-// once per launch (w = 0: a cell the sweep does not update).  Fast path
-// (FAST): a fluid cell whose faces are all open except those on the domain
-// boundary; the coefficients are the metric with the boundary faces' entries
-// zeroed, so both paths give the same bits for such a cell.  Flag path: the
-// oracle's rule, coefficient zero on a closed face, no update of a non-fluid
-// cell or one with ap = 0.
-template <bool FAST>
-__device__ __forceinline__ double reg_cell(int f, double pc, double r, double pE, double pW, double pN, double pS,
-                                           double cxp, double cxm, double cyp, double cym, double w, double c1)
+// once per launch (w = 0: a cell the sweep keeps).  As in FP32 one branch-free
+// form: the tile holds 0 in every cell the sweep keeps, so the metric
+// coefficients (zeroed on boundary faces) give the neighbour sum of the
+// flagged ones (0 times the neighbour's value across a closed face), and the
+// kept cells' own values stay where they are in memory, in both buffers
+// (k_faces_rhs).  With the oracle's rule evaluated per cell instead, a row
+// holding any such cell took 2.5 times the operations in one dependent chain,
+// and every tile waited for the tiles around the body.
+__device__ __forceinline__ double reg_cell(double pc, double r, double pE, double pW, double pN, double pS, double cxp,
+                                           double cxm, double cyp, double cym, double w, double c1)
 {
-    if constexpr (FAST) {
-        const double sum = (cxp * pE + cxm * pW) + (cyp * pN + cym * pS);
-        return sor_cell_w64(pc, r, sum, w, c1);
-    } else {
-        const double aE = face_coef<double, F_OPEN_E>(f, cxp);
-        const double aW = face_coef<double, F_OPEN_W>(f, cxm);
-        const double aN = face_coef<double, F_OPEN_N>(f, cyp);
-        const double aS = face_coef<double, F_OPEN_S>(f, cym);
-        const double sum = (aE * pE + aW * pW) + (aN * pN + aS * pS);
-        const double nv = sor_cell_w64(pc, r, sum, w, c1);
-        return w != 0.0 ? nv : pc;
-    }
+    const double sum = (cxp * pE + cxm * pW) + (cyp * pN + cym * pS);
+    return sor_cell_w64(pc, r, sum, w, c1);
 }
 
 // One row's cells of a half-sweep.  c1 = 1 - om; the cells' weights are in R
 // (UNI, FP32: K = w ax, the five-operation form with ratio = ay / ax).
-template <typename T, int NRW, int Q, bool FAST, int k, bool UNI = false>
-__device__ __forceinline__ void reg_row(RegTile<T, NRW> &R, int f, T sv, T nv, T cxpa, T cxma, T cxpb, T cxmb,
+template <typename T, int NRW, int Q, int k, bool UNI = false>
+__device__ __forceinline__ void reg_row(RegTile<T, NRW> &R, T sv, T nv, T cxpa, T cxma, T cxpb, T cxmb,
                                         T c1, T ratio = (T)0)
 {
     constexpr int ks = k > 0 ? k - 1 : 0, kn = k < NRW - 1 ? k + 1 : 0;
@@ -144,8 +133,7 @@ __device__ __forceinline__ void reg_row(RegTile<T, NRW> &R, int f, T sv, T nv, T
         else if constexpr (sizeof(T) == 4)  // slot a: odd column, west neighbour in lane l-1
             R.pa[k] = reg_cell_w(R.pa[k], R.ra[k], cxma, pW, cxpa, pE, pN, pS, R.cyp[k], R.cym[k], R.wa[k], c1);
         else
-            R.pa[k] = reg_cell<FAST>(f & 0xff, R.pa[k], R.ra[k], pE, pW, pN, pS, cxpa, cxma, R.cyp[k], R.cym[k],
-                                     R.wa[k], c1);
+            R.pa[k] = reg_cell(R.pa[k], R.ra[k], pE, pW, pN, pS, cxpa, cxma, R.cyp[k], R.cym[k], R.wa[k], c1);
     } else {
         const T pS = k == 0 ? sv : R.pb[ks];
         const T pN = k == NRW - 1 ? nv : R.pb[kn];
@@ -155,8 +143,7 @@ __device__ __forceinline__ void reg_row(RegTile<T, NRW> &R, int f, T sv, T nv, T
         else if constexpr (sizeof(T) == 4)  // slot b: even column, east neighbour in lane l+1
             R.pb[k] = reg_cell_w(R.pb[k], R.rb[k], cxpb, pE, cxmb, pW, pN, pS, R.cyp[k], R.cym[k], R.wb[k], c1);
         else
-            R.pb[k] = reg_cell<FAST>(f >> 8, R.pb[k], R.rb[k], pE, pW, pN, pS, cxpb, cxmb, R.cyp[k], R.cym[k],
-                                     R.wb[k], c1);
+            R.pb[k] = reg_cell(R.pb[k], R.rb[k], pE, pW, pN, pS, cxpb, cxmb, R.cyp[k], R.cym[k], R.wb[k], c1);
     }
 }
 
@@ -189,37 +176,6 @@ __device__ __forceinline__ void fast_rows(ROW &&row, PUB &&publish)
         (row.template operator()<K + A + 1>(), ...);
     }(std::make_integer_sequence<int, (NRW - 2 > A ? NRW - 2 - A : 0)>{});
     __builtin_amdgcn_sched_barrier(0);
-}
-
-// Half-sweep on the wave's rows.  Q: rows k with (k & 1) == Q update slot
-// a, the others slot b.  sv/nv: the neighbours in the rows just south/north
-// of the wave (of its first and last row's updated slot); publish: makes this
-// wave's first and last row known.  ALLFAST: every row of the wave takes the
-// fast path (no branches); otherwise smask marks the rows that take the flag
-// path.
-template <typename T, int NRW, int Q, bool ALLFAST, typename PUB>
-__device__ __forceinline__ void reg_half(RegTile<T, NRW> &R, const uint16_t (*fl)[64], int lane,
-                                         unsigned smask, T sv, T nv, T cxpa, T cxma, T cxpb, T cxmb, T c1,
-                                         PUB &&publish)
-{
-    if constexpr (ALLFAST) {
-        fast_rows<NRW>([&]<int k>() { reg_row<T, NRW, Q, true, k>(R, 0, sv, nv, cxpa, cxma, cxpb, cxmb, c1); },
-                       publish);
-    } else {
-        int f[NRW];  // flags of every row, read in one batch
-#pragma unroll
-        for (int k = 0; k < NRW; k++) f[k] = fl[k][lane];
-        [&]<int... K>(std::integer_sequence<int, K...>) {
-            (([&] {
-                 if ((smask >> K) & 1u)
-                     reg_row<T, NRW, Q, false, K>(R, f[K], sv, nv, cxpa, cxma, cxpb, cxmb, c1);
-                 else
-                     reg_row<T, NRW, Q, true, K>(R, 0, sv, nv, cxpa, cxma, cxpb, cxmb, c1);
-             }()),
-             ...);
-        }(std::make_integer_sequence<int, NRW>{});
-        publish();
-    }
 }
 
 // Neighbour synchronisation of the persistent sweep.  Every tile has a
@@ -295,11 +251,6 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
     // moved twice the bytes: 32 KB per half-sweep of a 16-wave FP32 block,
     // 256 LDS cycles, where three rows of updates take about 160.)
     __shared__ T xch[2][NW + 2][2][64];
-    // Face flags (slot a in bits 0-7, slot b in 8-15), read by the rows that
-    // take the flag path; kept in LDS rather than registers.
-    constexpr int kFlw = sizeof(T) == 8 ? NW : 1;  // FP64 only
-    __shared__ uint16_t sfl[kFlw][NRW][64];
-
     const int t = tile_of_block(ntiles_pad);
     const int nstage = (K + M - 1) / M;  // PERS: stages of the launch
     if constexpr (PERS) {
@@ -371,11 +322,6 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
     const T cxma = (ina && ga != 1) ? G(cxm_)[ga] : (T)0;
     const T cxpb = (inb && ga + 1 != nx - 2) ? G(cxp_)[ga + 1] : (T)0;
     const T cxmb = (inb && ga + 1 != 1) ? G(cxm_)[ga + 1] : (T)0;
-    // faces a fluid cell of each slot has open when it is a fast-path cell
-    const int xa = (ga != nx - 2 ? F_OPEN_E : 0) | (ga != 1 ? F_OPEN_W : 0);
-    const int xb = (ga + 1 != nx - 2 ? F_OPEN_E : 0) | (ga + 1 != 1 ? F_OPEN_W : 0);
-    constexpr int kFaces = F_FLUID | F_OPEN_E | F_OPEN_W | F_OPEN_N | F_OPEN_S;
-
     // WM, the weight mode of the launch (kernels rather than runtime
     // branches, which would hold both forms' registers at once):
     //   1: every case has a weight table (wtab / wtab64): the weights are
@@ -499,13 +445,11 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
         }
     }
 
-    // Per-row coefficients and (FP64) the fast-path test and per-cell
-    // weights.  Rows outside the interior take the fast path with zero y
-    // coefficients and weight 0: their values stay finite, are never stored
-    // and reach interior cells only through the zero coefficients of the
-    // domain's boundary faces.  FP32 weights come from k_weights32 (0
-    // outside the interior and for kept cells); wr = w r is formed here.
-    unsigned smask = 0;  // FP64: rows holding a cell off the fast path
+    // Per-row coefficients and the cells' weights (0 for a cell the sweep
+    // keeps: outside the interior, not fluid, or without an open face; its
+    // value in the tile is 0).  FP32 weights come from k_weights32; wr = w r
+    // is formed here.
+    unsigned smask = 0;  // FP64: rows holding an interior cell that is kept
 #pragma unroll
     for (int k = 0; k < NRW; k++) {
         const int gj = jt0 + k;
@@ -527,23 +471,10 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
             R.ra[k] = R.wa[k] * R.ra[k];
             R.rb[k] = R.wb[k] * R.rb[k];
         } else {
-            const int f = lf[k];
-            sfl[w][k][lane] = (uint16_t)f;
-            bool offfast = false;
-            if (rowint) {
-                const int y4 = F_FLUID | (gj != ny - 2 ? F_OPEN_N : 0) | (gj != 1 ? F_OPEN_S : 0);
-                const int ea = y4 | xa, eb = y4 | xb;  // the fast-path pattern of each slot
-                const bool fa = !ina || (ea != F_FLUID && (f & kFaces) == ea);
-                const bool fb = !inb || (eb != F_FLUID && ((f >> 8) & kFaces) == eb);
-                offfast = __any(!(fa && fb));
-            }
-            if (offfast) smask |= 1u << k;
-            // the weight om / sa over the open faces (for a fast-path cell the
-            // same bits as om / (cx + cy)); 0 for a cell the sweep keeps:
-            // outside the interior, not fluid, or without an open face.  With
-            // a table: the entry of the cell's flag pattern, formed with the
-            // same expression (a cell outside the interior has flags 0)
-            const int fa = f & 0xff, fb = f >> 8;
+            // the weight om / sa over the open faces.  With a table: the entry
+            // of the cell's flag pattern, formed with the same expression (a
+            // cell outside the interior has flags 0)
+            const int f = lf[k], fa = f & 0xff, fb = f >> 8;
             if constexpr (wuni) {
                 auto look = [&](int q) {
                     const int i = (q & 63) << 2;
@@ -560,19 +491,18 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
                 R.wa[k] = (rowint && (fa & F_FLUID) && sa_a != (T)0) ? sor_weight64(sa_a, om) : (T)0;
                 R.wb[k] = (rowint && (fb & F_FLUID) && sa_b != (T)0) ? sor_weight64(sa_b, om) : (T)0;
             }
+            if (rowint && __any((ina && R.wa[k] == (T)0) || (inb && R.wb[k] == (T)0))) smask |= 1u << k;
+            R.pa[k] = R.wa[k] != (T)0 ? R.pa[k] : (T)0;
+            R.pb[k] = R.wb[k] != (T)0 ? R.pb[k] : (T)0;
         }
     }
     const T c1 = (T)1 - om;
 
     const int Z = (c0 + jt0) & 1;  // parity of slot a in the wave's first row
     // Half-sweep h has colour h & 1, and slot a of row k has parity Z + k,
-    // so rows with (k & 1) == Q update slot a where Q = (Z ^ h) & 1.  A
-    // wave of fast-path rows (FP32: every wave) runs branch-free.
-    // FP32: each half-sweep first updates the rows that do not touch the
-    // neighbouring waves (hiding the LDS read of the neighbour rows), then
-    // the first and last row, and ends by publishing those two rows for
-    // the next half-sweep.  Within a half-sweep every updated cell reads
-    // only cells of the other colour, so the row order changes no result.
+    // so rows with (k & 1) == Q update slot a where Q = (Z ^ h) & 1.  Within
+    // a half-sweep every updated cell reads only cells of the other colour,
+    // so the row order (fast_rows) changes no result.
     if (w == 0) {
 #pragma unroll
         for (int b = 0; b < 2; b++)
@@ -597,13 +527,13 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
         xch[b][w + 1][0][lane] = updated<T, NRW, Q, 0>(R);
         xch[b][w + 1][1][lane] = updated<T, NRW, Q, NRW - 1>(R);
     };
-    auto half32 = [&]<int Q, bool UNI>(int h) {
+    auto half = [&]<int Q, bool UNI>(int h) {
         const int b = h & 1;
         if (live(h)) {
             const T sv = xch[b][w][1][lane], nv = xch[b][w + 2][0][lane];
             fast_rows<NRW>(
                 [&]<int k>() {
-                    reg_row<T, NRW, Q, true, k, UNI>(R, 0, sv, nv, cxpa, cxma, cxpb, cxmb, c1, uratio);
+                    reg_row<T, NRW, Q, k, UNI>(R, sv, nv, cxpa, cxma, cxpb, cxmb, c1, uratio);
                 },
                 [&]() { publish.template operator()<Q>(b ^ 1); });
         }
@@ -619,49 +549,25 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
         __syncthreads();
         if (Z == 0) {
             for (int h = 0; h < n; h += 2) {
-                half32.template operator()<0, UNI>(h);
-                half32.template operator()<1, UNI>(h + 1);
+                half.template operator()<0, UNI>(h);
+                half.template operator()<1, UNI>(h + 1);
             }
         } else {
             for (int h = 0; h < n; h += 2) {
-                half32.template operator()<1, UNI>(h);
-                half32.template operator()<0, UNI>(h + 1);
+                half.template operator()<1, UNI>(h);
+                half.template operator()<0, UNI>(h + 1);
             }
         }
     };
-    // n half-sweeps (n even).  FP64: one loop body picks the colour order
-    // per half-sweep (two copies of the unrolled pair would exceed the
-    // register budget)
+    // n half-sweeps (n even)
     auto sweeps = [&](int n) {
-        if constexpr (sizeof(T) == 4) {
-            if constexpr (WM == 2) {
-                if (uni)
-                    pairs.template operator()<true>(n);
-                else
-                    pairs.template operator()<false>(n);
-            } else {
-                pairs.template operator()<WM == 1>(n);
-            }
-        } else {
-            if (Z == 0)
-                publish.template operator()<1>(0);
+        if constexpr (WM == 2) {
+            if (uni)
+                pairs.template operator()<true>(n);
             else
-                publish.template operator()<0>(0);
-            __syncthreads();
-            for (int h = 0; h < n; h++) {
-                const int b = h & 1;
-                const T sv = xch[b][w][1][lane], nv = xch[b][w + 2][0][lane];
-#define IFF_HALF(Q_, F_)                                                                                           \
-    reg_half<T, NRW, Q_, F_>(R, sfl[kFlw > 1 ? w : 0], lane, smask, sv, nv, cxpa, cxma, cxpb, cxmb, c1,            \
-                             [&]() { publish.template operator()<Q_>(b ^ 1); })
-                if (smask == 0) {
-                    if (((Z ^ h) & 1) == 0) IFF_HALF(0, true); else IFF_HALF(1, true);
-                } else {
-                    if (((Z ^ h) & 1) == 0) IFF_HALF(0, false); else IFF_HALF(1, false);
-                }
-#undef IFF_HALF
-                __syncthreads();
-            }
+                pairs.template operator()<false>(n);
+        } else {
+            pairs.template operator()<sizeof(T) == 4 && WM == 1>(n);
         }
     };
     // store the stored region of the tile (rows H .. H+TY-1, columns H ..
@@ -677,7 +583,10 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
                 if (rr < H || rr >= H + TY || gj > ny - 2) continue;
                 if (border && !lb && rr >= 2 * H && rr < TY) continue;
                 T *row = out + (size_t)gj * P;  // wave-uniform
-                if (ga + 1 <= nx - 2)
+                if (sizeof(T) == 8 && ((smask >> k) & 1u)) {  // kept cells are not written
+                    if (R.wa[k] != (T)0) GW(row)[ga] = R.pa[k];
+                    if (R.wb[k] != (T)0) GW(row)[ga + 1] = R.pb[k];
+                } else if (ga + 1 <= nx - 2)
                     gstore_vec<V2>(row + ga, V2{R.pa[k], R.pb[k]});
                 else if (ga <= nx - 2)
                     GW(row)[ga] = R.pa[k];
@@ -759,12 +668,18 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
                 const int srow = (jt0 + k) * P * (int)sizeof(T);  // uniform: scalar offset
                 if (!((m_st >> k) & 1u)) continue;
                 const int vo = ((m_all >> k) & 1u) ? vo_all : vo_side;
-                if constexpr (sizeof(T) == 4)
+                if constexpr (sizeof(T) == 4) {
                     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, V2{R.pa[k], R.pb[k]}), ro, vo, srow,
                                                           kDev);
-                else
+                } else if ((smask >> k) & 1u) {  // kept cells are not written
+                    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, R.pa[k]), ro,
+                                                          R.wa[k] != (T)0 ? vo : kDrop, srow, kDev);
+                    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, R.pb[k]), ro,
+                                                          R.wb[k] != (T)0 ? vo : kDrop, srow + 8, kDev);
+                } else {
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, V2{R.pa[k], R.pb[k]}), ro, vo, srow,
                                                            kDev);
+                }
             }
             if (one) {  // (a right edge tile: its last column is in the right strip)
 #pragma unroll
@@ -774,7 +689,8 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
                     if constexpr (sizeof(T) == 4)
                         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(R.pa[k]), ro, vo_one, srow, kDev);
                     else
-                        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, R.pa[k]), ro, vo_one, srow, kDev);
+                        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, R.pa[k]), ro,
+                                                              R.wa[k] != (T)0 ? vo_one : kDrop, srow, kDev);
                 }
             }
             if (last) break;
@@ -801,8 +717,13 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
                         v = __builtin_bit_cast(V2, __builtin_amdgcn_raw_buffer_load_b64(ro, voff, srow, kDev));
                     else
                         v = __builtin_bit_cast(V2, __builtin_amdgcn_raw_buffer_load_b128(ro, voff, srow, kDev));
-                    R.pa[k] = v[0];
-                    R.pb[k] = v[1];
+                    if constexpr (sizeof(T) == 8) {  // kept cells stay 0
+                        R.pa[k] = R.wa[k] != (T)0 ? v[0] : (T)0;
+                        R.pb[k] = R.wb[k] != (T)0 ? v[1] : (T)0;
+                    } else {
+                        R.pa[k] = v[0];
+                        R.pb[k] = v[1];
+                    }
                 }
             };
             if (ld_side) halo(m_st);

@@ -39,15 +39,6 @@ Engine::Engine(int prec, size_t budget)
     : prec_(prec), vprec_(prec == IF_MIXED_V32 ? IF_MIXED : IF_FP64), pprec_(prec == IF_FP64 ? IF_FP64 : IF_MIXED),
       budget_(budget)
 {
-    // default Poisson launch shape, by measurement on the 2048 x 1024
-    // ellipse: FP32 sweeps are fastest on 16-wave tiles at 8 sweeps per
-    // launch; FP64 sweeps (IEEE division per cell) on 8-wave tiles at 4,
-    // or as persistent 16-wave chunks when those fill the device (refresh)
-    if (prec != IF_FP64) {
-        sweep_kind = 4;
-        sweep_ty = 64;
-        sweep_m = 8;
-    }
 }
 
 Engine::~Engine()
@@ -755,29 +746,28 @@ if_status Engine::refresh()
         }
         wmode_ = tab == rb ? 1 : uni > 0 ? 2 : 0;
     }
-    // FP64 default shape, by measurement: 16-wave tiles as persistent
-    // chunks of the smallest height (48, 64, 80 rows) whose tiles fit in
-    // one launch, i.e. the most tiles the device holds at once (1024^2:
-    // 48 rows, 3.5 us per sweep against 3.9 at 64 and 5.0 at 80; 2048 x
-    // 1024: only 80 rows fit, 4.6 us against 6.1 per-stage); per-stage
-    // launches of 8-wave tiles of 32 rows when none fits
-    if (shape_auto && pprec_ == IF_FP64) {
-        auto tiles_at = [&](int ty) {
+    // The default shape follows the resident set: a persistent shape that
+    // fits on the device (reg_auto_shape), else per-stage launches: FP32 deep
+    // 128 x 128 blocks once they fill the device (4096^2: 6.9 us per sweep
+    // against 7.8 at 64 x 8), FP64 8-wave tiles of 32 rows
+    if (shape_auto) {
+        auto tiles_at = [&](int ty, int m, int *most) {
             int nt = 0;
-            for (int id : order_)
-                nt += ((slots_[id]->NX + reg_out_cols(4) - 1) / reg_out_cols(4)) * ((slots_[id]->NY + ty - 1) / ty);
+            for (int id : order_) {
+                const Slot &sl = *slots_[id];
+                const int t = ((sl.NX + reg_out_cols(m) - 1) / reg_out_cols(m)) * ((sl.NY + ty - 1) / ty);
+                nt += t;
+                if (most) *most = std::max(*most, t);
+            }
             return nt;
         };
-        int ty = 32;
-        if (use_persistent)
-            for (int cand : {48, 64, 80})
-                if (pers_fits(IF_FP64, 16, cand, 4, tiles_at(cand), wmode_)) {
-                    ty = cand;
-                    break;
-                }
-        sweep_kind = ty == 32 ? 3 : 4;
-        sweep_ty = ty;
-        sweep_m = 4;
+        sweep_kind = 4;
+        if (!use_persistent || !reg_auto_shape(pprec_, wmode_, tiles_at, &sweep_ty, &sweep_m)) {
+            const bool deep = pprec_ != IF_FP64 && tiles_at(88, 10, nullptr) > 512;
+            sweep_kind = pprec_ == IF_FP64 ? 3 : 4;
+            sweep_ty = pprec_ == IF_FP64 ? 32 : deep ? 88 : 64;
+            sweep_m = pprec_ == IF_FP64 ? 4 : deep ? 10 : 8;
+        }
     }
     if (n > cap_cases_) {
         if (d_cases_) hipFree(d_cases_);
@@ -880,13 +870,13 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
 {
     if (finished) *finished = 0;
     if (agg) std::memset(agg, 0, sizeof(*agg));
-    const int M = std::max(1, sweep_m);
     for (int it = 0; it < nsteps; it++) {
         bool ran_pers = false;
         if (dirty_) {
             if_status rc = refresh();
             if (rc != IF_OK) return rc;
         }
+        const int M = std::max(1, sweep_m);  // (refresh may choose it)
         if (order_.empty()) break;
         const int n = (int)order_.size();
         const int K = std::max(1, check_k);
@@ -996,6 +986,7 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
             IFF_HIP(hipStreamSynchronize(st_));
             if (b.err) {
                 use_persistent = false;
+                dirty_ = true;  // the default shape is chosen again
                 pers = false;
                 if (agg) agg->persistent_timeouts++;
                 launch_sweeps = M;

@@ -1,5 +1,7 @@
 // Launch wrappers of the fractional-step kernels (kernels.hip).
 #pragma once
+#include <functional>
+
 #include "common.h"
 
 namespace iff {
@@ -35,6 +37,9 @@ void launch_ppe_sweep_reg(hipStream_t st, int prec, int waves, int ty, int m, co
 // table changes.
 bool pers_fits(int prec, int waves, int ty, int m, int nt, int wt);
 int pers_blocks(int prec, int waves, int ty, int m, int wt);  // 0: no persistent form
+// the default shape (kernel 4): tiles(tile_y, m, &most) counts the tiles of all
+// cases and of the largest one
+bool reg_auto_shape(int prec, int wt, const std::function<int(int, int, int *)> &tiles, int *ty, int *m);
 void launch_ppe_sweep_pers(hipStream_t st, int prec, int waves, int ty, int m, const CaseDev *cs,
                            const int2 *tiles, int nt, int K, GridBar *bar, unsigned *flags, int wt);
 void launch_ppe_check(hipStream_t st, int prec, const CaseDev *cs, int ncase, const int2 *tiles,

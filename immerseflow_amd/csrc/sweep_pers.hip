@@ -1,7 +1,7 @@
 // Persistent launches of the register-tile red-black SOR (sweep_reg.h).
-#include <algorithm>
-
 #include "sweep_reg.h"
+
+#include <functional>
 
 namespace iff {
 
@@ -42,15 +42,65 @@ static void pers_one(hipStream_t st, const CaseDev *cs, const int2 *tiles, int n
 }
 
 // the shapes with a persistent form: (waves, sweeps per stage, tile_y,
-// rows per wave), FP32 and FP64
-#define IFF_PERS_SHAPES32(X) \
+// rows per wave), FP32 and FP64; the last ones of each are the default
+// shapes' own (reg_auto_shape)
+#define IFF_PERS_SHAPES32(X)                                                                                \
     X(float, 16, 8, 96, 8) X(float, 16, 8, 64, 6) X(float, 16, 4, 48, 4) X(float, 8, 8, 32, 8) X(float, 8, 4, 32, 6) \
-    X(float, 16, 8, 16, 3) X(float, 16, 8, 32, 4) X(float, 16, 8, 48, 5) X(float, 16, 12, 32, 5) X(float, 16, 12, 48, 6) \
-    X(float, 16, 12, 80, 8) X(float, 16, 16, 32, 6) X(float, 16, 16, 64, 8) X(float, 16, 4, 16, 2) X(float, 16, 4, 32, 3) \
-    X(float, 16, 4, 80, 6) X(float, 16, 4, 112, 8) X(float, 16, 6, 72, 6) X(float, 16, 6, 104, 8) X(float, 16, 6, 24, 3) X(float, 16, 6, 40, 4)
-#define IFF_PERS_SHAPES64(X) X(double, 16, 4, 80, 6) X(double, 16, 4, 64, 5) X(double, 16, 4, 48, 4) \
-    X(double, 16, 4, 16, 2) X(double, 16, 4, 32, 3) X(double, 16, 6, 24, 3) X(double, 16, 6, 40, 4) X(double, 16, 8, 16, 3) \
-    X(double, 16, 8, 32, 4) X(double, 16, 8, 48, 5) X(double, 16, 8, 64, 6) X(double, 16, 6, 56, 5) X(double, 16, 6, 72, 6) X(double, 16, 3, 20, 2) X(double,16,2,24,2) X(double, 8,4,16,4) X(double,8,4,32,6) X(double,8,2,24,4) X(double,8,4,48,8) X(double,8,3,36,6)
+    X(float, 16, 12, 16, 4) X(float, 16, 16, 32, 6) X(float, 16, 12, 48, 6)
+#define IFF_PERS_SHAPES64(X)                                                                        \
+    X(double, 16, 4, 80, 6) X(double, 16, 4, 64, 5) X(double, 16, 4, 48, 4) X(double, 16, 8, 32, 4) \
+    X(double, 16, 8, 64, 6) X(double, 16, 12, 16, 4) X(double, 16, 8, 48, 5)
+
+// The default launch shape of kernel 4, for cases whose tiles at (tile_y,
+// sweeps per stage) are counted by tiles: the first shape that fits on the
+// device as one persistent launch, in this order.  A small grid is bound by
+// the latency of its half-sweeps and of the exchange after each stage, not by
+// arithmetic: low tiles (few rows per wave) shorten the one, deep stages the
+// other, and the halo they recompute costs nothing on idle CUs; from about one
+// tile per CU on the recomputation counts.  Measured (us per sweep, uniform
+// n x n, one circle):
+//   FP32   n   64: 64 x 8 (one tile) 0.46, 16 x 12 0.54, 32 x 16 0.60
+//             256: 16 x 12 0.60, 32 x 16 0.66, 48 x 12 0.75, 64 x 8 0.85, 96 x 8 1.04
+//             611: 32 x 16 0.71 (200 tiles), 16 x 12 0.79 (312), 64 x 8 0.94
+//             800: 48 x 12 0.81 (170), 32 x 16 1.11 (325), 64 x 8 0.92
+//            1024: 64 x 8 0.96 (176), 48 x 12 1.12 (286), 96 x 8 1.12
+//            1948: 96 x 8 1.94 (441, two per CU); per stage 64 x 8 2.88
+//   stretched 2048 x 1024: 64 x 8 1.66 (352), 96 x 8 1.79 (242)
+//   FP64   n   64: 64 x 4 (one tile) 0.96, 16 x 12 1.06
+//             256: 16 x 12 1.10, 32 x 8 1.30, 48 x 4 1.78, 80 x 4 2.38
+//             800: 32 x 8 1.43 (225), 48 x 8 1.59, 64 x 8 1.81
+//            1024: 48 x 8 1.80 (242), 64 x 8 1.92, 48 x 4 2.2
+//   stretched 2048 x 1024: only 80 x 4 fits, 2.9
+// False: none fits.
+bool reg_auto_shape(int prec, int wt, const std::function<int(int, int, int *)> &tiles, int *ty, int *m)
+{
+    struct Shape {
+        int ty, m, per_cu;  // tiles per CU it is chosen at, at most
+        bool single;        // only where every case is one tile
+    };
+    static const Shape s32[] = {{64, 8, 2, true}, {16, 12, 1, false}, {32, 16, 1, false}, {48, 12, 1, false},
+                                {64, 8, 2, false}, {96, 8, 2, false}};
+    static const Shape s64[] = {{64, 4, 1, true}, {16, 12, 1, false}, {32, 8, 1, false}, {48, 8, 1, false},
+                                {64, 8, 1, false}, {80, 4, 1, false}};
+    static int cus = -1;  // one device type per process
+    if (cus < 0) {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            return false;
+        cus = n;
+    }
+    for (const Shape &s : prec == IF_FP64 ? s64 : s32) {
+        int most = 0;  // tiles of the largest case
+        const int nt = tiles(s.ty, s.m, &most);
+        if ((s.single && most > 1) || nt > s.per_cu * cus || !pers_fits(prec, 16, s.ty, s.m, nt, wt)) continue;
+        *ty = s.ty;
+        *m = s.m;
+        return true;
+    }
+    return false;
+}
+
 int pers_blocks(int prec, int waves, int ty, int m, int wt)
 {
 #define IFF_PB(T_, W_, M_, TY_, NRW_)                                                      \

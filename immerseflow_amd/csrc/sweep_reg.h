@@ -234,7 +234,7 @@ __device__ __forceinline__ bool wait_neighbours(const unsigned *flags, int nb, u
 // left free, some of them take a few more registers and run at one block
 // per CU, a third slower.
 template <typename T, int M, int NW, int NRW, bool PERS, int WM>
-__global__ __launch_bounds__(64 * NW, (sizeof(T) == 4 && NW == 16 && (NRW == 8 || (PERS && NRW <= 8)) && WM != 2) ? 8 : 1)
+__global__ __launch_bounds__(64 * NW, (sizeof(T) == 4 && NW == 16 && (PERS ? WM == 1 || (WM == 0 && NRW <= 6) : NRW == 8 && WM != 2)) ? 8 : 1)
 void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pad, int s, int K, GridBar *bar,
                  unsigned *flags)
 {

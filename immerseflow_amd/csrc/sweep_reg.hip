@@ -59,10 +59,17 @@ void launch_ppe_sweep_reg(hipStream_t st, int prec, int waves, int ty, int m, co
     IFF_RG(T, 8, 4, 32) IFF_RG(T, 8, 4, 48) IFF_RG(T, 8, 4, 64)                           \
     IFF_RG(T, 8, 8, 32) IFF_RG(T, 8, 8, 48) IFF_RG(T, 8, 8, 64)                           \
     IFF_RG(T, 16, 4, 48) IFF_RG(T, 16, 4, 64) IFF_RG(T, 16, 4, 80) IFF_RG(T, 16, 8, 32) IFF_RG(T, 16, 8, 64)
+    // (the default shapes' own come last in each list: they run per stage
+    // only after a neighbour wait timed out)
     if (prec == IF_FP64) {
         IFF_RG_ALL(double)
+        IFF_RG(double, 16, 12, 16)
+        IFF_RG(double, 16, 8, 48)
     } else {
         IFF_RG_ALL(float)
+        IFF_RG(float, 16, 12, 16)
+        IFF_RG(float, 16, 16, 32)
+        IFF_RG(float, 16, 12, 48)
         IFF_RG(float, 16, 8, 96)
         IFF_RG(float, 16, 9, 92)
         IFF_RG(float, 16, 10, 88)

@@ -106,19 +106,26 @@ struct Ctrl {
     int ppe_done, ppe_sweeps, ppe_base;
     int ng;            // live ghost-cell count (rebuilt on the device for moving bodies)
     int ng_total;      // ghost cells found by the last build (may exceed capacity)
+    unsigned ticket;   // tiles that have finished the running convergence check
     double ad_res, ppe_res, div_max;
     double t;          // simulated time
     long long tot_ad, tot_ppe;
     double max_div;
 };
 
-// Synchronisation state of the persistent Poisson sweep (one per engine):
-// a sticky error flag set when a wait times out, and the wait limit in
-// ticks of the 100 MHz real-time counter.
+// Synchronisation state of an engine's Poisson loop.  Persistent sweep: a
+// sticky error flag set when a wait times out, and the wait limit in ticks of
+// the 100 MHz real-time counter.  Convergence checks: cases counted in the
+// running check, those among them still iterating or still in the viscous
+// loop, the checks completed so far, and the host word (pinned memory) that
+// each check's last case writes: checks completed << 3 | kProg* bits.
 struct GridBar {
-    unsigned err, pad;
+    unsigned err, cases, open, ad_open;
     unsigned long long timeout;
+    unsigned long long checks;
+    unsigned long long *host;
 };
+enum : unsigned { kProgDone = 1, kProgAdOpen = 2, kProgErr = 4 };
 
 // Everything a kernel needs to know about one case.
 // Per-step monitors of a case (probes and body force), in device memory.

@@ -81,7 +81,7 @@ public:
     long long sweep_launches = 0;
     double sweep_cells = 0.0;  // interior cell-sweeps inside the timed chunks
     int launch_sweeps = 0;     // red-black sweeps per launch in the last step (M; K when persistent)
-    int spec_depth = 3;
+    int spec_depth = 2;        // Poisson chunks enqueued: the running one and those behind it
 
     static size_t footprint(const if_case_desc &d, int prec);
     void mark_dirty() { dirty_ = true; }
@@ -89,8 +89,8 @@ public:
 private:
     if_status build_slot(Slot &s, const if_case_desc &d);
     if_status refresh();      // re-upload the resident case list / tile tables
-    if_status snapshot(int ring_slot);
-    bool all_done(const Ctrl *snap, int which) const;
+    void check(int K);        // one convergence check
+    if_status wait_checks(unsigned long long base, unsigned long long behind, unsigned long long *word);
     if_status read_ctrl_sync(std::vector<Ctrl> &out);
     if_status update_moving();
     // the K sweeps of one Poisson chunk, as kernel launches on st_
@@ -119,10 +119,12 @@ private:
     bool any_moving_ = false;
     bool any_monitor_ = false;
     bool dirty_ = true;
-    // speculation ring
-    static constexpr int kRing = 8;
-    Ctrl *h_snap_ = nullptr;           // pinned, kRing * cap_ctrl_
-    hipEvent_t ev_[kRing] = {};
+    // the progress word that the convergence checks write (pinned), and the
+    // checks enqueued so far
+    unsigned long long *h_prog_ = nullptr;
+    unsigned long long checks_ = 0;
+    int ad_pred_ = 0;                  // viscous iterations to enqueue: the last step's and one (0: unknown)
+    bool operator_ready_ = false;      // weights and line factors of the resident set are formed
     // device time stamps of the timed Poisson chunks: [0] count, then a
     // start and an end stamp per chunk (at most kStamps)
     static constexpr int kStamps = 2 * 64;

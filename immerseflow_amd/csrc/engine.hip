@@ -9,9 +9,9 @@
 //   -> pressure BC -> P7/P8 projection + divergence -> ghost cells -> end
 //
 // The two iterative loops end on the device (per-case flags in Ctrl).  The
-// host enqueues loop units speculatively and watches asynchronous snapshots
-// of the control blocks, so it stops enqueueing a few units after the last
-// case converged instead of waiting for a result after every unit.
+// host enqueues loop units speculatively and watches a word in pinned memory
+// that every convergence check writes, so it stops enqueueing a unit after the
+// last case converged instead of waiting for a result after every unit.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -27,8 +27,9 @@ namespace iff {
 
 constexpr int kTileY = 16;  // base tiling (reductions, stencil passes)
 
-// viscous iteration budgets up to this are enqueued without polling
-constexpr int kAdEnqueueAll = 32;
+// viscous iterations enqueued when the last step tells nothing, and at a time
+// when it told too few
+constexpr int kAdFirst = 32, kAdMore = 4;
 
 // waves per workgroup of the register-tile sweep kinds (2, 3, 4)
 static int reg_waves(int kind) { return kind == 4 ? 16 : kind == 3 ? 8 : 4; }
@@ -57,9 +58,7 @@ Engine::~Engine()
     if (d_flags_) hipFree(d_flags_);
     if (d_tiles_base_) hipFree(d_tiles_base_);
     if (d_tiles_sweep_) hipFree(d_tiles_sweep_);
-    if (h_snap_) hipHostFree(h_snap_);
-    for (auto &e : ev_)
-        if (e) hipEventDestroy(e);
+    if (h_prog_) hipHostFree((void *)h_prog_);
     if (d_stamps_) hipFree(d_stamps_);
     if (h_stamps_) hipHostFree(h_stamps_);
     if (st_) hipStreamDestroy(st_);
@@ -77,12 +76,13 @@ if_status Engine::init()
     // neighbour waits of the persistent sweep give up after 20 ms
     // (IFF_PERSISTENT_TIMEOUT_TICKS overrides it, for tests of the time-out
     // path); b lives until the synchronisation below
+    IFF_HIP(hipHostMalloc((void **)&h_prog_, sizeof(unsigned long long), hipHostMallocCoherent | hipHostMallocMapped));
+    *h_prog_ = 0;
     GridBar b{};
+    IFF_HIP(hipHostGetDevicePointer((void **)&b.host, (void *)h_prog_, 0));
     b.timeout = 2000000;
     if (const char *e = std::getenv("IFF_PERSISTENT_TIMEOUT_TICKS")) b.timeout = std::strtoull(e, nullptr, 10);
     IFF_HIP(hipMemcpyAsync(d_bar_, &b, sizeof(GridBar), hipMemcpyHostToDevice, st_));
-    IFF_HIP(hipHostMalloc((void **)&h_snap_, sizeof(Ctrl) * cap_ctrl_ * kRing, hipHostMallocDefault));
-    for (auto &e : ev_) IFF_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     IFF_HIP(hipMalloc(&d_stamps_, sizeof(unsigned long long) * (1 + kStamps)));
     IFF_HIP(hipMemsetAsync(d_stamps_, 0, sizeof(unsigned long long) * (1 + kStamps), st_));
     IFF_HIP(hipHostMalloc((void **)&h_stamps_, sizeof(unsigned long long) * (1 + kStamps), hipHostMallocDefault));
@@ -524,7 +524,7 @@ if_status Engine::build_slot(Slot &s, const if_case_desc &d)
         on.ng = off.ng = s.ng;
         on.ng_total = off.ng_total = s.ng;
         IFF_HIP(hipMemcpyAsync(c.ctrl, &on, sizeof(Ctrl), hipMemcpyHostToDevice, st_));
-        launch_ghost_vel(st_, vprec_, tmp, 1, s.gcap, 1);
+        launch_ghost_vel(st_, vprec_, tmp, 1, s.gcap);
         std::vector<int2> tl(s.ntx * s.nty);
         for (int t = 0; t < (int)tl.size(); t++) tl[t] = make_int2(0, t);
         IFF_HIP(hipMalloc(&scr.dtl, sizeof(int2) * tl.size()));
@@ -710,8 +710,8 @@ if_status Engine::capture_sweeps(int K, int M, bool any_rb, bool any_jac, bool a
     return IF_OK;
 }
 
-// After a step that ran persistent sweeps: a neighbour wait that timed out
-// (blocks not all resident) leaves the results invalid.  Reset the state,
+// After the autotuner ran persistent sweeps: a neighbour wait that timed out
+// (blocks not all resident) leaves the timings invalid.  Reset the state,
 // stop using the persistent form and report the failure.
 if_status Engine::check_barrier()
 {
@@ -725,12 +725,13 @@ if_status Engine::check_barrier()
     if (cap_flags_ > 0) IFF_HIP(hipMemsetAsync(d_flags_, 0, sizeof(unsigned) * cap_flags_, st_));
     IFF_HIP(hipStreamSynchronize(st_));
     return fail(IF_ERR_HIP, "persistent Poisson sweep: a neighbour wait timed out (blocks not co-resident); "
-                            "this step's result is invalid and the persistent form is now off");
+                            "the persistent form is now off");
 }
 
 if_status Engine::refresh()
 {
     g_valid_ = false;  // the captured launches point at the old tables
+    operator_ready_ = false;
     order_.clear();
     for (auto &s : slots_)
         if (s && s->state == 0) order_.push_back(s->id);
@@ -826,24 +827,34 @@ if_status Engine::refresh()
     return IF_OK;
 }
 
-if_status Engine::snapshot(int r)
+// One convergence check (every check writes the progress word once).
+void Engine::check(int K)
 {
-    const int n = std::max(1, (int)slots_.size());
-    IFF_HIP(hipMemcpyAsync(h_snap_ + (size_t)r * cap_ctrl_, d_ctrl_, sizeof(Ctrl) * n,
-                           hipMemcpyDeviceToHost, st_));
-    IFF_HIP(hipEventRecord(ev_[r], st_));
-    return IF_OK;
+    launch_ppe_check(st_, pprec_, d_cases_, (int)order_.size(), d_tiles_base_, nt_base_, K, d_bar_);
+    checks_++;
 }
 
-bool Engine::all_done(const Ctrl *snap, int which) const
+// Wait until at most `behind` of the enqueued checks have not completed, or
+// (base: the checks enqueued before the loop) one of this loop's has found
+// every case done; *word gets the progress word.  A check that never completes
+// is a failed launch: the stream says so.
+if_status Engine::wait_checks(unsigned long long base, unsigned long long behind, unsigned long long *word)
 {
-    for (int id : order_) {
-        const Ctrl &c = snap[id];
-        if (!c.active) continue;
-        if (which == 0 && !c.ad_done) return false;
-        if (which == 1 && !c.ppe_done) return false;
+    for (unsigned long long spin = 1;; spin++) {
+        const unsigned long long v = __atomic_load_n(h_prog_, __ATOMIC_ACQUIRE), n = v >> 3;
+        if (checks_ - n <= behind || (n > base && (v & kProgDone))) {
+            *word = v;
+            return IF_OK;
+        }
+        if (spin % 65536 == 0) {
+            const hipError_t q = hipStreamQuery(st_);
+            if (q == hipErrorNotReady) continue;
+            if (q != hipSuccess) return fail(IF_ERR_HIP, hipGetErrorString(q));
+            if (checks_ != __atomic_load_n(h_prog_, __ATOMIC_ACQUIRE) >> 3)
+                return fail(IF_ERR_HIP, "a convergence check did not complete");
+        }
+        __builtin_ia32_pause();
     }
-    return true;
 }
 
 // Moving bodies: place every moving body at t_{n+1}, reclassify, rebuild
@@ -871,7 +882,6 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
     if (finished) *finished = 0;
     if (agg) std::memset(agg, 0, sizeof(*agg));
     for (int it = 0; it < nsteps; it++) {
-        bool ran_pers = false;
         if (dirty_) {
             if_status rc = refresh();
             if (rc != IF_OK) return rc;
@@ -896,95 +906,78 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         launch_step_begin(st_, d_cases_, n);
         launch_source(st_, vprec_, d_cases_, d_tiles_base_, nt_base_);
 
-        // ---- P2: viscous Jacobi sweeps, ended per case on the device
-        auto spec = [&](int maxn, int which, auto &&unit) -> if_status {
-            int enq = 0, obs = 0;
-            bool done = false;
-            while (enq < maxn && !done) {
-                unit(enq);
-                if_status rc = snapshot(enq % kRing);
-                if (rc != IF_OK) return rc;
-                enq++;
-                while (obs < enq) {
-                    const int r = obs % kRing;
-                    if (enq - obs < spec_depth && enq < maxn) {
-                        const hipError_t q = hipEventQuery(ev_[r]);
-                        if (q == hipErrorNotReady) break;
-                        if (q != hipSuccess) return fail(IF_ERR_HIP, hipGetErrorString(q));
-                    } else {
-                        IFF_HIP(hipEventSynchronize(ev_[r]));
-                    }
-                    if (all_done(h_snap_ + (size_t)r * cap_ctrl_, which)) { done = true; break; }
-                    obs++;
-                }
-            }
-            return IF_OK;
-        };
-        auto ad_unit = [&](int) {
-            launch_ad_sweep(st_, vprec_, d_cases_, d_tiles_base_, nt_base_);
-            launch_ghost_vel(st_, vprec_, d_cases_, n, max_ng_, 0);
-            launch_ad_finalize(st_, d_cases_, n);
-        };
-        // A short viscous loop (the usual 25-iteration budget) is enqueued
-        // whole: the kernels end each case's iterations on the device, and
-        // polling snapshots would cost a copy per iteration.
-        if_status rc = IF_OK;
-        if (max_ad_ <= kAdEnqueueAll)
-            for (int u = 0; u < max_ad_; u++) ad_unit(u);
-        else
-            rc = spec(max_ad_, 0, ad_unit);
-        if (rc != IF_OK) return rc;
-
-        // ---- P3: faces + RHS
-        launch_faces(st_, vprec_, d_cases_, d_tiles_base_, nt_base_, 1, 1);
-        if (any_line) launch_line_factor(st_, pprec_, d_cases_, n, max_ring_);
-        if (pprec_ == IF_MIXED)
-            launch_weights32(st_, d_cases_, n, max_ring_);
-        else
-            launch_weight_table64(st_, d_cases_, n);
-
-        // ---- P4/P5: Poisson in chunks of K sweeps (unit 0 = the entry check)
-        const int nunits = 1 + (max_ppe_ + K - 1) / K;
         // persistent chunk: a register-tile shape with a persistent form in
         // this precision, and the grid fits on the device
         bool pers = any_rb && use_persistent && sweep_kind >= 2 &&
                     pers_fits(pprec_, reg_waves(sweep_kind), tiles_sweep_ty_, M, nt_sweep_, wmode_);
-        ran_pers = ran_pers || pers;
         if (any_rb) launch_sweeps = pers ? K : M;
-        if (use_graphs) {
+        // a chunk of one launch gains nothing from a graph
+        bool graph = use_graphs && !(pers && !any_jac && !any_line && !timing);
+        if_status rc = IF_OK;
+        if (graph) {
             rc = capture_sweeps(K, M, any_rb, any_jac, any_line, pers, timing);
             if (rc != IF_OK) return rc;
         }
-        if (timing) launch_stamp_reset(st_, d_stamps_);
-        hipError_t glaunch = hipSuccess;
-        bool reopened = false;  // the solve after a persistent time-out (no entry check)
-        auto ppe_unit = [&](int u) {
-            if (u == 0) {
-                if (!reopened) launch_ppe_check(st_, pprec_, d_cases_, n, d_tiles_base_, nt_base_, 0);
-                return;
+
+        // ---- P4/P5: Poisson in chunks of K sweeps; each chunk's check tells
+        // the host through the progress word.  One chunk is queued behind the
+        // running one; the chunks behind the last case's end do nothing.
+        const int nchunks = (max_ppe_ + K - 1) / K;
+        unsigned long long word = 0;
+        auto poisson = [&](bool entry_check) -> if_status {
+            const unsigned long long base = checks_;
+            if (entry_check) check(0);
+            for (int u = 0; u < nchunks; u++) {
+                if (graph) {
+                    const hipError_t e = hipGraphLaunch(g_sweeps_, st_);
+                    if (e != hipSuccess)
+                        return fail(IF_ERR_HIP, std::string("sweep graph launch: ") + hipGetErrorString(e));
+                } else {
+                    enqueue_sweeps(K, M, any_rb, any_jac, any_line, pers, timing);
+                }
+                check(K);
+                if_status r = wait_checks(base, spec_depth - 1, &word);
+                if (r != IF_OK) return r;
+                if ((word >> 3) > base && (word & kProgDone)) return IF_OK;
             }
-            if (use_graphs) {
-                const hipError_t e = hipGraphLaunch(g_sweeps_, st_);
-                if (e != hipSuccess && glaunch == hipSuccess) glaunch = e;
-            } else {
-                enqueue_sweeps(K, M, any_rb, any_jac, any_line, pers, timing);
-            }
-            launch_ppe_check(st_, pprec_, d_cases_, n, d_tiles_base_, nt_base_, K, pers ? d_bar_ : nullptr);
+            return wait_checks(base, 0, &word);
         };
-        rc = spec(nunits, 1, ppe_unit);
-        if (rc != IF_OK) return rc;
-        if (glaunch != hipSuccess) return fail(IF_ERR_HIP, std::string("sweep graph launch: ") + hipGetErrorString(glaunch));
-        if (pers) {
-            // A neighbour wait of the persistent sweep that timed out (the
-            // blocks were not all resident) ended the Poisson loop early,
-            // with a finite but unconverged pressure.  Turn the persistent
-            // form off, clear the flag and the stage counters, and solve
-            // again from that pressure with one launch per stage; the step
-            // then completes as usual.
-            GridBar b{};
-            IFF_HIP(hipMemcpyAsync(&b, d_bar_, sizeof(GridBar), hipMemcpyDeviceToHost, st_));
-            IFF_HIP(hipStreamSynchronize(st_));
-            if (b.err) {
+
+        // ---- P2: viscous Jacobi sweeps, ended per case on the device.  As
+        // many are enqueued as the last step needed and one more; a case that
+        // needs more keeps its Poisson loop closed (k_step_begin), the checks
+        // report it, and the passes from here on are enqueued again.
+        // (Enqueueing the whole budget cost three launches for each of the 20
+        // iterations of 25 that a step does not need: half of a 64^2 step.)
+        int ad_enq = 0, ad_next = ad_pred_ > 0 ? ad_pred_ : kAdFirst;
+        if (timing) launch_stamp_reset(st_, d_stamps_);
+        do {
+            for (int k = 0; k < ad_next && ad_enq < max_ad_; k++, ad_enq++) {
+                launch_ad_sweep(st_, vprec_, d_cases_, d_tiles_base_, nt_base_);
+                launch_ad_finish(st_, vprec_, d_cases_, n);
+            }
+            ad_next = kAdMore;
+            // ---- P3: faces + RHS
+            launch_faces(st_, vprec_, d_cases_, d_tiles_base_, nt_base_, 1, 1);
+            // what depends on the flags and the metric alone: once for a
+            // resident set, every step with moving bodies
+            if (!operator_ready_) {
+                if (any_line) launch_line_factor(st_, pprec_, d_cases_, n, max_ring_);
+                if (pprec_ == IF_MIXED)
+                    launch_weights32(st_, d_cases_, n, max_ring_);
+                else
+                    launch_weight_table64(st_, d_cases_, n);
+                operator_ready_ = !any_moving_;
+            }
+            rc = poisson(true);
+            if (rc != IF_OK) return rc;
+            if (word & kProgErr) {
+                // A neighbour wait of the persistent sweep that timed out (the
+                // blocks were not all resident) ended the Poisson loop early,
+                // with a finite but unconverged pressure.  Turn the persistent
+                // form off, clear the flag and the stage counters, and solve
+                // again from that pressure with one launch per stage; the step
+                // then completes as usual.
                 use_persistent = false;
                 dirty_ = true;  // the default shape is chosen again
                 pers = false;
@@ -994,23 +987,21 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
                 IFF_HIP(hipMemsetAsync(&d_bar_->err, 0, sizeof(unsigned), st_));
                 if (cap_flags_ > 0) IFF_HIP(hipMemsetAsync(d_flags_, 0, sizeof(unsigned) * cap_flags_, st_));
                 launch_ppe_rearm(st_, d_cases_, n);
-                if (use_graphs) {
+                graph = use_graphs;
+                if (graph) {
                     rc = capture_sweeps(K, M, any_rb, any_jac, any_line, false, timing);
                     if (rc != IF_OK) return rc;
                 }
                 if (timing) launch_stamp_reset(st_, d_stamps_);
-                reopened = true;
-                rc = spec(nunits, 1, ppe_unit);
+                rc = poisson(false);
                 if (rc != IF_OK) return rc;
-                if (glaunch != hipSuccess)
-                    return fail(IF_ERR_HIP, std::string("sweep graph launch: ") + hipGetErrorString(glaunch));
             }
-        }
+        } while ((word & kProgAdOpen) && ad_enq < max_ad_);
 
         // ---- pressure BC, projection, divergence, ghost cells
         launch_pressure_bc(st_, d_cases_, n, max_ring_, max_ng_);
         launch_project(st_, vprec_, d_cases_, d_tiles_base_, nt_base_);
-        launch_ghost_vel(st_, vprec_, d_cases_, n, max_ng_, 1);
+        launch_ghost_vel(st_, vprec_, d_cases_, n, max_ng_);
         if (any_monitor_) launch_monitor(st_, vprec_, d_cases_, n, d_tiles_base_, nt_base_);
         launch_step_end(st_, d_cases_, n);
         for (int id : order_) slots_[id]->steps_host++;
@@ -1021,10 +1012,8 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         std::vector<Ctrl> all;
         rc = read_ctrl_sync(all);
         if (rc != IF_OK) return rc;
-        if (ran_pers) {
-            rc = check_barrier();
-            if (rc != IF_OK) return rc;
-        }
+        ad_pred_ = 0;
+        for (int id : order_) ad_pred_ = std::max(ad_pred_, all[id].ad_iter + 1);
         const int timed = timing ? (int)std::min<unsigned long long>(h_stamps_[0], kStamps) / 2 : 0;
         if (timed > 0) {
             int maxsw = 0;
@@ -1224,7 +1213,7 @@ if_status Engine::autotune(if_tune_result *out)
         (void)hipEventRecord(e0, st_);
         for (int r = 0; r < kReps; r++) {
             launch_tune_arm(st_, d_cases_, n, d_ctrl_, saved);
-            launch_ppe_check(st_, pprec_, d_cases_, n, d_tiles_base_, nt_base_, 2 * best.m);
+            check(2 * best.m);
         }
         (void)hipEventRecord(e1, st_);
         float ms = 0.f;
@@ -1627,7 +1616,7 @@ if_status Engine::restart(int k, const double *u, const double *v, const double 
               hipMemcpyAsync(dtl, tl.data(), sizeof(int2) * tl.size(), hipMemcpyHostToDevice, st_) == hipSuccess &&
               hipMemcpyAsync(s->dev.ctrl, &on, sizeof(Ctrl), hipMemcpyHostToDevice, st_) == hipSuccess;
     if (ok) {
-        launch_ghost_vel(st_, vprec_, tmp, 1, s->gcap, 1);
+        launch_ghost_vel(st_, vprec_, tmp, 1, s->gcap);
         if (!uf) launch_faces(st_, vprec_, tmp, dtl, (int)tl.size(), 0, 0);
         ok = hipMemcpyAsync(s->dev.ctrl, &ct, sizeof(Ctrl), hipMemcpyHostToDevice, st_) == hipSuccess &&
              hipStreamSynchronize(st_) == hipSuccess;

@@ -9,8 +9,8 @@ namespace iff {
 void launch_step_begin(hipStream_t st, const CaseDev *cs, int ncase);
 void launch_source(hipStream_t st, int prec, const CaseDev *cs, const int2 *tiles, int nt);
 void launch_ad_sweep(hipStream_t st, int prec, const CaseDev *cs, const int2 *tiles, int nt);
-void launch_ad_finalize(hipStream_t st, const CaseDev *cs, int ncase);
-void launch_ghost_vel(hipStream_t st, int prec, const CaseDev *cs, int ncase, int max_ng, int mode);
+void launch_ad_finish(hipStream_t st, int prec, const CaseDev *cs, int ncase);
+void launch_ghost_vel(hipStream_t st, int prec, const CaseDev *cs, int ncase, int max_ng);
 void launch_pressure_bc(hipStream_t st, const CaseDev *cs, int ncase, int max_ring, int max_ng);
 bool sweep_variant_ok(int ty, int m);
 void launch_ppe_sweep(hipStream_t st, int prec, int solver, int ty, int m, const CaseDev *cs,
@@ -43,7 +43,7 @@ bool reg_auto_shape(int prec, int wt, const std::function<int(int, int, int *)> 
 void launch_ppe_sweep_pers(hipStream_t st, int prec, int waves, int ty, int m, const CaseDev *cs,
                            const int2 *tiles, int nt, int K, GridBar *bar, unsigned *flags, int wt);
 void launch_ppe_check(hipStream_t st, int prec, const CaseDev *cs, int ncase, const int2 *tiles,
-                      int nt, int K, const GridBar *bar = nullptr);
+                      int nt, int K, GridBar *bar);
 void launch_ppe_rearm(hipStream_t st, const CaseDev *cs, int ncase);
 // zebra line SOR: the per-step factors (pivots, c', 1/m) of every line
 // case, then one sweep (both colours) at chunk position s

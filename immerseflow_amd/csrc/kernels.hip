@@ -108,7 +108,10 @@ __global__ void k_step_begin(const CaseDev *cs, int ncase)
     c->ad_done = (cs[k].ad_itermax <= 0) ? 1 : 0;
     c->ad_iter = 0;
     c->ad_res = 0.0;
-    c->ppe_done = 0;
+    // the Poisson loop opens when the viscous loop ends (k_ad_finish): passes
+    // enqueued behind too few viscous iterations do nothing, and the host
+    // enqueues them again
+    c->ppe_done = c->ad_done ? 0 : 1;
     c->ppe_sweeps = 0;
     c->ppe_res = 0.0;
 }
@@ -228,45 +231,13 @@ __global__ __launch_bounds__(256) void k_ad_sweep(const CaseDev *cs, const int2 
     if (threadIdx.x == 0) c.part[tc.t] = acc;
 }
 
-// One block per case: the stopping rule of ADSolver.cu:315 on the device.
-__global__ __launch_bounds__(256) void k_ad_finalize(const CaseDev *cs, int ncase)
-{
-    const CaseDev &c = cs[blockIdx.x];
-    Ctrl *ct = c.ctrl;
-    if (!ct->active || ct->ad_done) return;
-    const int nt = c.ntx * c.nty;
-    double s = 0.0;
-    for (int k = threadIdx.x; k < nt; k += 256) s += c.part[k];
-    s = block_sum(s);
-    if (threadIdx.x == 0) {
-        ct->ad_res = s;
-        ct->ad_iter += 1;
-        ct->ad_base ^= 1;
-        ct->tot_ad += 1;
-        if (!(s <= 1.0e300)) ct->failed = 1;
-        if (!(s > c.ad_tol) || ct->ad_iter >= c.ad_itermax) ct->ad_done = 1;
-    }
-}
-
 // ---------------------------------------------------------------------------
-// ghost-cell (image point) updates.  mode 0: on the new AD iterate (skipped
-// once the case's AD loop is done); mode 1: on the current velocity.
-// Stencil nodes are fluid cells (or the ghost itself with weight 0), which
+// ghost-cell (image point) updates.  Stencil nodes are fluid cells (or the ghost itself with weight 0), which
 // these kernels never write: no ordering between ghost cells is needed.
 // ---------------------------------------------------------------------------
 template <typename TS>
-__global__ __launch_bounds__(256) void k_ghost_vel(const CaseDev *cs, int mode)
+__device__ __forceinline__ void ghost_vel(const CaseDev &c, TS *u, TS *v, int g)
 {
-    const CaseDev &c = cs[blockIdx.y];
-    const Ctrl *ct = c.ctrl;
-    const int g = blockIdx.x * 256 + threadIdx.x;
-    if (g >= ct->ng || !ct->active) return;
-    int buf = ct->ad_base;
-    if (mode == 0) {
-        if (ct->ad_done) return;
-        buf = 1 - buf;
-    }
-    TS *u = fld<TS>(c.u[buf]), *v = fld<TS>(c.v[buf]);
     const GhostDev &o = c.gh[g];
     const BodyDev &b = c.bodies[o.body];
     double su = o.cd * b.ub, sv = o.cd * b.vb;
@@ -277,6 +248,64 @@ __global__ __launch_bounds__(256) void k_ghost_vel(const CaseDev *cs, int mode)
     }
     u[o.gidx] = (TS)su;
     v[o.gidx] = (TS)sv;
+}
+
+template <typename TS>
+__global__ __launch_bounds__(256) void k_ghost_vel(const CaseDev *cs)
+{
+    const CaseDev &c = cs[blockIdx.y];
+    const Ctrl *ct = c.ctrl;
+    const int g = blockIdx.x * 256 + threadIdx.x;
+    if (g >= ct->ng || !ct->active) return;
+    ghost_vel(c, fld<TS>(c.u[ct->ad_base]), fld<TS>(c.v[ct->ad_base]), g);
+}
+
+// The end of a viscous iteration, one block per case: ghost cells of the new
+// iterate (twelve waves), and the stopping rule of ADSolver.cu:315 (the first
+// four, summing the partials in the fixed order).  One launch where the ghost
+// cells and the rule took two: at 64^2 an iteration's kernels last 2 us each,
+// and the launches between them bound the loop.
+constexpr int kAdFinish = 1024, kAdGhost0 = kAdFinish - 256;
+template <typename TS>
+__global__ __launch_bounds__(kAdFinish) void k_ad_finish(const CaseDev *cs, int ncase)
+{
+    const CaseDev &c = cs[blockIdx.x];
+    Ctrl *ct = c.ctrl;
+    if (!ct->active || ct->ad_done) return;
+    const int buf = 1 - ct->ad_base, ng = ct->ng;
+    TS *u = fld<TS>(c.u[buf]), *v = fld<TS>(c.v[buf]);
+    double s = 0.0;
+    if (threadIdx.x < 256) {
+        const int nt = c.ntx * c.nty;
+        const double *part = c.part;
+        int k = threadIdx.x;
+        for (; k + 768 < nt; k += 1024) {  // four loads in flight, added in order
+            const double a = part[k], b = part[k + 256], d = part[k + 512], e = part[k + 768];
+            s += a;
+            s += b;
+            s += d;
+            s += e;
+        }
+        for (; k < nt; k += 256) s += part[k];
+    } else {
+        for (int g = (int)threadIdx.x - 256; g < ng; g += kAdGhost0) ghost_vel(c, u, v, g);
+    }
+    __shared__ double sw[4];
+    s = wave_sum(s);
+    if (threadIdx.x < 256 && (threadIdx.x & 63) == 0) sw[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        s = (sw[0] + sw[1]) + (sw[2] + sw[3]);
+        ct->ad_res = s;
+        ct->ad_iter += 1;
+        ct->ad_base ^= 1;
+        ct->tot_ad += 1;
+        if (!(s <= 1.0e300)) ct->failed = 1;
+        if (!(s > c.ad_tol) || ct->ad_iter >= c.ad_itermax) {
+            ct->ad_done = 1;
+            ct->ppe_done = 0;  // opens the Poisson loop (k_step_begin)
+        }
+    }
 }
 
 // Pressure: homogeneous Neumann on the domain ring (edges), then ghost
@@ -1088,16 +1117,103 @@ void launch_line_sor(hipStream_t st, int prec, const CaseDev *cs, int ncase, int
     }
 }
 
-// FP64 residual r = rhs - A p (max norm per tile) after a chunk of K sweeps
-// done in launches of M sweeps (K = 0: the check before any sweep).
-__global__ __launch_bounds__(256) void k_ppe_resid(const CaseDev *cs, const int2 *tiles,
-                                                   int ntiles, int ntiles_pad, int K)
+// The end of a convergence check.  Each tile of an iterating case has its
+// maximum m; the case's last tile to arrive takes the maximum over them and
+// applies the stopping rule (FP64: the ping-pong base advances by the chunk's
+// launches; mixed: it flips once when an update happened); the check's last
+// case tells the host.  One launch, with no copy behind it, where the rule
+// was a second kernel and the host read a copy of the control blocks: 10 us
+// per check of a small grid.  Partials and counters go through device scope
+// (tiles run on all XCDs); m is the block's maximum in thread 0.
+// bar->err: a neighbour wait of the persistent sweep has timed out: the loop
+// ends here too (ppe_done, not failed); the host then solves again with one
+// launch per stage.
+__device__ __forceinline__ void check_case(const CaseDev *cs, int ncase, bool open, bool ad_open, GridBar *bar)
+{
+    if (open) __hip_atomic_fetch_add(&bar->open, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (ad_open) __hip_atomic_fetch_add(&bar->ad_open, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+    if (__hip_atomic_fetch_add(&bar->cases, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (unsigned)ncase - 1)
+        return;
+    const unsigned nopen = __hip_atomic_exchange(&bar->open, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned nad = __hip_atomic_exchange(&bar->ad_open, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned err = __hip_atomic_load(&bar->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&bar->cases, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long k = bar->checks + 1;
+    bar->checks = k;
+    __hip_atomic_store(bar->host, k << 3 | (nopen == 0 ? kProgDone : 0) | (nad ? kProgAdOpen : 0) | (err ? kProgErr : 0),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// false: the case takes no part in this check (tile 0 counts it)
+__device__ __forceinline__ bool check_open(const CaseDev *cs, const TileCtx &tc, int ncase, GridBar *bar)
+{
+    const Ctrl *ct = cs[tc.cid].ctrl;
+    if (ct->active && !ct->ppe_done) return true;
+    if (tc.t == 0 && threadIdx.x == 0) check_case(cs, ncase, false, ct->active && !ct->ad_done, bar);
+    return false;
+}
+
+__device__ __forceinline__ void check_end(const CaseDev *cs, const TileCtx &tc, int ncase, int K, bool mixed, double m,
+                                          GridBar *bar)
+{
+    const CaseDev &c = cs[tc.cid];
+    Ctrl *ct = c.ctrl;
+    const unsigned nt = (unsigned)(c.ntx * c.nty);
+    __shared__ unsigned last;
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(&c.part[tc.t], m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+        last = __hip_atomic_fetch_add(&ct->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nt - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    // four independent loads in flight per thread (the maximum does not
+    // depend on the order)
+    auto part = [&](unsigned k) {
+        return __hip_atomic_load(&c.part[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    double m0 = 0.0, m1 = 0.0, m2 = 0.0, m3 = 0.0;
+    unsigned k = threadIdx.x;
+    for (; k + 768 < nt; k += 1024) {
+        m0 = fmax(m0, part(k));
+        m1 = fmax(m1, part(k + 256));
+        m2 = fmax(m2, part(k + 512));
+        m3 = fmax(m3, part(k + 768));
+    }
+    for (; k < nt; k += 256) m0 = fmax(m0, part(k));
+    m = block_max(fmax(fmax(m0, m1), fmax(m2, m3)));
+    if (threadIdx.x != 0) return;
+    ct->ticket = 0;
+    int kexec = c.ppe_itermax - ct->ppe_sweeps;
+    if (kexec > K) kexec = K;
+    const int nl = (kexec + c.ppe_m - 1) / c.ppe_m;  // launches of the chunk
+    ct->ppe_sweeps += kexec;
+    ct->tot_ppe += kexec;
+    if (mixed) {
+        if (kexec > 0) ct->ppe_base ^= 1;
+    } else {
+        ct->ppe_base = (ct->ppe_base + nl) & 1;
+    }
+    const double res = c.dt * m;
+    ct->ppe_res = res;
+    if (!(res <= 1.0e300)) ct->failed = 1;
+    bool done = !(res > c.ppe_tol) || ct->ppe_sweeps >= c.ppe_itermax || ct->failed;
+    if (__hip_atomic_load(&bar->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) done = true;
+    if (done) ct->ppe_done = 1;
+    check_case(cs, ncase, !done, false, bar);
+}
+
+// FP64 residual r = rhs - A p (max norm) after a chunk of K sweeps done in
+// launches of M sweeps (K = 0: the check before any sweep), and the check.
+__global__ __launch_bounds__(256) void k_ppe_resid(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pad,
+                                                   int K, int ncase, GridBar *bar)
 {
     TileCtx tc;
     if (!tile_setup(tiles, ntiles, ntiles_pad, cs, tc)) return;
+    if (!check_open(cs, tc, ncase, bar)) return;
     const CaseDev &c = cs[tc.cid];
     const Ctrl *ct = c.ctrl;
-    if (!ct->active || ct->ppe_done) return;
     int kexec = c.ppe_itermax - ct->ppe_sweeps;
     if (kexec > K) kexec = K;
     const int nl = (kexec + c.ppe_m - 1) / c.ppe_m;  // launches of the chunk
@@ -1124,21 +1240,21 @@ __global__ __launch_bounds__(256) void k_ppe_resid(const CaseDev *cs, const int2
             m = fmax(m, absinf(rr));
         }
     }
-    m = block_max(m);
-    if (threadIdx.x == 0) c.part[tc.t] = m;
+    check_end(cs, tc, ncase, K, false, block_max(m), bar);
 }
 
 // Mixed precision: p_new = p + e (FP64) after a chunk of FP32 error sweeps,
 // then the FP64 residual of p_new, stored as FP32 for the next chunk
-// (defect correction / iterative refinement).  K = 0: residual only.
-__global__ __launch_bounds__(256) void k_ppe_update_resid(const CaseDev *cs, const int2 *tiles,
-                                                          int ntiles, int ntiles_pad, int K)
+// (defect correction / iterative refinement), and the check.  K = 0: residual
+// only.
+__global__ __launch_bounds__(256) void k_ppe_update_resid(const CaseDev *cs, const int2 *tiles, int ntiles,
+                                                          int ntiles_pad, int K, int ncase, GridBar *bar)
 {
     TileCtx tc;
     if (!tile_setup(tiles, ntiles, ntiles_pad, cs, tc)) return;
+    if (!check_open(cs, tc, ncase, bar)) return;
     const CaseDev &c = cs[tc.cid];
     const Ctrl *ct = c.ctrl;
-    if (!ct->active || ct->ppe_done) return;
     int kexec = c.ppe_itermax - ct->ppe_sweeps;
     if (kexec > K) kexec = K;
     const int nl = (kexec + c.ppe_m - 1) / c.ppe_m;  // launches of the chunk
@@ -1182,53 +1298,7 @@ __global__ __launch_bounds__(256) void k_ppe_update_resid(const CaseDev *cs, con
             c.r32[id] = r32;
         }
     }
-    m = block_max(m);
-    if (threadIdx.x == 0) c.part[tc.t] = m;
-}
-
-// One block per case: the Poisson stopping rule on the device.
-// nl_rule: 0 = FP64 ping-pong (base advances by the launch count),
-//          1 = mixed (base flips once when an update happened).
-// bar (persistent chunks only): once a neighbour wait of the persistent
-// sweep has timed out, the loop ends here too (ppe_done, not failed); the
-// host then solves again with one launch per stage.
-__global__ __launch_bounds__(256) void k_ppe_finalize(const CaseDev *cs, int ncase, int K, int mixed,
-                                                      const GridBar *bar)
-{
-    const CaseDev &c = cs[blockIdx.x];
-    Ctrl *ct = c.ctrl;
-    if (!ct->active || ct->ppe_done) return;
-    const int nt = c.ntx * c.nty;
-    // four independent loads in flight per thread (the maximum does not
-    // depend on the order)
-    const double *part = c.part;
-    double m0 = 0.0, m1 = 0.0, m2 = 0.0, m3 = 0.0;
-    int k = threadIdx.x;
-    for (; k + 768 < nt; k += 1024) {
-        m0 = fmax(m0, part[k]);
-        m1 = fmax(m1, part[k + 256]);
-        m2 = fmax(m2, part[k + 512]);
-        m3 = fmax(m3, part[k + 768]);
-    }
-    for (; k < nt; k += 256) m0 = fmax(m0, part[k]);
-    double m = block_max(fmax(fmax(m0, m1), fmax(m2, m3)));
-    if (threadIdx.x == 0) {
-        int kexec = c.ppe_itermax - ct->ppe_sweeps;
-        if (kexec > K) kexec = K;
-        const int nl = (kexec + c.ppe_m - 1) / c.ppe_m;  // launches of the chunk
-        ct->ppe_sweeps += kexec;
-        ct->tot_ppe += kexec;
-        if (mixed) {
-            if (kexec > 0) ct->ppe_base ^= 1;
-        } else {
-            ct->ppe_base = (ct->ppe_base + nl) & 1;
-        }
-        const double res = c.dt * m;
-        ct->ppe_res = res;
-        if (!(res <= 1.0e300)) ct->failed = 1;
-        if (!(res > c.ppe_tol) || ct->ppe_sweeps >= c.ppe_itermax || ct->failed) ct->ppe_done = 1;
-        if (bar && __hip_atomic_load(&bar->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) ct->ppe_done = 1;
-    }
+    check_end(cs, tc, ncase, K, true, block_max(m), bar);
 }
 
 // Re-open the Poisson loop of every running case (after a persistent chunk
@@ -1438,17 +1508,18 @@ void launch_ad_sweep(hipStream_t st, int prec, const CaseDev *cs, const int2 *ti
         hipLaunchKernelGGL(k_ad_sweep<float>, tile_grid(nt), dim3(256), 0, st, cs, tiles, nt, tile_pad(nt));
 }
 
-void launch_ad_finalize(hipStream_t st, const CaseDev *cs, int ncase)
+void launch_ad_finish(hipStream_t st, int prec, const CaseDev *cs, int ncase)
 {
-    hipLaunchKernelGGL(k_ad_finalize, dim3(ncase), dim3(256), 0, st, cs, ncase);
+    if (prec == IF_FP64) hipLaunchKernelGGL(k_ad_finish<double>, dim3(ncase), dim3(kAdFinish), 0, st, cs, ncase);
+    else hipLaunchKernelGGL(k_ad_finish<float>, dim3(ncase), dim3(kAdFinish), 0, st, cs, ncase);
 }
 
-void launch_ghost_vel(hipStream_t st, int prec, const CaseDev *cs, int ncase, int max_ng, int mode)
+void launch_ghost_vel(hipStream_t st, int prec, const CaseDev *cs, int ncase, int max_ng)
 {
     if (max_ng <= 0) return;
     dim3 g((max_ng + 255) / 256, ncase);
-    if (prec == IF_FP64) hipLaunchKernelGGL(k_ghost_vel<double>, g, dim3(256), 0, st, cs, mode);
-    else hipLaunchKernelGGL(k_ghost_vel<float>, g, dim3(256), 0, st, cs, mode);
+    if (prec == IF_FP64) hipLaunchKernelGGL(k_ghost_vel<double>, g, dim3(256), 0, st, cs);
+    else hipLaunchKernelGGL(k_ghost_vel<float>, g, dim3(256), 0, st, cs);
 }
 
 void launch_pressure_bc(hipStream_t st, const CaseDev *cs, int ncase, int max_ring, int max_ng)
@@ -1544,14 +1615,13 @@ void launch_ppe_sweep(hipStream_t st, int prec, int solver, int ty, int m, const
 }
 
 void launch_ppe_check(hipStream_t st, int prec, const CaseDev *cs, int ncase, const int2 *tiles,
-                      int nt, int K, const GridBar *bar)
+                      int nt, int K, GridBar *bar)
 {
     if (prec == IF_FP64)
-        hipLaunchKernelGGL(k_ppe_resid, tile_grid(nt), dim3(256), 0, st, cs, tiles, nt, tile_pad(nt), K);
+        hipLaunchKernelGGL(k_ppe_resid, tile_grid(nt), dim3(256), 0, st, cs, tiles, nt, tile_pad(nt), K, ncase, bar);
     else
         hipLaunchKernelGGL(k_ppe_update_resid, tile_grid(nt), dim3(256), 0, st, cs, tiles, nt,
-                           tile_pad(nt), K);
-    hipLaunchKernelGGL(k_ppe_finalize, dim3(ncase), dim3(256), 0, st, cs, ncase, K, prec == IF_FP64 ? 0 : 1, bar);
+                           tile_pad(nt), K, ncase, bar);
 }
 
 void launch_project(hipStream_t st, int prec, const CaseDev *cs, const int2 *tiles, int nt)

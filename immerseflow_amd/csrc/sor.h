@@ -18,6 +18,10 @@ __device__ __forceinline__ int tile_of_block(int ntiles_pad)
     return (b & 7) * per + (b >> 3);
 }
 
+// s_waitcnt operand (gfx9 encoding) waiting for vmcnt = 0 only: vmcnt
+// bits 3:0 and 15:14 zero, expcnt (6:4) and lgkmcnt (11:8) at their maxima
+constexpr int kWaitVmcnt0 = 0x0F70;
+
 // Global-memory accessors: pointers read from the case descriptor are
 // generic; casting them to the global address space makes the compiler
 // emit global_load/store instead of flat accesses (which also count against

@@ -191,9 +191,6 @@ __device__ __forceinline__ void fast_rows(ROW &&row, PUB &&publish)
 // host checks err after the step.
 constexpr int kDev = 16;                             // cache policy: sc1 (device scope)
 constexpr unsigned kRsrc3 = 0x00020000;              // buffer resource word 3 (gfx9)
-// s_waitcnt operand (gfx9 encoding) waiting for vmcnt = 0 only: vmcnt
-// bits 3:0 and 15:14 zero, expcnt (6:4) and lgkmcnt (11:8) at their maxima
-constexpr int kWaitVmcnt0 = 0x0F70;
 
 // wait (wave 0; lanes 0-7 one neighbour each, nb < 0: none) until every
 // flags[nb] has reached target; true: give up.  The error flag is read by the

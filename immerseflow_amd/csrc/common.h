@@ -106,7 +106,7 @@ struct Ctrl {
     int ppe_done, ppe_sweeps, ppe_base;
     int ng;            // live ghost-cell count (rebuilt on the device for moving bodies)
     int ng_total;      // ghost cells found by the last build (may exceed capacity)
-    unsigned ticket;   // tiles that have finished the running convergence check
+    unsigned ticket;   // tiles (or groups of them) through the running convergence check
     double ad_res, ppe_res, div_max;
     double t;          // simulated time
     long long tot_ad, tot_ppe;
@@ -124,7 +124,9 @@ struct GridBar {
     unsigned long long timeout;
     unsigned long long checks;
     unsigned long long *host;
+    unsigned *tickets;  // kTicketGroups counters per case, kTicketStride apart
 };
+constexpr int kTicketGroups = 32, kTicketStride = 16;
 enum : unsigned { kProgDone = 1, kProgAdOpen = 2, kProgErr = 4 };
 
 // Everything a kernel needs to know about one case.

@@ -141,6 +141,7 @@ public:
     long long persistent_timeouts = 0;  // persistent chunks re-solved per stage
 
 private:
+    unsigned *d_tickets_ = nullptr;  // the checks' group counters (GridBar)
     GridBar *d_bar_ = nullptr;     // error flag of the persistent sweep
     unsigned *d_flags_ = nullptr;  // its per-tile stage counters
     int cap_flags_ = 0;

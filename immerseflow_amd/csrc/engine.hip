@@ -55,6 +55,7 @@ Engine::~Engine()
     if (d_cases_) hipFree(d_cases_);
     if (d_ctrl_) hipFree(d_ctrl_);
     if (d_bar_) hipFree(d_bar_);
+    if (d_tickets_) hipFree(d_tickets_);
     if (d_flags_) hipFree(d_flags_);
     if (d_tiles_base_) hipFree(d_tiles_base_);
     if (d_tiles_sweep_) hipFree(d_tiles_sweep_);
@@ -80,6 +81,10 @@ if_status Engine::init()
     *h_prog_ = 0;
     GridBar b{};
     IFF_HIP(hipHostGetDevicePointer((void **)&b.host, (void *)h_prog_, 0));
+    const size_t tickets = sizeof(unsigned) * kTicketGroups * kTicketStride * cap_ctrl_;
+    IFF_HIP(hipMalloc(&d_tickets_, tickets));
+    IFF_HIP(hipMemsetAsync(d_tickets_, 0, tickets, st_));
+    b.tickets = d_tickets_;
     b.timeout = 2000000;
     if (const char *e = std::getenv("IFF_PERSISTENT_TIMEOUT_TICKS")) b.timeout = std::strtoull(e, nullptr, 10);
     IFF_HIP(hipMemcpyAsync(d_bar_, &b, sizeof(GridBar), hipMemcpyHostToDevice, st_));

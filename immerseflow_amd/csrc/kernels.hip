@@ -1164,7 +1164,20 @@ __device__ __forceinline__ void check_end(const CaseDev *cs, const TileCtx &tc, 
     if (threadIdx.x == 0) {
         __hip_atomic_store(&c.part[tc.t], m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-        last = __hip_atomic_fetch_add(&ct->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nt - 1;
+        // tickets of one address are served one after another, about 20 ns
+        // each, so beyond 128 tiles they are taken in groups first (a check of
+        // 16 resident cases of 64^2 .. 2048^2: 203 us, in groups 126)
+        unsigned n = nt;
+        bool go = true;
+        if (nt > 128) {
+            const unsigned g = (unsigned)tc.t % kTicketGroups;
+            unsigned *tk = bar->tickets + ((size_t)tc.cid * kTicketGroups + g) * kTicketStride;
+            n = kTicketGroups;
+            go = __hip_atomic_fetch_add(tk, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                 (nt - g + kTicketGroups - 1) / kTicketGroups - 1;
+            if (go) __hip_atomic_store(tk, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        last = go && __hip_atomic_fetch_add(&ct->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
     }
     __syncthreads();
     if (!last) return;

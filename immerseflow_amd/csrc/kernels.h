@@ -55,6 +55,11 @@ void launch_project(hipStream_t st, int prec, const CaseDev *cs, const int2 *til
 void launch_step_end(hipStream_t st, const CaseDev *cs, int ncase);
 void launch_monitor(hipStream_t st, int prec, const CaseDev *cs, int ncase, const int2 *tiles, int nt,
                     int sample = 0, double *part = nullptr);
+// the rectangle (i0, j0), w x h of a pitched field to a dense double array and
+// back (flags and iblank: to the dense array only)
+enum class FieldType { f64, f32, iblank, flags };
+void launch_pack(hipStream_t st, FieldType type, const void *f, int P, int i0, int j0, int w, int h, double *d);
+void launch_unpack(hipStream_t st, FieldType type, void *f, int P, int i0, int j0, int w, int h, const double *d);
 void launch_fill_tiles(hipStream_t st, int2 *tiles, int nt);
 // device time stamps of the Poisson chunks (buf[0]: count, then the stamps)
 void launch_stamp(hipStream_t st, unsigned long long *buf, int cap);

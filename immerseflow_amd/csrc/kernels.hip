@@ -14,6 +14,8 @@
 //
 // Expressions are evaluated in the operation order of the reference kernels
 // (and of the FP64 oracle), compiled without FP contraction.
+#include <algorithm>
+
 #include "common.h"
 #include "kernels.h"
 #include "sor.h"
@@ -1780,6 +1782,58 @@ void launch_stamp(hipStream_t st, unsigned long long *buf, int cap)
 void launch_stamp_reset(hipStream_t st, unsigned long long *buf)
 {
     hipLaunchKernelGGL(k_stamp_reset, dim3(1), dim3(64), 0, st, buf);
+}
+
+// Field rectangles between the pitched layout and a dense array (the
+// reference's).  A row per block row: bound by memory, both sides coalesced.
+template <FieldType F>
+__global__ __launch_bounds__(256) void k_pack(const void *f, int P, int i0, int j0, int w, int h, double *d)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= w) return;
+    for (int j = blockIdx.y; j < h; j += gridDim.y) {
+        const size_t src = (size_t)(j0 + j) * P + i0 + i;
+        double v;
+        if constexpr (F == FieldType::f64) v = ((const double *)f)[src];
+        else if constexpr (F == FieldType::f32) v = (double)((const float *)f)[src];
+        else if constexpr (F == FieldType::iblank) v = (((const uint8_t *)f)[src] & F_FLUID) ? 1.0 : 0.0;
+        else v = (double)((const uint8_t *)f)[src];
+        d[(size_t)j * w + i] = v;
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_unpack(T *f, int P, int i0, int j0, int w, int h, const double *d)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= w) return;
+    for (int j = blockIdx.y; j < h; j += gridDim.y) f[(size_t)(j0 + j) * P + i0 + i] = (T)d[(size_t)j * w + i];
+}
+
+static dim3 rect_grid(int w, int h) { return dim3((unsigned)((w + 255) / 256), (unsigned)std::min(h, 32768)); }
+
+void launch_pack(hipStream_t st, FieldType type, const void *f, int P, int i0, int j0, int w, int h, double *d)
+{
+    const dim3 g = rect_grid(w, h);
+    switch (type) {
+    case FieldType::f64: hipLaunchKernelGGL(k_pack<FieldType::f64>, g, dim3(256), 0, st, f, P, i0, j0, w, h, d); break;
+    case FieldType::f32: hipLaunchKernelGGL(k_pack<FieldType::f32>, g, dim3(256), 0, st, f, P, i0, j0, w, h, d); break;
+    case FieldType::iblank:
+        hipLaunchKernelGGL(k_pack<FieldType::iblank>, g, dim3(256), 0, st, f, P, i0, j0, w, h, d);
+        break;
+    case FieldType::flags:
+        hipLaunchKernelGGL(k_pack<FieldType::flags>, g, dim3(256), 0, st, f, P, i0, j0, w, h, d);
+        break;
+    }
+}
+
+void launch_unpack(hipStream_t st, FieldType type, void *f, int P, int i0, int j0, int w, int h, const double *d)
+{
+    const dim3 g = rect_grid(w, h);
+    if (type == FieldType::f64)
+        hipLaunchKernelGGL(k_unpack<double>, g, dim3(256), 0, st, (double *)f, P, i0, j0, w, h, d);
+    else if (type == FieldType::f32)
+        hipLaunchKernelGGL(k_unpack<float>, g, dim3(256), 0, st, (float *)f, P, i0, j0, w, h, d);
 }
 
 // The tile table of one case, tiles (0, t) for t < nt, written on the device.

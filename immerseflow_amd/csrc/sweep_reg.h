@@ -182,7 +182,7 @@ __device__ __forceinline__ void fast_rows(ROW &&row, PUB &&publish)
 // stage counter (flags[t], advanced by the number of stages per launch by
 // every tile, so all counters agree when a launch starts).  A block
 // publishes "stage l done" after its border strips are written, then waits
-// until the 8 neighbouring tiles of its case have published the same stage.
+// until the tiles of its case that its halo reaches have published the same stage.
 // Strips are written and halos read at device scope (sc1: write-through,
 // and loads that miss in the per-XCD L2), so no cache flush is needed; the
 // waits are bounded: past bar->timeout ticks of the 100 MHz real-time
@@ -192,7 +192,7 @@ __device__ __forceinline__ void fast_rows(ROW &&row, PUB &&publish)
 constexpr int kDev = 16;                             // cache policy: sc1 (device scope)
 constexpr unsigned kRsrc3 = 0x00020000;              // buffer resource word 3 (gfx9)
 
-// wait (wave 0; lanes 0-7 one neighbour each, nb < 0: none) until every
+// wait (wave 0; a lane for each neighbour, nb < 0: none) until every
 // flags[nb] has reached target; true: give up.  The error flag is read by the
 // other lanes of the same load, so a stage costs one memory round trip after
 // its last neighbour, not one more for the flag.
@@ -205,6 +205,27 @@ __device__ __forceinline__ bool wait_neighbours(const unsigned *flags, int nb, u
         const unsigned v = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (__any(nb < 0 && v != 0)) return true;
         if (__all(nb < 0 || (int)(v - target) >= 0)) return false;
+        if (__builtin_amdgcn_s_memrealtime() - t0 > tmo) {
+            __hip_atomic_store(&bar->err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return true;
+        }
+        __builtin_amdgcn_s_sleep(1);
+    }
+}
+
+// the same for all n tiles of a case, by all threads of the block (the
+// answer is this wave's)
+__device__ __forceinline__ bool wait_all(const unsigned *flags, int n, unsigned target, GridBar *bar)
+{
+    const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+    const unsigned long long tmo = bar->timeout;
+    while (true) {
+        bool ok = true;
+        for (int i = threadIdx.x; i < n; i += blockDim.x)
+            ok = ok && (int)(__hip_atomic_load(&flags[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - target) >= 0;
+        const unsigned err = __hip_atomic_load(&bar->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__any(err != 0)) return true;
+        if (__all(ok)) return false;
         if (__builtin_amdgcn_s_memrealtime() - t0 > tmo) {
             __hip_atomic_store(&bar->err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return true;
@@ -600,11 +621,15 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
         const int ms = ntxs * ntys == 1 && kexec > M ? kexec : M;
         const int nexec = (kexec + ms - 1) / ms;  // stages with sweeps for this case
         const unsigned f0 = __hip_atomic_load(&flags[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // the neighbouring tiles of the case (lanes 0-7 of wave 0)
+        // the tiles of the case that this one's halo reaches into (a lane of
+        // wave 0 each): the next columns of tiles, and RY rows of them where
+        // the tile is lower than its halo
+        constexpr int RY = (H + TY - 1) / TY, NB = 3 * (2 * RY + 1) - 1;
+        static_assert(TW >= H && NB < 64, "halo reach");
         int nb = -1;
-        if (w == 0 && lane < 8) {
-            const int d = lane < 4 ? lane : lane + 1;  // 3 x 3 without the centre
-            const int qx = tx + d % 3 - 1, qy = ty + d / 3 - 1;
+        if (w == 0 && lane < NB) {
+            const int d = lane < NB / 2 ? lane : lane + 1;  // without the centre
+            const int qx = tx + d % 3 - 1, qy = ty + d / 3 - RY;
             if (qx >= 0 && qx < ntxs && qy >= 0 && qy < ntys) nb = t - tl.y + qy * ntxs + qx;
         }
         const int nrec = P * ny * (int)sizeof(T);  // bytes of a field
@@ -691,17 +716,67 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
                 }
             }
             if (last) break;
-            // publish stage l once every wave's stores are complete, wait
-            // for the neighbours' stage l
-            __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-            __syncthreads();
-            if (threadIdx.x == 0)
-                __hip_atomic_store(&flags[t], f0 + (unsigned)(l + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            // after a timed-out wait anywhere in the launch, stop sweeping:
-            // the error buffers keep finite values, the step reports the
-            // failure and the solve resumes from the current pressure
-            const bool bad = w == 0 && wait_neighbours(flags, nb, f0 + (unsigned)(l + 1), bar);
-            if (__builtin_amdgcn_readfirstlane(__syncthreads_or(bad))) break;
+            if (check && threadIdx.x == 0) {
+                double m = red[0];
+#pragma unroll
+                for (int q = 1; q < NW; q++) m = fmax(m, red[sizeof(T) == 8 ? q : 0]);
+                __hip_atomic_store(&pa.vals[(size_t)(chunk & 1) * ntiles + t], m, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            }
+            if (!alone) {
+                // publish stage l once every wave's stores are complete, wait
+                // for the neighbours' stage l (at a check: every tile's)
+                __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+                __syncthreads();
+                if (threadIdx.x == 0)
+                    __hip_atomic_store(&flags[t], f0 + (unsigned)(l + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                // after a timed-out wait anywhere in the launch, stop sweeping:
+                // the fields keep finite values, the step reports the
+                // failure and the solve resumes from the current pressure
+                const bool bad = check ? wait_all(flags + (t - tl.y), ntxs * ntys, f0 + (unsigned)(l + 1), bar)
+                                       : w == 0 && wait_neighbours(flags, nb, f0 + (unsigned)(l + 1), bar);
+                if (__builtin_amdgcn_readfirstlane(__syncthreads_or(bad))) {
+                    // (at a check other tiles may have seen every flag and end
+                    // here: this one leaves its part of the result too)
+                    whole = check;
+                    if (solve && tl.y == 0 && threadIdx.x == 0) {
+                        ctw->ppe_done = 1;
+                        check_case(pa.ncase, false, false, bar);
+                    }
+                    break;
+                }
+            }
+            if (check) {
+                double m = 0.0;
+                if (alone) {
+                    for (int q = lane; q < NW; q += 64) m = red[sizeof(T) == 8 ? q : 0];
+                } else {
+                    for (int q = lane; q < ntxs * ntys; q += 64)
+                        m = fmax(m, __hip_atomic_load(&pa.vals[(size_t)(chunk & 1) * ntiles + (t - tl.y) + q],
+                                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                }
+                const double res = c.dt * uniform(wave_max(m));
+                done += kc;
+                chunk++;
+                const bool failed = !(res <= 1.0e300);
+                const bool stop = !(res > c.ppe_tol) || done >= left || failed;
+                if (stop || chunk == pa.nchunk) {
+                    whole = true;
+                    if (tl.y == 0 && threadIdx.x == 0) {
+                        ctw->ppe_sweeps += done;
+                        ctw->tot_ppe += done;
+                        ctw->ppe_base = (base + l + 1) & 1;
+                        ctw->ppe_res = res;
+                        if (failed) ctw->failed = 1;
+                        if (stop) ctw->ppe_done = 1;
+                        check_case(pa.ncase, !stop, false, bar);
+                    }
+                    break;
+                }
+                kc = rest = min(K, left - done);
+                if (alone) __syncthreads();  // red is read before the next chunk's maxima
+            }
+            if (alone) continue;
             // halo ring: the cells of the tile outside its stored region
             // that lie in the domain's interior (device-scope loads)
             auto halo = [&](unsigned rows) {

@@ -143,6 +143,7 @@ public:
 private:
     unsigned *d_tickets_ = nullptr;  // the checks' group counters (GridBar)
     GridBar *d_bar_ = nullptr;     // error flag of the persistent sweep
+    double *d_vals_ = nullptr;     // the persistent solve's residuals, two per tile
     unsigned *d_flags_ = nullptr;  // its per-tile stage counters
     int cap_flags_ = 0;
 };

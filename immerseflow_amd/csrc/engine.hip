@@ -25,6 +25,7 @@
 
 namespace iff {
 
+constexpr int kSolveSweeps = 4096;  // sweeps of a persistent FP64 solve launch
 constexpr int kTileY = 16;  // base tiling (reductions, stencil passes)
 
 // viscous iterations enqueued when the last step tells nothing, and at a time
@@ -57,6 +58,7 @@ Engine::~Engine()
     if (d_bar_) hipFree(d_bar_);
     if (d_tickets_) hipFree(d_tickets_);
     if (d_flags_) hipFree(d_flags_);
+    if (d_vals_) hipFree(d_vals_);
     if (d_tiles_base_) hipFree(d_tiles_base_);
     if (d_tiles_sweep_) hipFree(d_tiles_sweep_);
     if (h_prog_) hipHostFree((void *)h_prog_);
@@ -651,7 +653,7 @@ void Engine::enqueue_sweeps(int K, int M, bool any_rb, bool any_jac, bool any_li
     if (stamp) launch_stamp(st_, d_stamps_, kStamps);
     if (any_rb && pers)  // the whole chunk in one launch
         launch_ppe_sweep_pers(st_, pprec_, reg_waves(sweep_kind), tiles_sweep_ty_, M, d_cases_, d_tiles_sweep_, nt_sweep_,
-                              K, d_bar_, d_flags_, wmode_);
+                              K, PersArgs{d_bar_, d_flags_, d_vals_, 0, n}, wmode_);
     for (int s = 0; s < K; s++) {
         if (any_rb && !pers && s % M == 0) {
             if (sweep_kind >= 2)
@@ -821,9 +823,12 @@ if_status Engine::refresh()
     // stage counters of the persistent sweep: one per sweep tile, all equal
     if (nt_sweep_ > cap_flags_) {
         if (d_flags_) hipFree(d_flags_);
+        if (d_vals_) hipFree(d_vals_);
         d_flags_ = nullptr;
+        d_vals_ = nullptr;
         cap_flags_ = std::max(nt_sweep_, 2 * cap_flags_);
         IFF_HIP(hipMalloc(&d_flags_, sizeof(unsigned) * cap_flags_));
+        IFF_HIP(hipMalloc(&d_vals_, 2 * sizeof(double) * cap_flags_));
     }
     if (cap_flags_ > 0) IFF_HIP(hipMemsetAsync(d_flags_, 0, sizeof(unsigned) * cap_flags_, st_));
     tiles_sweep_ty_ = sty;
@@ -916,6 +921,10 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         bool pers = any_rb && use_persistent && sweep_kind >= 2 &&
                     pers_fits(pprec_, reg_waves(sweep_kind), tiles_sweep_ty_, M, nt_sweep_, wmode_);
         if (any_rb) launch_sweeps = pers ? K : M;
+        // FP64: chunks and their checks in one launch, up to kSolveSweeps
+        // sweeps of it (timing brackets single chunks)
+        const bool solve = pprec_ == IF_FP64 && !any_jac && !any_line && !timing;
+        const int nsolve = std::max(1, kSolveSweeps / K);
         // a chunk of one launch gains nothing from a graph
         bool graph = use_graphs && !(pers && !any_jac && !any_line && !timing);
         if_status rc = IF_OK;
@@ -932,6 +941,18 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         auto poisson = [&](bool entry_check) -> if_status {
             const unsigned long long base = checks_;
             if (entry_check) check(0);
+            if (pers && solve) {
+                for (int u = 0; u < nchunks; u += nsolve) {
+                    launch_ppe_sweep_pers(st_, pprec_, reg_waves(sweep_kind), tiles_sweep_ty_, M, d_cases_,
+                                          d_tiles_sweep_, nt_sweep_, K,
+                                          PersArgs{d_bar_, d_flags_, d_vals_, nsolve, n}, wmode_);
+                    checks_++;
+                    if_status r = wait_checks(base, 0, &word);
+                    if (r != IF_OK) return r;
+                    if (word & kProgDone) return IF_OK;
+                }
+                return IF_OK;
+            }
             for (int u = 0; u < nchunks; u++) {
                 if (graph) {
                     const hipError_t e = hipGraphLaunch(g_sweeps_, st_);
@@ -1184,7 +1205,7 @@ if_status Engine::autotune(if_tune_result *out)
         auto timed = [&]() {
             if (pc)
                 launch_ppe_sweep_pers(st_, pprec_, reg_waves(c.kind), c.ty, c.m, d_cases_, d_tiles_sweep_, nt_sweep_, kp,
-                                      d_bar_, d_flags_, wmode_);
+                                      PersArgs{d_bar_, d_flags_, d_vals_, 0, n}, wmode_);
             else
                 sweep_launch(c, s0, 2 * c.m);
         };

@@ -40,8 +40,16 @@ int pers_blocks(int prec, int waves, int ty, int m, int wt);  // 0: no persisten
 // the default shape (kernel 4): tiles(tile_y, m, &most) counts the tiles of all
 // cases and of the largest one
 bool reg_auto_shape(int prec, int wt, const std::function<int(int, int, int *)> &tiles, int *ty, int *m);
+struct PersArgs {
+    GridBar *bar;
+    unsigned *flags;
+    // FP64: chunks of K sweeps, each with its convergence check, up to nchunk
+    // in this launch (0: K sweeps without a check); vals: two values per tile
+    double *vals;
+    int nchunk, ncase;
+};
 void launch_ppe_sweep_pers(hipStream_t st, int prec, int waves, int ty, int m, const CaseDev *cs,
-                           const int2 *tiles, int nt, int K, GridBar *bar, unsigned *flags, int wt);
+                           const int2 *tiles, int nt, int K, const PersArgs &pa, int wt);
 void launch_ppe_check(hipStream_t st, int prec, const CaseDev *cs, int ncase, const int2 *tiles,
                       int nt, int K, GridBar *bar);
 void launch_ppe_rearm(hipStream_t st, const CaseDev *cs, int ncase);

@@ -30,13 +30,6 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
-__device__ __forceinline__ double wave_max(double v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-    return v;
-}
-
 // Block (256 threads) reductions in a fixed order.
 __device__ __forceinline__ double block_sum(double v)
 {
@@ -58,13 +51,6 @@ __device__ __forceinline__ double block_max(double v)
     const double r = fmax(fmax(s[0], s[1]), fmax(s[2], s[3]));
     __syncthreads();
     return r;
-}
-
-// |r| for a max-reduction that lets a non-finite value surface as +inf.
-__device__ __forceinline__ double absinf(double r)
-{
-    const double a = fabs(r);
-    return (a <= 1.0e300) ? a : HUGE_VAL;
 }
 
 template <typename T> __device__ __forceinline__ T *fld(void *p) { return (T *)p; }
@@ -1130,29 +1116,12 @@ void launch_line_sor(hipStream_t st, int prec, const CaseDev *cs, int ncase, int
 // bar->err: a neighbour wait of the persistent sweep has timed out: the loop
 // ends here too (ppe_done, not failed); the host then solves again with one
 // launch per stage.
-__device__ __forceinline__ void check_case(const CaseDev *cs, int ncase, bool open, bool ad_open, GridBar *bar)
-{
-    if (open) __hip_atomic_fetch_add(&bar->open, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (ad_open) __hip_atomic_fetch_add(&bar->ad_open, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-    if (__hip_atomic_fetch_add(&bar->cases, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (unsigned)ncase - 1)
-        return;
-    const unsigned nopen = __hip_atomic_exchange(&bar->open, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned nad = __hip_atomic_exchange(&bar->ad_open, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned err = __hip_atomic_load(&bar->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(&bar->cases, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned long long k = bar->checks + 1;
-    bar->checks = k;
-    __hip_atomic_store(bar->host, k << 3 | (nopen == 0 ? kProgDone : 0) | (nad ? kProgAdOpen : 0) | (err ? kProgErr : 0),
-                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 // false: the case takes no part in this check (tile 0 counts it)
 __device__ __forceinline__ bool check_open(const CaseDev *cs, const TileCtx &tc, int ncase, GridBar *bar)
 {
     const Ctrl *ct = cs[tc.cid].ctrl;
     if (ct->active && !ct->ppe_done) return true;
-    if (tc.t == 0 && threadIdx.x == 0) check_case(cs, ncase, false, ct->active && !ct->ad_done, bar);
+    if (tc.t == 0 && threadIdx.x == 0) check_case(ncase, false, ct->active && !ct->ad_done, bar);
     return false;
 }
 
@@ -1216,7 +1185,7 @@ __device__ __forceinline__ void check_end(const CaseDev *cs, const TileCtx &tc, 
     bool done = !(res > c.ppe_tol) || ct->ppe_sweeps >= c.ppe_itermax || ct->failed;
     if (__hip_atomic_load(&bar->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) done = true;
     if (done) ct->ppe_done = 1;
-    check_case(cs, ncase, !done, false, bar);
+    check_case(ncase, !done, false, bar);
 }
 
 // FP64 residual r = rhs - A p (max norm) after a chunk of K sweeps done in

@@ -159,4 +159,38 @@ __device__ __forceinline__ double from_east(double x)
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
+__device__ __forceinline__ double wave_max(double v)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+    return v;
+}
+
+// |r| for a max-reduction that lets a non-finite value surface as +inf.
+__device__ __forceinline__ double absinf(double r)
+{
+    const double a = fabs(r);
+    return (a <= 1.0e300) ? a : HUGE_VAL;
+}
+
+// One case's part in a convergence check (one thread): still iterating (open),
+// or its viscous loop has not ended yet (ad_open).  The last of the ncase
+// cases tells the host.
+__device__ __forceinline__ void check_case(int ncase, bool open, bool ad_open, GridBar *bar)
+{
+    if (open) __hip_atomic_fetch_add(&bar->open, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (ad_open) __hip_atomic_fetch_add(&bar->ad_open, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+    if (__hip_atomic_fetch_add(&bar->cases, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (unsigned)ncase - 1)
+        return;
+    const unsigned nopen = __hip_atomic_exchange(&bar->open, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned nad = __hip_atomic_exchange(&bar->ad_open, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned err = __hip_atomic_load(&bar->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&bar->cases, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long k = bar->checks + 1;
+    bar->checks = k;
+    __hip_atomic_store(bar->host, k << 3 | (nopen == 0 ? kProgDone : 0) | (nad ? kProgAdOpen : 0) | (err ? kProgErr : 0),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 }  // namespace iff

@@ -25,13 +25,12 @@ static int pers_capacity()
 }
 
 template <typename T, int M, int NW, int NRW>
-static void pers_one(hipStream_t st, const CaseDev *cs, const int2 *tiles, int nt, int K, GridBar *bar,
-                     unsigned *flags, int wt)
+static void pers_one(hipStream_t st, const CaseDev *cs, const int2 *tiles, int nt, int K, const PersArgs &pa, int wt)
 {
     const int pad = ((nt + 7) / 8) * 8;
 #define IFF_PLW(WM_)                                                                                           \
     hipLaunchKernelGGL((k_rbsor_reg<T, M, NW, NRW, true, WM_>), dim3(pad), dim3(64 * NW), 0, st, cs, tiles, nt, \
-                       pad, 0, K, bar, flags)
+                       pad, 0, K, pa)
     if (wt == 1)
         IFF_PLW(1);
     else if (sizeof(T) == 4 && wt == 2)
@@ -124,11 +123,11 @@ bool pers_fits(int prec, int waves, int ty, int m, int nt, int wt)
 }
 
 void launch_ppe_sweep_pers(hipStream_t st, int prec, int waves, int ty, int m, const CaseDev *cs,
-                           const int2 *tiles, int nt, int K, GridBar *bar, unsigned *flags, int wt)
+                           const int2 *tiles, int nt, int K, const PersArgs &pa, int wt)
 {
 #define IFF_PL(T_, W_, M_, TY_, NRW_)                                      \
     if (waves == W_ && m == M_ && ty == TY_) {                            \
-        pers_one<T_, M_, W_, NRW_>(st, cs, tiles, nt, K, bar, flags, wt); \
+        pers_one<T_, M_, W_, NRW_>(st, cs, tiles, nt, K, pa, wt); \
         return;                                                           \
     }
     if (prec == IF_FP64) {

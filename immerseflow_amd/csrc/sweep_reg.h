@@ -253,8 +253,7 @@ __device__ __forceinline__ bool wait_all(const unsigned *flags, int n, unsigned 
 // per CU, a third slower.
 template <typename T, int M, int NW, int NRW, bool PERS, int WM>
 __global__ __launch_bounds__(64 * NW, (sizeof(T) == 4 && NW == 16 && (PERS ? WM == 1 || (WM == 0 && NRW <= 6) : NRW == 8 && WM != 2)) ? 8 : 1)
-void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pad, int s, int K, GridBar *bar,
-                 unsigned *flags)
+void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pad, int s, int K, PersArgs pa)
 {
     constexpr int H = 2 * M;
     constexpr int TW = 128 - 2 * H;   // stored columns per tile
@@ -270,7 +269,10 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
     // 256 LDS cycles, where three rows of updates take about 160.)
     __shared__ T xch[2][NW + 2][2][64];
     const int t = tile_of_block(ntiles_pad);
-    const int nstage = (K + M - 1) / M;  // PERS: stages of the launch
+    const int nstage = (K + M - 1) / M;  // PERS: stages of a plain launch
+    GridBar *const bar = pa.bar;
+    unsigned *const flags = pa.flags;
+    const bool solve = PERS && sizeof(T) == 8 && pa.nchunk > 0;
     if constexpr (PERS) {
         bool run = false;
         if (t < ntiles) {
@@ -279,7 +281,12 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
             run = cr.ppe_solver == IF_PPE_RBSOR && cc->active && !cc->ppe_done && cr.ppe_itermax > cc->ppe_sweeps;
         }
         if (!run) {  // whole workgroup: nobody waits on this tile, advance its counter
-            if (t < ntiles && threadIdx.x == 0) {
+            if (solve) {
+                if (t < ntiles && tiles[t].y == 0 && threadIdx.x == 0) {
+                    const Ctrl *cc = cs[tiles[t].x].ctrl;
+                    check_case(pa.ncase, false, cc->active && !cc->ad_done, bar);
+                }
+            } else if (t < ntiles && threadIdx.x == 0) {
                 const unsigned f0 = __hip_atomic_load(&flags[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_store(&flags[t], f0 + (unsigned)nstage, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
@@ -467,6 +474,9 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
     // keeps: outside the interior, not fluid, or without an open face; its
     // value in the tile is 0).  FP32 weights come from k_weights32; wr = w r
     // is formed here.
+    // FP64, solve: the cells' open faces for the residual (flag bits 0-5 of
+    // slot a in bits 0-5, of slot b in 6-11, two rows a register)
+    unsigned of[PERS && sizeof(T) == 8 ? (NRW + 1) / 2 : 1] = {};
     unsigned smask = 0;  // FP64: rows holding an interior cell that is kept
 #pragma unroll
     for (int k = 0; k < NRW; k++) {
@@ -509,6 +519,7 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
                 R.wa[k] = (rowint && (fa & F_FLUID) && sa_a != (T)0) ? sor_weight64(sa_a, om) : (T)0;
                 R.wb[k] = (rowint && (fb & F_FLUID) && sa_b != (T)0) ? sor_weight64(sa_b, om) : (T)0;
             }
+            if constexpr (PERS) of[k / 2] |= (unsigned)((fa & 63) | (fb & 63) << 6) << (16 * (k & 1));
             if (rowint && __any((ina && R.wa[k] == (T)0) || (inb && R.wb[k] == (T)0))) smask |= 1u << k;
             R.pa[k] = R.wa[k] != (T)0 ? R.pa[k] : (T)0;
             R.pb[k] = R.wb[k] != (T)0 ? R.pb[k] : (T)0;
@@ -618,8 +629,7 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
         // read, so it runs the whole chunk at once, and leaves its output in
         // the last stage's buffer
         const int ntys = (ny - 2 + TY - 1) / TY;
-        const int ms = ntxs * ntys == 1 && kexec > M ? kexec : M;
-        const int nexec = (kexec + ms - 1) / ms;  // stages with sweeps for this case
+        const bool alone = ntxs * ntys == 1;
         const unsigned f0 = __hip_atomic_load(&flags[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // the tiles of the case that this one's halo reaches into (a lane of
         // wave 0 each): the next columns of tiles, and RY rows of them where
@@ -676,15 +686,60 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
         // the buffer accesses
         const __amdgpu_buffer_rsrc_t rs0 = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(buf0), 0, nrec, kRsrc3);
         const __amdgpu_buffer_rsrc_t rs1 = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(buf1), 0, nrec, kRsrc3);
-        for (int l = 0; l < nexec; l++) {
-            int me = kexec - l * ms;
-            if (me > ms) me = ms;
-            sweeps(2 * me);
-            const bool last = l + 1 == nexec;
-            const __amdgpu_buffer_rsrc_t ro = ((ms == M ? l + 1 : (kexec + M - 1) / M) & 1) ? rs1 : rs0;
-            // stage output at device scope: the border strips, or (last
-            // stage of the case) the whole stored region
-            const unsigned m_all = last ? m_st : m_strip;
+        // Solve (FP64, pa.nchunk > 0): the launch runs chunks of K sweeps until
+        // the residual of the case passes its stopping rule, it runs out of
+        // sweeps, or pa.nchunk are done.  A chunk's last stage does at most
+        // M - 1 sweeps, so that a ring of exact cells is left around the
+        // stored region and the tile has its residual from its registers;
+        // the maxima meet at the stage's flags, waited for by the case's tiles all
+        // together.  A launch for each chunk and for each check cost 28 us
+        // per 10 sweeps of a 256^2 grid, of which 11 were sweeps.
+        Ctrl *const ctw = c.ctrl;
+        const int left = uniform(c.ppe_itermax - ct->ppe_sweeps);
+        const int base = uniform(ct->ppe_base);
+        // the residual's maximum over the stored cells, from the tile after a
+        // stage's last sweep: k_ppe_resid's expression and operand order, with
+        // the open faces' coefficients (a kept cell is held as 0, and its
+        // faces are closed).  xch[1 - c] holds the neighbour rows' cells of
+        // colour c.
+        auto residual = [&]() __attribute__((always_inline)) {
+            double m = 0.0;
+            if constexpr (sizeof(T) == 8) {
+                const int cn = (Z + NRW - 1) & 1;
+                const T sa = xch[Z][w][1][lane], sb = xch[1 - Z][w][1][lane];
+                const T na = xch[cn][w + 2][0][lane], nb_ = xch[1 - cn][w + 2][0][lane];
+                auto cell = [&](unsigned f, T pc, T r, T pE, T pW, T pN, T pS, T cxp, T cxm, T cyp, T cym) {
+                    const T aE = face_coef<T, F_OPEN_E>((int)f, cxp), aW = face_coef<T, F_OPEN_W>((int)f, cxm);
+                    const T aN = face_coef<T, F_OPEN_N>((int)f, cyp), aS = face_coef<T, F_OPEN_S>((int)f, cym);
+                    const T ap = -((aE + aW) + (aN + aS));
+                    const T sum = (aE * pE + aW * pW) + (aN * pN + aS * pS);
+                    return absinf(r - (ap * pc + sum));
+                };
+#pragma unroll
+                for (int k = 0; k < NRW; k++) {
+                    if (!((m_st >> k) & 1u)) continue;
+                    // (opaque: the coefficients of all rows, formed once before
+                    // the loop, would not fit in the registers)
+                    asm volatile("" : "+v"(of[k / 2]));
+                    const unsigned f = of[k / 2] >> (16 * (k & 1));
+                    const T pSa = k == 0 ? sa : R.pa[k > 0 ? k - 1 : 0], pSb = k == 0 ? sb : R.pb[k > 0 ? k - 1 : 0];
+                    const T pNa = k == NRW - 1 ? na : R.pa[k < NRW - 1 ? k + 1 : k];
+                    const T pNb = k == NRW - 1 ? nb_ : R.pb[k < NRW - 1 ? k + 1 : k];
+                    const T ma = cell(f & 63, R.pa[k], R.ra[k], R.pb[k], from_west(R.pb[k]), pNa, pSa, cxpa, cxma,
+                                      R.cyp[k], R.cym[k]);
+                    const T mb = cell(f >> 6 & 63, R.pb[k], R.rb[k], from_east(R.pa[k]), R.pa[k], pNb, pSb, cxpb, cxmb,
+                                      R.cyp[k], R.cym[k]);
+                    if (stl && R.wa[k] != (T)0) m = fmax(m, ma);
+                    if (stl && R.wb[k] != (T)0) m = fmax(m, mb);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            return wave_max(m);
+        };
+        // stage output at device scope: the border strips, or (the end of
+        // the case) the whole stored region
+        auto put = [&](const __amdgpu_buffer_rsrc_t ro, bool whole) __attribute__((always_inline)) {
+            const unsigned m_all = whole ? m_st : m_strip;
 #pragma unroll
             for (int k = 0; k < NRW; k++) {
                 const int srow = (jt0 + k) * P * (int)sizeof(T);  // uniform: scalar offset
@@ -715,6 +770,27 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
                                                               R.wa[k] != (T)0 ? vo_one : kDrop, srow, kDev);
                 }
             }
+        };
+        __shared__ double red[sizeof(T) == 8 ? NW : 1];
+        int done = 0, chunk = 0;      // sweeps and chunks behind the running chunk
+        int kc = kexec, rest = kexec;  // sweeps of the running chunk, and what is left of them
+        bool whole = false;
+        int l = 0;
+        for (;; l++) {
+            int me = alone || rest < M ? rest : M;
+            if (solve && !alone && rest == M) me = (M + 1) / 2;
+            sweeps(2 * me);
+            rest -= me;
+            const bool check = solve && rest == 0;
+            const bool last = !solve && rest == 0;
+            // (a plain launch leaves its output where launches of M sweeps do)
+            const __amdgpu_buffer_rsrc_t ro = ((solve || !alone ? l + 1 : (kexec + M - 1) / M) & 1) ? rs1 : rs0;
+            if (check) {
+                const double m = residual();
+                if (lane == 0) red[w] = m;
+                __syncthreads();
+            }
+            if (!alone || last) put(ro, last);
             if (last) break;
             if (check && threadIdx.x == 0) {
                 double m = red[0];
@@ -800,6 +876,10 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
             };
             if (ld_side) halo(m_st);
             if (ldl) halo(m_halo);
+        }
+        if (solve) {  // (every stage has advanced the counter)
+            if (whole) put((l + 1) & 1 ? rs1 : rs0, true);
+            return;
         }
         __syncthreads();
         if (threadIdx.x == 0)

@@ -9,7 +9,7 @@ static void reg_one(hipStream_t st, const CaseDev *cs, const int2 *tiles, int nt
     const int pad = ((nt + 7) / 8) * 8;
 #define IFF_RL(WM_)                                                                                             \
     hipLaunchKernelGGL((k_rbsor_reg<T, M, NW, NRW, false, WM_>), dim3(pad), dim3(64 * NW), 0, st, cs, tiles, nt, \
-                       pad, s, K, (GridBar *)nullptr, (unsigned *)nullptr)
+                       pad, s, K, PersArgs{})
     if (wt == 1)
         IFF_RL(1);
     else if (sizeof(T) == 4 && wt == 2)

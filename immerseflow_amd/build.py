@@ -19,7 +19,7 @@ BUILD = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "libimmerseflow_amd.so")
 CLI = os.path.join(PKG, "immerseflow")
 
-HIP_SOURCES = ["kernels.hip", "sweep_stream.hip", "sweep_reg.hip", "sweep_pers.hip", "geometry.hip", "engine.hip", "compat.hip"]
+HIP_SOURCES = ["kernels.hip", "sweep_stream.hip", "sweep_reg.hip", "sweep_pers.hip", "line_pers.hip", "geometry.hip", "engine.hip", "compat.hip"]
 CPP_SOURCES = ["io.cpp", "abi.cpp"]
 
 COMMON = ["-O3", "-fPIC", "-std=c++20", "-ffp-contract=off",

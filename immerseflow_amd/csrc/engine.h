@@ -94,8 +94,8 @@ private:
     if_status read_ctrl_sync(std::vector<Ctrl> &out);
     if_status update_moving();
     // the K sweeps of one Poisson chunk, as kernel launches on st_
-    void enqueue_sweeps(int K, int M, bool any_rb, bool any_jac, bool any_line, bool pers, bool stamp);
-    if_status capture_sweeps(int K, int M, bool any_rb, bool any_jac, bool any_line, bool pers, bool stamp);
+    void enqueue_sweeps(int K, int M, bool any_rb, bool any_jac, bool any_line, bool pers, bool lpers, bool stamp);
+    if_status capture_sweeps(int K, int M, bool any_rb, bool any_jac, bool any_line, bool pers, bool lpers, bool stamp);
     if_status check_barrier();
     void drop_graph();
 
@@ -133,7 +133,7 @@ private:
     // captured sweep chunk, valid for the resident set of the last
     // refresh() and the launch shape in g_key_
     hipGraphExec_t g_sweeps_ = nullptr;
-    int g_key_[9] = {};
+    int g_key_[10] = {};
     bool g_valid_ = false;     // g_sweeps_ matches the current tables
 
 public:
@@ -146,6 +146,16 @@ private:
     double *d_vals_ = nullptr;     // the persistent solve's residuals, two per tile
     unsigned *d_flags_ = nullptr;  // its per-tile stage counters
     int cap_flags_ = 0;
+    // persistent line SOR: the resident line cases' blocks of rows, a launch
+    // for each number of cells a lane holds; none if any case has no such form
+    struct LineGroup {
+        int B, first, count;
+    };
+    std::vector<LineGroup> line_groups_;
+    int2 *d_line_blocks_ = nullptr;
+    unsigned *d_line_flags_ = nullptr;
+    int cap_line_ = 0;
+    if_status zero_flags();
 };
 
 }  // namespace iff

@@ -59,6 +59,8 @@ Engine::~Engine()
     if (d_tickets_) hipFree(d_tickets_);
     if (d_flags_) hipFree(d_flags_);
     if (d_vals_) hipFree(d_vals_);
+    if (d_line_blocks_) hipFree(d_line_blocks_);
+    if (d_line_flags_) hipFree(d_line_flags_);
     if (d_tiles_base_) hipFree(d_tiles_base_);
     if (d_tiles_sweep_) hipFree(d_tiles_sweep_);
     if (h_prog_) hipHostFree((void *)h_prog_);
@@ -647,13 +649,18 @@ void Engine::drop_graph()
 // given resident set and shape: the kernels read the loop state (buffer
 // parity, sweep counts, done flags) from the control blocks on the device,
 // so a captured chunk replays unchanged.
-void Engine::enqueue_sweeps(int K, int M, bool any_rb, bool any_jac, bool any_line, bool pers, bool stamp)
+void Engine::enqueue_sweeps(int K, int M, bool any_rb, bool any_jac, bool any_line, bool pers, bool lpers,
+                            bool stamp)
 {
     const int n = (int)order_.size();
     if (stamp) launch_stamp(st_, d_stamps_, kStamps);
     if (any_rb && pers)  // the whole chunk in one launch
         launch_ppe_sweep_pers(st_, pprec_, reg_waves(sweep_kind), tiles_sweep_ty_, M, d_cases_, d_tiles_sweep_, nt_sweep_,
                               K, PersArgs{d_bar_, d_flags_, d_vals_, 0, n}, wmode_);
+    if (any_line && lpers)
+        for (const LineGroup &g : line_groups_)
+            launch_line_pers(st_, pprec_, g.B, d_cases_, d_line_blocks_ + g.first, g.count, K,
+                             PersArgs{d_bar_, d_line_flags_ + g.first, nullptr, 0, n});
     for (int s = 0; s < K; s++) {
         if (any_rb && !pers && s % M == 0) {
             if (sweep_kind >= 2)
@@ -667,7 +674,7 @@ void Engine::enqueue_sweeps(int K, int M, bool any_rb, bool any_jac, bool any_li
         }
         if (any_jac)  // point Jacobi runs on the base tiling
             launch_ppe_sweep(st_, pprec_, IF_PPE_JACOBI, kTileY, 1, d_cases_, d_tiles_base_, nt_base_, s, K);
-        if (any_line) launch_line_sor(st_, pprec_, d_cases_, n, max_ring_, s, K);
+        if (any_line && !lpers) launch_line_sor(st_, pprec_, d_cases_, n, max_ring_, s, K);
     }
     if (stamp) launch_stamp(st_, d_stamps_, kStamps);
 }
@@ -680,14 +687,15 @@ void Engine::enqueue_sweeps(int K, int M, bool any_rb, bool any_jac, bool any_li
 // place (hipGraphExecUpdate: new kernel arguments and launch sizes); only
 // a different topology destroys it and instantiates a new one.  The stream
 // is idle whenever this runs (every step ends with a synchronisation).
-if_status Engine::capture_sweeps(int K, int M, bool any_rb, bool any_jac, bool any_line, bool pers, bool stamp)
+if_status Engine::capture_sweeps(int K, int M, bool any_rb, bool any_jac, bool any_line, bool pers, bool lpers,
+                            bool stamp)
 {
-    const int key[9] = {K, M, sweep_kind, tiles_sweep_ty_, (int)any_rb, (int)any_jac, (int)any_line, (int)pers,
-                        (int)stamp};
-    if (g_sweeps_ && g_valid_ && std::equal(key, key + 9, g_key_)) return IF_OK;
+    const int key[10] = {K, M, sweep_kind, tiles_sweep_ty_, (int)any_rb, (int)any_jac, (int)any_line, (int)pers,
+                         (int)lpers, (int)stamp};
+    if (g_sweeps_ && g_valid_ && std::equal(key, key + 10, g_key_)) return IF_OK;
     hipGraph_t g = nullptr;
     IFF_HIP(hipStreamBeginCapture(st_, hipStreamCaptureModeThreadLocal));
-    enqueue_sweeps(K, M, any_rb, any_jac, any_line, pers, stamp);
+    enqueue_sweeps(K, M, any_rb, any_jac, any_line, pers, lpers, stamp);
     hipError_t e = hipStreamEndCapture(st_, &g);
     if (e != hipSuccess) return fail(IF_ERR_HIP, std::string("sweep graph capture: ") + hipGetErrorString(e));
     bool updated = false;
@@ -712,7 +720,7 @@ if_status Engine::capture_sweeps(int K, int M, bool any_rb, bool any_jac, bool a
         graph_instantiations++;
     }
     (void)hipGraphDestroy(g);
-    std::copy(key, key + 9, g_key_);
+    std::copy(key, key + 10, g_key_);
     g_valid_ = true;
     return IF_OK;
 }
@@ -729,7 +737,8 @@ if_status Engine::check_barrier()
     use_persistent = false;
     drop_graph();
     IFF_HIP(hipMemsetAsync(&d_bar_->err, 0, sizeof(unsigned), st_));
-    if (cap_flags_ > 0) IFF_HIP(hipMemsetAsync(d_flags_, 0, sizeof(unsigned) * cap_flags_, st_));
+    const if_status rc = zero_flags();
+    if (rc != IF_OK) return rc;
     IFF_HIP(hipStreamSynchronize(st_));
     return fail(IF_ERR_HIP, "persistent Poisson sweep: a neighbour wait timed out (blocks not co-resident); "
                             "the persistent form is now off");
@@ -830,10 +839,50 @@ if_status Engine::refresh()
         IFF_HIP(hipMalloc(&d_flags_, sizeof(unsigned) * cap_flags_));
         IFF_HIP(hipMalloc(&d_vals_, 2 * sizeof(double) * cap_flags_));
     }
-    if (cap_flags_ > 0) IFF_HIP(hipMemsetAsync(d_flags_, 0, sizeof(unsigned) * cap_flags_, st_));
+    // the persistent line SOR's blocks of rows, grouped by cells a lane
+    line_groups_.clear();
+    std::vector<int2> lb;
+    bool line_ok = true;
+    for (int B = 2; B <= 8; B++) {
+        LineGroup g{B, (int)lb.size(), 0};
+        const int rows = line_pers_rows(pprec_, B);
+        for (int k = 0; k < n; k++) {
+            const Slot &s = *slots_[order_[k]];
+            if (s.desc.ppe_solver != IF_PPE_LINE || s.dev.lB != B || rows == 0) continue;
+            for (int t = 0; t < (s.NY + rows - 1) / rows; t++) lb.push_back(make_int2(k, t));
+        }
+        g.count = (int)lb.size() - g.first;
+        if (g.count > 0) line_groups_.push_back(g);
+        if (g.count > 0 && !line_pers_fits(pprec_, B, g.count)) line_ok = false;
+    }
+    for (int id : order_)
+        if (slots_[id]->desc.ppe_solver == IF_PPE_LINE && line_pers_rows(pprec_, slots_[id]->dev.lB) == 0)
+            line_ok = false;
+    if (!line_ok) line_groups_.clear();
+    if ((int)lb.size() > cap_line_) {
+        if (d_line_blocks_) hipFree(d_line_blocks_);
+        if (d_line_flags_) hipFree(d_line_flags_);
+        d_line_blocks_ = nullptr;
+        d_line_flags_ = nullptr;
+        cap_line_ = std::max((int)lb.size(), 2 * cap_line_);
+        IFF_HIP(hipMalloc(&d_line_blocks_, sizeof(int2) * cap_line_));
+        IFF_HIP(hipMalloc(&d_line_flags_, sizeof(unsigned) * cap_line_));
+    }
+    if (!lb.empty())
+        IFF_HIP(hipMemcpyAsync(d_line_blocks_, lb.data(), sizeof(int2) * lb.size(), hipMemcpyHostToDevice, st_));
+    rc = zero_flags();
+    if (rc != IF_OK) return rc;
     tiles_sweep_ty_ = sty;
     IFF_HIP(hipStreamSynchronize(st_));  // host vectors go out of scope
     dirty_ = false;
+    return IF_OK;
+}
+
+// Every tile's and block's stage counter to 0.
+if_status Engine::zero_flags()
+{
+    if (cap_flags_ > 0) IFF_HIP(hipMemsetAsync(d_flags_, 0, sizeof(unsigned) * cap_flags_, st_));
+    if (cap_line_ > 0) IFF_HIP(hipMemsetAsync(d_line_flags_, 0, sizeof(unsigned) * cap_line_, st_));
     return IF_OK;
 }
 
@@ -921,15 +970,16 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         bool pers = any_rb && use_persistent && sweep_kind >= 2 &&
                     pers_fits(pprec_, reg_waves(sweep_kind), tiles_sweep_ty_, M, nt_sweep_, wmode_);
         if (any_rb) launch_sweeps = pers ? K : M;
+        bool lpers = any_line && use_persistent && !line_groups_.empty();
         // FP64: chunks and their checks in one launch, up to kSolveSweeps
         // sweeps of it (timing brackets single chunks)
         const bool solve = pprec_ == IF_FP64 && !any_jac && !any_line && !timing;
         const int nsolve = std::max(1, kSolveSweeps / K);
         // a chunk of one launch gains nothing from a graph
-        bool graph = use_graphs && !(pers && !any_jac && !any_line && !timing);
+        bool graph = use_graphs && !(!any_jac && (!any_rb || pers) && (!any_line || lpers) && !timing);
         if_status rc = IF_OK;
         if (graph) {
-            rc = capture_sweeps(K, M, any_rb, any_jac, any_line, pers, timing);
+            rc = capture_sweeps(K, M, any_rb, any_jac, any_line, pers, lpers, timing);
             if (rc != IF_OK) return rc;
         }
 
@@ -959,7 +1009,7 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
                     if (e != hipSuccess)
                         return fail(IF_ERR_HIP, std::string("sweep graph launch: ") + hipGetErrorString(e));
                 } else {
-                    enqueue_sweeps(K, M, any_rb, any_jac, any_line, pers, timing);
+                    enqueue_sweeps(K, M, any_rb, any_jac, any_line, pers, lpers, timing);
                 }
                 check(K);
                 if_status r = wait_checks(base, spec_depth - 1, &word);
@@ -1006,16 +1056,17 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
                 // then completes as usual.
                 use_persistent = false;
                 dirty_ = true;  // the default shape is chosen again
-                pers = false;
+                pers = lpers = false;
                 if (agg) agg->persistent_timeouts++;
                 launch_sweeps = M;
                 persistent_timeouts++;
                 IFF_HIP(hipMemsetAsync(&d_bar_->err, 0, sizeof(unsigned), st_));
-                if (cap_flags_ > 0) IFF_HIP(hipMemsetAsync(d_flags_, 0, sizeof(unsigned) * cap_flags_, st_));
+                rc = zero_flags();
+                if (rc != IF_OK) return rc;
                 launch_ppe_rearm(st_, d_cases_, n);
                 graph = use_graphs;
                 if (graph) {
-                    rc = capture_sweeps(K, M, any_rb, any_jac, any_line, false, timing);
+                    rc = capture_sweeps(K, M, any_rb, any_jac, any_line, false, false, timing);
                     if (rc != IF_OK) return rc;
                 }
                 if (timing) launch_stamp_reset(st_, d_stamps_);
@@ -1047,7 +1098,7 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
             const int nfull = std::min(timed, maxsw / K);
             for (int u = 0; u < nfull; u++) {
                 sweep_ms += 1e3 * (double)(h_stamps_[2 + 2 * u] - h_stamps_[1 + 2 * u]) / stamp_hz_;
-                sweep_launches += pers ? 1 : (K + m_eff - 1) / m_eff;
+                sweep_launches += pers || (!any_rb && lpers) ? 1 : (K + m_eff - 1) / m_eff;
             }
             for (int id : order_)
                 sweep_cells += (double)std::min(all[id].ppe_sweeps, nfull * K) *

@@ -50,6 +50,13 @@ struct PersArgs {
 };
 void launch_ppe_sweep_pers(hipStream_t st, int prec, int waves, int ty, int m, const CaseDev *cs,
                            const int2 *tiles, int nt, int K, const PersArgs &pa, int wt);
+// Zebra line SOR, persistent (rows of B cells a lane): rows stored per block (0:
+// no such form), whether that many blocks are resident at once, one chunk of K
+// sweeps.  blocks: (case, block of rows); pa.flags: one counter per block.
+int line_pers_rows(int prec, int B);
+bool line_pers_fits(int prec, int B, int nblocks);
+void launch_line_pers(hipStream_t st, int prec, int B, const CaseDev *cs, const int2 *blocks, int nblocks, int K,
+                      const PersArgs &pa);
 void launch_ppe_check(hipStream_t st, int prec, const CaseDev *cs, int ncase, const int2 *tiles,
                       int nt, int K, GridBar *bar);
 void launch_ppe_rearm(hipStream_t st, const CaseDev *cs, int ncase);

@@ -21,6 +21,7 @@ __device__ __forceinline__ int tile_of_block(int ntiles_pad)
 // s_waitcnt operand (gfx9 encoding) waiting for vmcnt = 0 only: vmcnt
 // bits 3:0 and 15:14 zero, expcnt (6:4) and lgkmcnt (11:8) at their maxima
 constexpr int kWaitVmcnt0 = 0x0F70;
+constexpr int kDev = 16;                             // cache policy: sc1 (device scope)
 
 // Global-memory accessors: pointers read from the case descriptor are
 // generic; casting them to the global address space makes the compiler
@@ -191,6 +192,27 @@ __device__ __forceinline__ void check_case(int ncase, bool open, bool ad_open, G
     bar->checks = k;
     __hip_atomic_store(bar->host, k << 3 | (nopen == 0 ? kProgDone : 0) | (nad ? kProgAdOpen : 0) | (err ? kProgErr : 0),
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Neighbour wait of a persistent sweep (wave 0; a lane for each neighbour,
+// nb < 0: none) until every flags[nb] has reached target; true: give up.  The
+// error flag is read by the other lanes of the same load, so a stage costs one
+// memory round trip after its last neighbour, not one more for the flag.
+__device__ __forceinline__ bool wait_neighbours(const unsigned *flags, int nb, unsigned target, GridBar *bar)
+{
+    const unsigned *at = nb >= 0 ? &flags[nb] : &bar->err;
+    const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+    const unsigned long long tmo = bar->timeout;
+    while (true) {
+        const unsigned v = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__any(nb < 0 && v != 0)) return true;
+        if (__all(nb < 0 || (int)(v - target) >= 0)) return false;
+        if (__builtin_amdgcn_s_memrealtime() - t0 > tmo) {
+            __hip_atomic_store(&bar->err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return true;
+        }
+        __builtin_amdgcn_s_sleep(1);
+    }
 }
 
 }  // namespace iff

@@ -189,31 +189,9 @@ __device__ __forceinline__ void fast_rows(ROW &&row, PUB &&publish)
 // counter bar->err is set, every later wait returns at once and every
 // block stops at its next stage boundary, so the kernel always ends; the
 // host checks err after the step.
-constexpr int kDev = 16;                             // cache policy: sc1 (device scope)
 constexpr unsigned kRsrc3 = 0x00020000;              // buffer resource word 3 (gfx9)
 
-// wait (wave 0; a lane for each neighbour, nb < 0: none) until every
-// flags[nb] has reached target; true: give up.  The error flag is read by the
-// other lanes of the same load, so a stage costs one memory round trip after
-// its last neighbour, not one more for the flag.
-__device__ __forceinline__ bool wait_neighbours(const unsigned *flags, int nb, unsigned target, GridBar *bar)
-{
-    const unsigned *at = nb >= 0 ? &flags[nb] : &bar->err;
-    const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
-    const unsigned long long tmo = bar->timeout;
-    while (true) {
-        const unsigned v = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (__any(nb < 0 && v != 0)) return true;
-        if (__all(nb < 0 || (int)(v - target) >= 0)) return false;
-        if (__builtin_amdgcn_s_memrealtime() - t0 > tmo) {
-            __hip_atomic_store(&bar->err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return true;
-        }
-        __builtin_amdgcn_s_sleep(1);
-    }
-}
-
-// the same for all n tiles of a case, by all threads of the block (the
+// wait_neighbours (sor.h) for all n tiles of a case, by all threads of the block (the
 // answer is this wave's)
 __device__ __forceinline__ bool wait_all(const unsigned *flags, int n, unsigned target, GridBar *bar)
 {

@@ -85,3 +85,31 @@ def test_fields_round_trip(precision, nx, ny):
         for f in FIELDS:
             assert np.array_equal(c.get(f), want[f]), f
         assert np.all(c.get("iblank") == (c.get("flags").astype(np.uint8) & 1))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("nx,ny,check", [
+    (5, 4, 1),        # fewer cells than lanes
+    (128, 33, 2),     # 2 cells a lane; a chunk is one stage, split for its parity
+    (129, 60, 7),     # 3, and a last segment of one cell
+    (256, 24, 40),    # 4
+    (300, 41, 9),     # 5
+    (384, 100, 3),    # 6
+    (430, 9, 5),      # 7
+    (512, 50, 12),    # 8, the most
+    (520, 20, 6),     # 9: one launch per colour in both
+])
+def test_persistent_line_equals_launches(precision, nx, ny, check):
+    prec = {"fp64": iff.IF_FP64, "mixed": iff.IF_MIXED}[precision]
+    g = _cases(nx, ny, 0.2, nx == 256)
+    out = []
+    for persistent in (True, False):
+        with iff.Case(g["xf"], g["yf"], precision=prec, dt=0.002, re=100.0, bodies=g["bodies"], ppe_tol=1e-8,
+                      ppe_solver=iff.IF_PPE_LINE, ppe_omega=1.5, ppe_itermax=235, check_every=check) as c:
+            c.persistent(persistent)
+            st = [c.step(1) for _ in range(3)]
+            assert all(s["persistent_timeouts"] == 0 for s in st)
+            out.append(([s["ppe_sweeps"] for s in st], [s["ppe_res"] for s in st], {f: c.get(f) for f in FIELDS}))
+    assert out[0][:2] == out[1][:2]
+    for f in FIELDS:
+        assert np.array_equal(out[0][2][f], out[1][2][f]), f

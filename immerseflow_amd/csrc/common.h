@@ -46,7 +46,8 @@ enum : uint8_t {
 // element (i,j) is f[i + j*P].
 // ---------------------------------------------------------------------------
 constexpr int kPitchAlign = 64;
-constexpr int kTileX = 64;   // tile width (one wave64 row)
+constexpr int kTileX = 64;     // tile width (one wave64 row)
+constexpr int kTileRows = 16;  // tile height of the stencil passes
 
 inline int pitch_for(int nx) { return ((nx + kPitchAlign - 1) / kPitchAlign) * kPitchAlign; }
 template <typename T> constexpr int lead_elems() { return 256 / (int)sizeof(T) - 1; }

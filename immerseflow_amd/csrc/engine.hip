@@ -26,7 +26,7 @@
 namespace iff {
 
 constexpr int kSolveSweeps = 4096;  // sweeps of a persistent FP64 solve launch
-constexpr int kTileY = 16;  // base tiling (reductions, stencil passes)
+constexpr int kTileY = kTileRows;  // base tiling (reductions, stencil passes)
 
 // viscous iterations enqueued when the last step tells nothing, and at a time
 // when it told too few

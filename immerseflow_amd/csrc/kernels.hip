@@ -75,6 +75,21 @@ __device__ __forceinline__ bool tile_setup(const int2 *tiles, int ntiles,
     return true;
 }
 
+// The stencil passes: a wave takes kRowsT rows of its tile, one after the other
+// (fewer at the top of the grid), and loads all of them before it computes and
+// stores.  These passes do little arithmetic: on a small grid one lasts as long as
+// its chain of loads (row by row 7 to 12 us at 64^2), on a large one the
+// loads in flight set the bandwidth.  at(q): row q of the wave, within the array.
+constexpr int kRowsT = kTileRows / 4;
+struct RowLoads {
+    int j0, jmax;
+    __device__ RowLoads(const TileCtx &tc, int ny)
+        : j0(1 + tc.ty * kTileRows + kRowsT * __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)), jmax(ny - 1)
+    {
+    }
+    __device__ int at(int q) const { return min(j0 + q, jmax); }
+};
+
 // Velocity of the body owning the first solid side of a blanked face.
 __device__ __forceinline__ double blank_vel(const CaseDev &c, int ida, int idb,
                                             int comp)
@@ -109,17 +124,16 @@ __global__ void k_step_begin(const CaseDev *cs, int ncase)
 // P1: explicit convective source (ADSource, ADSolver.cu:46-79)
 // ---------------------------------------------------------------------------
 template <typename TS, typename AX>
-__device__ __forceinline__ TS conv_source(const TS *q, int id, int P, const AX &ax,
+__device__ __forceinline__ TS conv_source(TS qc, TS qE, TS qW, TS qN, TS qS, const AX &ax,
                                           const AX &ay, int i, int j, TS ufe,
                                           TS ufw, TS vfn, TS vfs)
 {
-    const TS dx_i = ax.d[i], dx_ip1 = ax.d[i + 1], dx_im1 = ax.d[i - 1];
-    const TS dy_j = ay.d[j], dy_jp1 = ay.d[j + 1], dy_jm1 = ay.d[j - 1];
-    const TS qc = q[id];
-    return (qc - ax.cs[i] * ((ax.ip[i] * (q[id + 1] * dx_i + qc * dx_ip1) * ufe)
-                             - (ax.im[i] * (qc * dx_im1 + q[id - 1] * dx_i) * ufw)))
-           - ay.cs[j] * ((ay.ip[j] * (q[id + P] * dy_j + qc * dy_jp1) * vfn)
-                         - (ay.im[j] * (qc * dy_jm1 + q[id - P] * dy_j) * vfs));
+    const TS dx_i = G(ax.d)[i], dx_ip1 = G(ax.d)[i + 1], dx_im1 = G(ax.d)[i - 1];
+    const TS dy_j = G(ay.d)[j], dy_jp1 = G(ay.d)[j + 1], dy_jm1 = G(ay.d)[j - 1];
+    return (qc - G(ax.cs)[i] * ((G(ax.ip)[i] * (qE * dx_i + qc * dx_ip1) * ufe)
+                                - (G(ax.im)[i] * (qc * dx_im1 + qW * dx_i) * ufw)))
+           - G(ay.cs)[j] * ((G(ay.ip)[j] * (qN * dy_j + qc * dy_jp1) * vfn)
+                            - (G(ay.im)[j] * (qc * dy_jm1 + qS * dy_j) * vfs));
 }
 
 template <typename TS>
@@ -133,23 +147,42 @@ __global__ __launch_bounds__(256) void k_source(const CaseDev *cs, const int2 *t
     const int i = 1 + tc.tx * kTileX + (threadIdx.x & 63);
     if (i > c.nx - 2) return;
     const int base = c.ctrl->ad_base;
-    const TS *u = fld<TS>(c.u[base]);
-    const TS *v = fld<TS>(c.v[base]);
-    TS *sx = fld<TS>(c.sx), *sy = fld<TS>(c.sy);
-    const double *uf = c.uf[0], *vf = c.vf[0];
-    const int P = c.P;
-    for (int r = threadIdx.x >> 6; r < c.tile_y; r += 4) {
-        const int j = 1 + tc.ty * c.tile_y + r;
-        if (j > c.ny - 2) break;
+    const auto u = G((const TS *)c.u[base]), v = G((const TS *)c.v[base]);
+    const auto sx = GW(fld<TS>(c.sx)), sy = GW(fld<TS>(c.sy));
+    const auto uf = G((const double *)c.uf[0]), vf = G((const double *)c.vf[0]);
+    const int P = c.P, ny = c.ny;
+    RowLoads rl(tc, ny);
+    TS uc[kRowsT + 2], vc[kRowsT + 2], uE[kRowsT], uW[kRowsT], vE[kRowsT], vW[kRowsT];
+    double fe[kRowsT], fw[kRowsT], fn[kRowsT + 1];
+#pragma unroll
+    for (int q = 0; q < kRowsT + 2; q++) {
+        const int id = i + rl.at(q - 1) * P;
+        uc[q] = u[id];
+        vc[q] = v[id];
+        if (q <= kRowsT) fn[q] = vf[id];
+    }
+#pragma unroll
+    for (int q = 0; q < kRowsT; q++) {
+        const int id = i + rl.at(q) * P;
+        uE[q] = u[id + 1];
+        uW[q] = u[id - 1];
+        vE[q] = v[id + 1];
+        vW[q] = v[id - 1];
+        fe[q] = uf[id];
+        fw[q] = uf[id - 1];
+    }
+#pragma unroll
+    for (int q = 0; q < kRowsT; q++) {
+        const int j = rl.j0 + q;
+        if (j > ny - 2) break;
         const int id = i + j * P;
-        const TS ufe = (TS)uf[id], ufw = (TS)uf[id - 1];
-        const TS vfn = (TS)vf[id], vfs = (TS)vf[id - P];
+        const TS ufe = (TS)fe[q], ufw = (TS)fw[q], vfn = (TS)fn[q + 1], vfs = (TS)fn[q];
         if constexpr (sizeof(TS) == 8) {
-            sx[id] = conv_source<TS>(u, id, P, c.x, c.y, i, j, ufe, ufw, vfn, vfs);
-            sy[id] = conv_source<TS>(v, id, P, c.x, c.y, i, j, ufe, ufw, vfn, vfs);
+            sx[id] = conv_source<TS>(uc[q + 1], uE[q], uW[q], uc[q + 2], uc[q], c.x, c.y, i, j, ufe, ufw, vfn, vfs);
+            sy[id] = conv_source<TS>(vc[q + 1], vE[q], vW[q], vc[q + 2], vc[q], c.x, c.y, i, j, ufe, ufw, vfn, vfs);
         } else {
-            sx[id] = conv_source<TS>(u, id, P, c.xf, c.yf, i, j, ufe, ufw, vfn, vfs);
-            sy[id] = conv_source<TS>(v, id, P, c.xf, c.yf, i, j, ufe, ufw, vfn, vfs);
+            sx[id] = conv_source<TS>(uc[q + 1], uE[q], uW[q], uc[q + 2], uc[q], c.xf, c.yf, i, j, ufe, ufw, vfn, vfs);
+            sy[id] = conv_source<TS>(vc[q + 1], vE[q], vW[q], vc[q + 2], vc[q], c.xf, c.yf, i, j, ufe, ufw, vfn, vfs);
         }
     }
 }
@@ -161,13 +194,13 @@ __global__ __launch_bounds__(256) void k_source(const CaseDev *cs, const int2 *t
 // rule of set_velocity_BC (:199-217) applied to the new iterate.
 // ---------------------------------------------------------------------------
 template <typename TS, typename AX>
-__device__ __forceinline__ TS jacobi_cell(const TS *q, const TS *s, int id, int P,
+__device__ __forceinline__ TS jacobi_cell(TS s, TS qE, TS qW, TS qN, TS qS,
                                           const AX &ax, const AX &ay, int i, int j,
                                           TS blank)
 {
-    const TS t = s[id] + ax.ap[i] * q[id + 1] + ax.am[i] * q[id - 1]
-                 + ay.ap[j] * q[id + P] + ay.am[j] * q[id - P];
-    return blank * t / (ax.ad[i] + ay.ad[j]);
+    const TS t = s + G(ax.ap)[i] * qE + G(ax.am)[i] * qW
+                 + G(ay.ap)[j] * qN + G(ay.am)[j] * qS;
+    return blank * t / (G(ax.ad)[i] + G(ay.ad)[j]);
 }
 
 template <typename TS>
@@ -180,36 +213,61 @@ __global__ __launch_bounds__(256) void k_ad_sweep(const CaseDev *cs, const int2 
     const Ctrl *ct = c.ctrl;
     if (!ct->active || ct->ad_done) return;
     const int base = ct->ad_base;
-    const TS *u = fld<TS>(c.u[base]), *v = fld<TS>(c.v[base]);
-    TS *un = fld<TS>(c.u[1 - base]), *vn = fld<TS>(c.v[1 - base]);
-    const TS *sx = fld<TS>(c.sx), *sy = fld<TS>(c.sy);
+    const auto u = G((const TS *)c.u[base]), v = G((const TS *)c.v[base]);
+    const auto un = GW(fld<TS>(c.u[1 - base])), vn = GW(fld<TS>(c.v[1 - base]));
+    const auto sx = G((const TS *)c.sx), sy = G((const TS *)c.sy);
+    const auto fl_ = G(c.flags);
     const int P = c.P, nx = c.nx, ny = c.ny;
     const TS ub2 = (TS)c.ubc * (TS)2.0, vb2 = (TS)c.vbc * (TS)2.0;
     const double w = c.ad_omega;
     const int i = 1 + tc.tx * kTileX + (threadIdx.x & 63);
     double acc = 0.0;
     if (i <= nx - 2) {
-        for (int r = threadIdx.x >> 6; r < c.tile_y; r += 4) {
-            const int j = 1 + tc.ty * c.tile_y + r;
+        // a wave's rows are four apart (the residual's sum keeps that order),
+        // all loaded first (RowLoads)
+        const int j0 = 1 + tc.ty * kTileRows + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+        TS uc[kRowsT], uE[kRowsT], uW[kRowsT], uN[kRowsT], uS[kRowsT], su[kRowsT];
+        TS vc[kRowsT], vE[kRowsT], vW[kRowsT], vN[kRowsT], vS[kRowsT], sv[kRowsT];
+        unsigned f[kRowsT];
+#pragma unroll
+        for (int q = 0; q < kRowsT; q++) {
+            const int id = i + min(j0 + 4 * q, ny - 2) * P;
+            f[q] = fl_[id];
+            uc[q] = u[id];
+            uE[q] = u[id + 1];
+            uW[q] = u[id - 1];
+            uN[q] = u[id + P];
+            uS[q] = u[id - P];
+            su[q] = sx[id];
+            vc[q] = v[id];
+            vE[q] = v[id + 1];
+            vW[q] = v[id - 1];
+            vN[q] = v[id + P];
+            vS[q] = v[id - P];
+            sv[q] = sy[id];
+        }
+#pragma unroll
+        for (int q = 0; q < kRowsT; q++) {
+            const int j = j0 + 4 * q;
             if (j > ny - 2) break;
             const int id = i + j * P;
-            const bool fl = c.flags[id] & F_FLUID;
+            const bool fl = f[q] & F_FLUID;
             const TS blank = fl ? (TS)1.0 : (TS)0.0;
             TS qu, qv;
             if constexpr (sizeof(TS) == 8) {
-                qu = jacobi_cell<TS>(u, sx, id, P, c.x, c.y, i, j, blank);
-                qv = jacobi_cell<TS>(v, sy, id, P, c.x, c.y, i, j, blank);
+                qu = jacobi_cell<TS>(su[q], uE[q], uW[q], uN[q], uS[q], c.x, c.y, i, j, blank);
+                qv = jacobi_cell<TS>(sv[q], vE[q], vW[q], vN[q], vS[q], c.x, c.y, i, j, blank);
             } else {
-                qu = jacobi_cell<TS>(u, sx, id, P, c.xf, c.yf, i, j, blank);
-                qv = jacobi_cell<TS>(v, sy, id, P, c.xf, c.yf, i, j, blank);
+                qu = jacobi_cell<TS>(su[q], uE[q], uW[q], uN[q], uS[q], c.xf, c.yf, i, j, blank);
+                qv = jacobi_cell<TS>(sv[q], vE[q], vW[q], vN[q], vS[q], c.xf, c.yf, i, j, blank);
             }
             if (w != 1.0) {  // w_AD relaxation (ADSolver.cu:95,116)
-                qu = (TS)(1.0 - w) * u[id] + (TS)w * qu;
-                qv = (TS)(1.0 - w) * v[id] + (TS)w * qv;
+                qu = (TS)(1.0 - w) * uc[q] + (TS)w * qu;
+                qv = (TS)(1.0 - w) * vc[q] + (TS)w * qv;
             }
             un[id] = qu;
             vn[id] = qv;
-            if (fl) acc += (double)fabs(qu - u[id]) + (double)fabs(qv - v[id]);
+            if (fl) acc += (double)fabs(qu - uc[q]) + (double)fabs(qv - vc[q]);
             if (i == 1) { un[id - 1] = -qu + ub2; vn[id - 1] = -qv + vb2; }
             if (i == nx - 2) { un[id + 1] = -qu + ub2; vn[id + 1] = -qv + vb2; }
             if (j == 1) { un[id - P] = -qu + ub2; vn[id - P] = -qv + vb2; }
@@ -351,40 +409,55 @@ __global__ __launch_bounds__(256) void k_faces_rhs(const CaseDev *cs, const int2
     const int nx = c.nx, ny = c.ny, P = c.P;
     if (i > nx - 2) return;
     const int base = c.ctrl->ad_base;
-    const TS *u = fld<TS>(c.u[base]), *v = fld<TS>(c.v[base]);
-    double *uf = c.uf[out_buf], *vf = c.vf[out_buf];
+    const auto u = G((const TS *)c.u[base]), v = G((const TS *)c.v[base]);
+    const auto uf = GW(c.uf[out_buf]), vf = GW(c.vf[out_buf]);
+    const auto rhs = GW(c.rhs);
     const AxisD &ax = c.x, &ay = c.y;
-    const double dxi = ax.d[i], dxp = ax.d[i + 1], dxm = ax.d[i - 1];
     const bool keep = with_rhs && c.ppe_solver == IF_PPE_RBSOR && !c.e[0];
-    const double *pb = c.p[c.ctrl->ppe_base];
-    double *pn = c.p[1 - c.ctrl->ppe_base];
-    for (int r = threadIdx.x >> 6; r < c.tile_y; r += 4) {
-        const int j = 1 + tc.ty * c.tile_y + r;
+    const auto pb = G((const double *)c.p[c.ctrl->ppe_base]);
+    const auto pn = GW(c.p[1 - c.ctrl->ppe_base]);
+    RowLoads rl(tc, ny);
+    unsigned fl[kRowsT];
+    TS uC[kRowsT], uE[kRowsT], uW[kRowsT], vC[kRowsT + 2];
+#pragma unroll
+    for (int q = 0; q < kRowsT + 2; q++) vC[q] = v[i + rl.at(q - 1) * P];
+#pragma unroll
+    for (int q = 0; q < kRowsT; q++) {
+        const int id = i + rl.at(q) * P;
+        fl[q] = G(c.flags)[id];
+        uC[q] = u[id];
+        uE[q] = u[id + 1];
+        uW[q] = u[id - 1];
+    }
+    const double dxi = G(ax.d)[i], dxp = G(ax.d)[i + 1], dxm = G(ax.d)[i - 1];
+    const double ipi = G(ax.ip)[i], ipw = G(ax.ip)[i - 1], rdx = G(ax.rd)[i];
+#pragma unroll
+    for (int q = 0; q < kRowsT; q++) {
+        const int j = rl.j0 + q;
         if (j > ny - 2) break;
         const int id = i + j * P;
-        const uint8_t f = c.flags[id];
-        const double uc = (double)u[id], vc = (double)v[id];
+        const unsigned f = fl[q];
+        const double uc = (double)uC[q], vc = (double)vC[q + 1];
         double ufe, ufw, vfn, vfs;
         if (i == nx - 2) ufe = c.ubc;
-        else if (f & F_OPEN_E) ufe = ax.ip[i] * ((double)u[id + 1] * dxi + uc * dxp);
+        else if (f & F_OPEN_E) ufe = ipi * ((double)uE[q] * dxi + uc * dxp);
         else ufe = blank_vel(c, id, id + 1, 0);
         if (i == 1) ufw = c.ubc;
-        else if (f & F_OPEN_W) ufw = ax.ip[i - 1] * (uc * dxm + (double)u[id - 1] * dxi);
+        else if (f & F_OPEN_W) ufw = ipw * (uc * dxm + (double)uW[q] * dxi);
         else ufw = blank_vel(c, id - 1, id, 0);
-        const double dyj = ay.d[j], dyp = ay.d[j + 1], dym = ay.d[j - 1];
+        const double dyj = G(ay.d)[j], dyp = G(ay.d)[j + 1], dym = G(ay.d)[j - 1];
         if (j == ny - 2) vfn = c.vbc;
-        else if (f & F_OPEN_N) vfn = ay.ip[j] * ((double)v[id + P] * dyj + vc * dyp);
+        else if (f & F_OPEN_N) vfn = G(ay.ip)[j] * ((double)vC[q + 2] * dyj + vc * dyp);
         else vfn = blank_vel(c, id, id + P, 1);
         if (j == 1) vfs = c.vbc;
-        else if (f & F_OPEN_S) vfs = ay.ip[j - 1] * (vc * dym + (double)v[id - P] * dyj);
+        else if (f & F_OPEN_S) vfs = G(ay.ip)[j - 1] * (vc * dym + (double)vC[q] * dyj);
         else vfs = blank_vel(c, id - P, id, 1);
         uf[id] = ufe;
         vf[id] = vfn;
         if (i == 1) uf[id - 1] = ufw;
         if (j == 1) vf[id - P] = vfs;
         if (with_rhs)
-            c.rhs[id] = (f & F_FLUID) ? ((ufe - ufw) * ax.rd[i] + (vfn - vfs) * ay.rd[j]) * c.rdt
-                                      : 0.0;
+            rhs[id] = (f & F_FLUID) ? ((ufe - ufw) * rdx + (vfn - vfs) * G(ay.rd)[j]) * c.rdt : 0.0;
         // FP64 red-black solves: the register-tile sweeps do not write the
         // cells they keep (not fluid, or without an open face), so both
         // pressure buffers hold their values from here on
@@ -1158,26 +1231,39 @@ __global__ __launch_bounds__(256) void k_ppe_resid(const CaseDev *cs, const int2
     int kexec = c.ppe_itermax - ct->ppe_sweeps;
     if (kexec > K) kexec = K;
     const int nl = (kexec + c.ppe_m - 1) / c.ppe_m;  // launches of the chunk
-    const double *p = c.p[(ct->ppe_base + nl) & 1];
+    const auto p = G((const double *)c.p[(ct->ppe_base + nl) & 1]);
     const int nx = c.nx, ny = c.ny, P = c.P;
     const int i = 1 + tc.tx * kTileX + (threadIdx.x & 63);
     double m = 0.0;
     if (i <= nx - 2) {
-        const double cpx = c.x.cp[i], cmx = c.x.cm[i];
-        for (int r = threadIdx.x >> 6; r < c.tile_y; r += 4) {
-            const int j = 1 + tc.ty * c.tile_y + r;
+        RowLoads rl(tc, ny);
+        const double cpx = G(c.x.cp)[i], cmx = G(c.x.cm)[i];
+        unsigned fl[kRowsT];
+        double pC[kRowsT + 2], pE[kRowsT], pW[kRowsT], rh[kRowsT];
+#pragma unroll
+        for (int q = 0; q < kRowsT + 2; q++) pC[q] = p[i + rl.at(q - 1) * P];
+#pragma unroll
+        for (int q = 0; q < kRowsT; q++) {
+            const int id = i + rl.at(q) * P;
+            fl[q] = G(c.flags)[id];
+            rh[q] = G(c.rhs)[id];
+            pE[q] = p[id + 1];
+            pW[q] = p[id - 1];
+        }
+#pragma unroll
+        for (int q = 0; q < kRowsT; q++) {
+            const int j = rl.j0 + q;
             if (j > ny - 2) break;
-            const int id = i + j * P;
-            const uint8_t f = c.flags[id];
+            const unsigned f = fl[q];
             if (!(f & F_FLUID)) continue;
             const double aE = (f & F_OPEN_E) ? cpx : 0.0;
             const double aW = (f & F_OPEN_W) ? cmx : 0.0;
-            const double aN = (f & F_OPEN_N) ? c.y.cp[j] : 0.0;
-            const double aS = (f & F_OPEN_S) ? c.y.cm[j] : 0.0;
+            const double aN = (f & F_OPEN_N) ? G(c.y.cp)[j] : 0.0;
+            const double aS = (f & F_OPEN_S) ? G(c.y.cm)[j] : 0.0;
             const double ap = -((aE + aW) + (aN + aS));
             if (ap == 0.0) continue;
-            const double sum = (aE * p[id + 1] + aW * p[id - 1]) + (aN * p[id + P] + aS * p[id - P]);
-            const double rr = c.rhs[id] - (ap * p[id] + sum);
+            const double sum = (aE * pE[q] + aW * pW[q]) + (aN * pC[q + 2] + aS * pC[q]);
+            const double rr = rh[q] - (ap * pC[q + 1] + sum);
             m = fmax(m, absinf(rr));
         }
     }
@@ -1200,43 +1286,69 @@ __global__ __launch_bounds__(256) void k_ppe_update_resid(const CaseDev *cs, con
     if (kexec > K) kexec = K;
     const int nl = (kexec + c.ppe_m - 1) / c.ppe_m;  // launches of the chunk
     const bool upd = kexec > 0;
-    const double *p = c.p[ct->ppe_base];
-    double *pn = c.p[1 - ct->ppe_base];
-    const float *e = c.e[nl & 1];
+    const auto p = G((const double *)c.p[ct->ppe_base]);
+    const auto pn = GW(c.p[1 - ct->ppe_base]);
+    const auto e = G((const float *)c.e[nl & 1]);
+    const auto r32_ = GW(c.r32);
     const int nx = c.nx, ny = c.ny, P = c.P;
     const int i = 1 + tc.tx * kTileX + (threadIdx.x & 63);
     double m = 0.0;
     if (i <= nx - 2) {
-        const double cpx = c.x.cp[i], cmx = c.x.cm[i];
-        for (int r = threadIdx.x >> 6; r < c.tile_y; r += 4) {
-            const int j = 1 + tc.ty * c.tile_y + r;
-            if (j > ny - 2) break;
-            const int id = i + j * P;
-            const uint8_t f = c.flags[id];
-            double pc = p[id], pE = p[id + 1], pW = p[id - 1], pN = p[id + P], pS = p[id - P];
-            if (upd) {
-                pc += (double)e[id];
-                pE += (double)e[id + 1];
-                pW += (double)e[id - 1];
-                pN += (double)e[id + P];
-                pS += (double)e[id - P];
-                pn[id] = pc;
+        RowLoads rl(tc, ny);
+        const double cpx = G(c.x.cp)[i], cmx = G(c.x.cm)[i];
+        const bool uni = c.uni;
+        const float uinv = c.uinv;
+        unsigned fl[kRowsT];
+        double pC[kRowsT + 2], pE[kRowsT], pW[kRowsT], rh[kRowsT];
+#pragma unroll
+        for (int q = 0; q < kRowsT + 2; q++) pC[q] = p[i + rl.at(q - 1) * P];
+#pragma unroll
+        for (int q = 0; q < kRowsT; q++) {
+            const int id = i + rl.at(q) * P;
+            fl[q] = G(c.flags)[id];
+            rh[q] = G(c.rhs)[id];
+            pE[q] = p[id + 1];
+            pW[q] = p[id - 1];
+        }
+        if (upd) {
+            float eC[kRowsT + 2], eE[kRowsT], eW[kRowsT];
+#pragma unroll
+            for (int q = 0; q < kRowsT + 2; q++) eC[q] = e[i + rl.at(q - 1) * P];
+#pragma unroll
+            for (int q = 0; q < kRowsT; q++) {
+                const int id = i + rl.at(q) * P;
+                eE[q] = e[id + 1];
+                eW[q] = e[id - 1];
             }
+#pragma unroll
+            for (int q = 0; q < kRowsT + 2; q++) pC[q] += (double)eC[q];
+#pragma unroll
+            for (int q = 0; q < kRowsT; q++) {
+                pE[q] += (double)eE[q];
+                pW[q] += (double)eW[q];
+                if (rl.j0 + q <= ny - 2) pn[i + (rl.j0 + q) * P] = pC[q + 1];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kRowsT; q++) {
+            const int j = rl.j0 + q;
+            if (j > ny - 2) break;
+            const unsigned f = fl[q];
             float r32 = 0.0f;
             if (f & F_FLUID) {
                 const double aE = (f & F_OPEN_E) ? cpx : 0.0;
                 const double aW = (f & F_OPEN_W) ? cmx : 0.0;
-                const double aN = (f & F_OPEN_N) ? c.y.cp[j] : 0.0;
-                const double aS = (f & F_OPEN_S) ? c.y.cm[j] : 0.0;
+                const double aN = (f & F_OPEN_N) ? G(c.y.cp)[j] : 0.0;
+                const double aS = (f & F_OPEN_S) ? G(c.y.cm)[j] : 0.0;
                 const double ap = -((aE + aW) + (aN + aS));
                 if (ap != 0.0) {
-                    const double sum = (aE * pE + aW * pW) + (aN * pN + aS * pS);
-                    const double rr = c.rhs[id] - (ap * pc + sum);
-                    r32 = c.uni ? (float)rr * c.uinv : (float)rr;
+                    const double sum = (aE * pE[q] + aW * pW[q]) + (aN * pC[q + 2] + aS * pC[q]);
+                    const double rr = rh[q] - (ap * pC[q + 1] + sum);
+                    r32 = uni ? (float)rr * uinv : (float)rr;
                     m = fmax(m, absinf(rr));
                 }
             }
-            c.r32[id] = r32;
+            r32_[i + j * P] = r32;
         }
     }
     check_end(cs, tc, ncase, K, true, block_max(m), bar);
@@ -1354,49 +1466,72 @@ __global__ __launch_bounds__(256) void k_project(const CaseDev *cs, const int2 *
     if (!ct->active) return;
     const int nx = c.nx, ny = c.ny, P = c.P;
     const int i = 1 + tc.tx * kTileX + (threadIdx.x & 63);
-    const double *p = c.p[ct->ppe_base];
-    const double *ufs = c.uf[1], *vfs_ = c.vf[1];
-    double *ufn = c.uf[0], *vfn_ = c.vf[0];
-    TS *u = fld<TS>(c.u[ct->ad_base]), *v = fld<TS>(c.v[ct->ad_base]);
+    const auto p = G((const double *)c.p[ct->ppe_base]);
+    const auto ufs = G((const double *)c.uf[1]), vfs_ = G((const double *)c.vf[1]);
+    const auto ufn = GW(c.uf[0]), vfn_ = GW(c.vf[0]);
+    const auto u = GW(fld<TS>(c.u[ct->ad_base])), v = GW(fld<TS>(c.v[ct->ad_base]));
     const double dt = c.dt;
     const TS ub2 = (TS)c.ubc * (TS)2.0, vb2 = (TS)c.vbc * (TS)2.0;
     const AxisD &ax = c.x, &ay = c.y;
     double m = 0.0;
     if (i <= nx - 2) {
-        const double dxi = ax.d[i], dxp = ax.d[i + 1], dxm = ax.d[i - 1];
-        for (int r = threadIdx.x >> 6; r < c.tile_y; r += 4) {
-            const int j = 1 + tc.ty * c.tile_y + r;
+        RowLoads rl(tc, ny);
+        unsigned fl[kRowsT];
+        double pC[kRowsT + 2], pE_[kRowsT], pW_[kRowsT], fe[kRowsT], fw[kRowsT], fn[kRowsT + 1];
+        TS u0[kRowsT], v0[kRowsT];
+#pragma unroll
+        for (int q = 0; q < kRowsT + 2; q++) {
+            const int id = i + rl.at(q - 1) * P;
+            pC[q] = p[id];
+            if (q <= kRowsT) fn[q] = vfs_[id];
+        }
+#pragma unroll
+        for (int q = 0; q < kRowsT; q++) {
+            const int id = i + rl.at(q) * P;
+            fl[q] = G(c.flags)[id];
+            pE_[q] = p[id + 1];
+            pW_[q] = p[id - 1];
+            fe[q] = ufs[id];
+            fw[q] = ufs[id - 1];
+            u0[q] = u[id];
+            v0[q] = v[id];
+        }
+        const double dxi = G(ax.d)[i], dxp = G(ax.d)[i + 1], dxm = G(ax.d)[i - 1];
+        const double gi = G(ax.g)[i], gw = G(ax.g)[i - 1], ipi = G(ax.ip)[i], imi = G(ax.im)[i], rdx = G(ax.rd)[i];
+#pragma unroll
+        for (int q = 0; q < kRowsT; q++) {
+            const int j = rl.j0 + q;
             if (j > ny - 2) break;
             const int id = i + j * P;
-            const uint8_t f = c.flags[id];
-            const double pc = p[id], pE = p[id + 1], pW = p[id - 1], pN = p[id + P], pS = p[id - P];
+            const unsigned f = fl[q];
+            const double pc = pC[q + 1], pE = pE_[q], pW = pW_[q], pN = pC[q + 2], pS = pC[q];
             // faces owned by this cell (east, north) and its west/south
             // neighbours' (recomputed for the divergence, same expression)
-            double ue = ufs[id], uw = ufs[id - 1], vn = vfs_[id], vs = vfs_[id - P];
-            if (f & F_OPEN_E) ue = ue - dt * ((pE - pc) * ax.g[i]);
-            if (f & F_OPEN_W) uw = uw - dt * ((pc - pW) * ax.g[i - 1]);
-            if (f & F_OPEN_N) vn = vn - dt * ((pN - pc) * ay.g[j]);
-            if (f & F_OPEN_S) vs = vs - dt * ((pc - pS) * ay.g[j - 1]);
+            double ue = fe[q], uw = fw[q], vn = fn[q + 1], vs = fn[q];
+            if (f & F_OPEN_E) ue = ue - dt * ((pE - pc) * gi);
+            if (f & F_OPEN_W) uw = uw - dt * ((pc - pW) * gw);
+            if (f & F_OPEN_N) vn = vn - dt * ((pN - pc) * G(ay.g)[j]);
+            if (f & F_OPEN_S) vs = vs - dt * ((pc - pS) * G(ay.g)[j - 1]);
             ufn[id] = ue;
             vfn_[id] = vn;
             if (i == 1) ufn[id - 1] = uw;
             if (j == 1) vfn_[id - P] = vs;
             // cell velocities
-            const double dyj = ay.d[j], dyp = ay.d[j + 1], dym = ay.d[j - 1];
-            const double pe = ax.ip[i] * (pE * dxi + pc * dxp);
-            const double pw = ax.im[i] * (pc * dxm + pW * dxi);
-            const double pn = ay.ip[j] * (pN * dyj + pc * dyp);
-            const double ps = ay.im[j] * (pc * dym + pS * dyj);
+            const double dyj = G(ay.d)[j], dyp = G(ay.d)[j + 1], dym = G(ay.d)[j - 1];
+            const double pe = ipi * (pE * dxi + pc * dxp);
+            const double pw = imi * (pc * dxm + pW * dxi);
+            const double pn = G(ay.ip)[j] * (pN * dyj + pc * dyp);
+            const double ps = G(ay.im)[j] * (pc * dym + pS * dyj);
             const double blank = (f & F_FLUID) ? 1.0 : 0.0;
-            const TS qu = (TS)(blank * ((double)u[id] - dt * ((pe - pw) * ax.rd[i])));
-            const TS qv = (TS)(blank * ((double)v[id] - dt * ((pn - ps) * ay.rd[j])));
+            const TS qu = (TS)(blank * ((double)u0[q] - dt * ((pe - pw) * rdx)));
+            const TS qv = (TS)(blank * ((double)v0[q] - dt * ((pn - ps) * G(ay.rd)[j])));
             u[id] = qu;
             v[id] = qv;
             if (i == 1) { u[id - 1] = -qu + ub2; v[id - 1] = -qv + vb2; }
             if (i == nx - 2) { u[id + 1] = -qu + ub2; v[id + 1] = -qv + vb2; }
             if (j == 1) { u[id - P] = -qu + ub2; v[id - P] = -qv + vb2; }
             if (j == ny - 2) { u[id + P] = -qu + ub2; v[id + P] = -qv + vb2; }
-            if (f & F_FLUID) m = fmax(m, absinf((ue - uw) * ax.rd[i] + (vn - vs) * ay.rd[j]));
+            if (f & F_FLUID) m = fmax(m, absinf((ue - uw) * rdx + (vn - vs) * G(ay.rd)[j]));
         }
     }
     m = block_max(m);

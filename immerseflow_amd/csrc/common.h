@@ -104,7 +104,8 @@ struct Ctrl {
     int failed;        // non-finite residual seen
     int steps_done, steps_target;
     int ad_done, ad_iter, ad_base;   // u,v live in buffer ad_base
-    int ppe_done, ppe_sweeps, ppe_base;
+    int ppe_done, ppe_sweeps, ppe_base;  // ppe_done: 1 by the rule, 2 by a timed-out wait
+    int closed;        // this step's projection is done
     int ng;            // live ghost-cell count (rebuilt on the device for moving bodies)
     int ng_total;      // ghost cells found by the last build (may exceed capacity)
     unsigned ticket;   // tiles (or groups of them) through the running convergence check

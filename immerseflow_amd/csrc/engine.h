@@ -123,6 +123,7 @@ private:
     // checks enqueued so far
     unsigned long long *h_prog_ = nullptr;
     unsigned long long checks_ = 0;
+    int chunk_pred_ = 0;               // chunks of the last step's longest solve
     int ad_pred_ = 0;                  // viscous iterations to enqueue: the last step's and one (0: unknown)
     bool operator_ready_ = false;      // weights and line factors of the resident set are formed
     // device time stamps of the timed Poisson chunks: [0] count, then a

@@ -988,8 +988,21 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         // running one; the chunks behind the last case's end do nothing.
         const int nchunks = (max_ppe_ + K - 1) / K;
         unsigned long long word = 0;
+        // The step's end, per case and once (step_tail); where no monitor
+        // samples it, enqueued behind the chunk that ended the last step's
+        // solve too, before its check is known: the device goes on without
+        // the host (64^2: 20 us to wake up, 5 launches, an empty chunk).
+        bool tail_in = false;  // enqueued behind the last check
+        auto tail = [&]() {
+            launch_pressure_bc(st_, d_cases_, n, max_ring_, max_ng_);
+            launch_project(st_, vprec_, d_cases_, d_tiles_base_, nt_base_);
+            launch_ghost_vel(st_, vprec_, d_cases_, n, max_ng_, true);
+            if (any_monitor_) launch_monitor(st_, vprec_, d_cases_, n, d_tiles_base_, nt_base_);
+            launch_step_end(st_, d_cases_, n);
+        };
         auto poisson = [&](bool entry_check) -> if_status {
             const unsigned long long base = checks_;
+            tail_in = false;
             if (entry_check) check(0);
             if (pers && solve) {
                 for (int u = 0; u < nchunks; u += nsolve) {
@@ -997,9 +1010,13 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
                                           d_tiles_sweep_, nt_sweep_, K,
                                           PersArgs{d_bar_, d_flags_, d_vals_, nsolve, n}, wmode_);
                     checks_++;
+                    if (!any_monitor_) tail();
                     if_status r = wait_checks(base, 0, &word);
                     if (r != IF_OK) return r;
-                    if (word & kProgDone) return IF_OK;
+                    if (word & kProgDone) {
+                        tail_in = !any_monitor_;
+                        return IF_OK;
+                    }
                 }
                 return IF_OK;
             }
@@ -1012,9 +1029,14 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
                     enqueue_sweeps(K, M, any_rb, any_jac, any_line, pers, lpers, timing);
                 }
                 check(K);
-                if_status r = wait_checks(base, spec_depth - 1, &word);
+                const bool expect = u + 1 == chunk_pred_ && !any_monitor_;
+                if (expect) tail();
+                if_status r = wait_checks(base, expect ? 0 : spec_depth - 1, &word);
                 if (r != IF_OK) return r;
-                if ((word >> 3) > base && (word & kProgDone)) return IF_OK;
+                if ((word >> 3) > base && (word & kProgDone)) {
+                    tail_in = expect;
+                    return IF_OK;
+                }
             }
             return wait_checks(base, 0, &word);
         };
@@ -1076,11 +1098,7 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         } while ((word & kProgAdOpen) && ad_enq < max_ad_);
 
         // ---- pressure BC, projection, divergence, ghost cells
-        launch_pressure_bc(st_, d_cases_, n, max_ring_, max_ng_);
-        launch_project(st_, vprec_, d_cases_, d_tiles_base_, nt_base_);
-        launch_ghost_vel(st_, vprec_, d_cases_, n, max_ng_);
-        if (any_monitor_) launch_monitor(st_, vprec_, d_cases_, n, d_tiles_base_, nt_base_);
-        launch_step_end(st_, d_cases_, n);
+        if (!tail_in) tail();
         for (int id : order_) slots_[id]->steps_host++;
 
         if (timing)  // completes with the synchronisation below
@@ -1090,7 +1108,12 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         rc = read_ctrl_sync(all);
         if (rc != IF_OK) return rc;
         ad_pred_ = 0;
-        for (int id : order_) ad_pred_ = std::max(ad_pred_, all[id].ad_iter + 1);
+        int most = 0;
+        for (int id : order_) {
+            ad_pred_ = std::max(ad_pred_, all[id].ad_iter + 1);
+            most = std::max(most, all[id].ppe_sweeps);
+        }
+        chunk_pred_ = (most + K - 1) / K;
         const int timed = timing ? (int)std::min<unsigned long long>(h_stamps_[0], kStamps) / 2 : 0;
         if (timed > 0) {
             int maxsw = 0;

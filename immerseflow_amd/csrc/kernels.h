@@ -10,7 +10,7 @@ void launch_step_begin(hipStream_t st, const CaseDev *cs, int ncase);
 void launch_source(hipStream_t st, int prec, const CaseDev *cs, const int2 *tiles, int nt);
 void launch_ad_sweep(hipStream_t st, int prec, const CaseDev *cs, const int2 *tiles, int nt);
 void launch_ad_finish(hipStream_t st, int prec, const CaseDev *cs, int ncase);
-void launch_ghost_vel(hipStream_t st, int prec, const CaseDev *cs, int ncase, int max_ng);
+void launch_ghost_vel(hipStream_t st, int prec, const CaseDev *cs, int ncase, int max_ng, bool tail = false);
 void launch_pressure_bc(hipStream_t st, const CaseDev *cs, int ncase, int max_ring, int max_ng);
 bool sweep_variant_ok(int ty, int m);
 void launch_ppe_sweep(hipStream_t st, int prec, int solver, int ty, int m, const CaseDev *cs,

@@ -90,6 +90,14 @@ struct RowLoads {
     __device__ int at(int q) const { return min(j0 + q, jmax); }
 };
 
+// The step's end (pressure boundary, projection, bookkeeping) of a case whose
+// loops have ended, once.  The host enqueues it behind the chunk that it expects
+// to be the last one, without waiting for that chunk's check.
+__device__ __forceinline__ bool step_tail(const Ctrl *ct)
+{
+    return ct->active && ct->ad_done && ct->ppe_done == 1 && !ct->closed;
+}
+
 // Velocity of the body owning the first solid side of a blanked face.
 __device__ __forceinline__ double blank_vel(const CaseDev &c, int ida, int idb,
                                             int comp)
@@ -116,6 +124,7 @@ __global__ void k_step_begin(const CaseDev *cs, int ncase)
     // enqueued behind too few viscous iterations do nothing, and the host
     // enqueues them again
     c->ppe_done = c->ad_done ? 0 : 1;
+    c->closed = 0;
     c->ppe_sweeps = 0;
     c->ppe_res = 0.0;
 }
@@ -298,12 +307,12 @@ __device__ __forceinline__ void ghost_vel(const CaseDev &c, TS *u, TS *v, int g)
 }
 
 template <typename TS>
-__global__ __launch_bounds__(256) void k_ghost_vel(const CaseDev *cs)
+__global__ __launch_bounds__(256) void k_ghost_vel(const CaseDev *cs, bool tail)
 {
     const CaseDev &c = cs[blockIdx.y];
     const Ctrl *ct = c.ctrl;
     const int g = blockIdx.x * 256 + threadIdx.x;
-    if (g >= ct->ng || !ct->active) return;
+    if (g >= ct->ng || !(tail ? step_tail(ct) : ct->active)) return;
     ghost_vel(c, fld<TS>(c.u[ct->ad_base]), fld<TS>(c.v[ct->ad_base]), g);
 }
 
@@ -360,7 +369,7 @@ __global__ __launch_bounds__(kAdFinish) void k_ad_finish(const CaseDev *cs, int 
 __global__ __launch_bounds__(256) void k_p_ring(const CaseDev *cs)
 {
     const CaseDev &c = cs[blockIdx.y];
-    if (!c.ctrl->active) return;
+    if (!step_tail(c.ctrl)) return;
     double *p = c.p[c.ctrl->ppe_base];
     const int k = blockIdx.x * 256 + threadIdx.x;
     const int P = c.P, nx = c.nx, ny = c.ny;
@@ -380,7 +389,7 @@ __global__ __launch_bounds__(256) void k_ghost_p(const CaseDev *cs)
 {
     const CaseDev &c = cs[blockIdx.y];
     const int g = blockIdx.x * 256 + threadIdx.x;
-    if (g >= c.ctrl->ng || !c.ctrl->active) return;
+    if (g >= c.ctrl->ng || !step_tail(c.ctrl)) return;
     double *p = c.p[c.ctrl->ppe_base];
     const GhostDev &o = c.gh[g];
     const BodyDev &b = c.bodies[o.body];
@@ -1213,8 +1222,12 @@ __device__ __forceinline__ void check_end(const CaseDev *cs, const TileCtx &tc, 
     ct->ppe_res = res;
     if (!(res <= 1.0e300)) ct->failed = 1;
     bool done = !(res > c.ppe_tol) || ct->ppe_sweeps >= c.ppe_itermax || ct->failed;
-    if (__hip_atomic_load(&bar->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) done = true;
-    if (done) ct->ppe_done = 1;
+    if (done) {
+        ct->ppe_done = 1;
+    } else if (__hip_atomic_load(&bar->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+        ct->ppe_done = 2;
+        done = true;
+    }
     check_case(ncase, !done, false, bar);
 }
 
@@ -1362,7 +1375,7 @@ __global__ void k_ppe_rearm(const CaseDev *cs, int ncase)
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= ncase) return;
     Ctrl *c = cs[k].ctrl;
-    if (!c->active || c->failed) return;
+    if (!c->active || c->failed || c->closed) return;
     c->ppe_done = 0;
     c->ppe_sweeps = 0;
 }
@@ -1463,7 +1476,7 @@ __global__ __launch_bounds__(256) void k_project(const CaseDev *cs, const int2 *
     if (!tile_setup(tiles, ntiles, ntiles_pad, cs, tc)) return;
     const CaseDev &c = cs[tc.cid];
     const Ctrl *ct = c.ctrl;
-    if (!ct->active) return;
+    if (!step_tail(ct)) return;
     const int nx = c.nx, ny = c.ny, P = c.P;
     const int i = 1 + tc.tx * kTileX + (threadIdx.x & 63);
     const auto p = G((const double *)c.p[ct->ppe_base]);
@@ -1542,12 +1555,13 @@ __global__ __launch_bounds__(256) void k_step_end(const CaseDev *cs, int ncase)
 {
     const CaseDev &c = cs[blockIdx.x];
     Ctrl *ct = c.ctrl;
-    if (!ct->active) return;
+    if (!step_tail(ct)) return;
     const int nt = c.ntx * c.nty;
     double m = 0.0;
     for (int k = threadIdx.x; k < nt; k += 256) m = fmax(m, c.part[k]);
     m = block_max(m);
     if (threadIdx.x == 0) {
+        ct->closed = 1;
         ct->div_max = m;
         if (m > ct->max_div || !(m <= 1.0e300)) ct->max_div = m;
         if (!(m <= 1.0e300)) ct->failed = 1;
@@ -1590,12 +1604,12 @@ void launch_ad_finish(hipStream_t st, int prec, const CaseDev *cs, int ncase)
     else hipLaunchKernelGGL(k_ad_finish<float>, dim3(ncase), dim3(kAdFinish), 0, st, cs, ncase);
 }
 
-void launch_ghost_vel(hipStream_t st, int prec, const CaseDev *cs, int ncase, int max_ng)
+void launch_ghost_vel(hipStream_t st, int prec, const CaseDev *cs, int ncase, int max_ng, bool tail)
 {
     if (max_ng <= 0) return;
     dim3 g((max_ng + 255) / 256, ncase);
-    if (prec == IF_FP64) hipLaunchKernelGGL(k_ghost_vel<double>, g, dim3(256), 0, st, cs);
-    else hipLaunchKernelGGL(k_ghost_vel<float>, g, dim3(256), 0, st, cs);
+    if (prec == IF_FP64) hipLaunchKernelGGL(k_ghost_vel<double>, g, dim3(256), 0, st, cs, tail);
+    else hipLaunchKernelGGL(k_ghost_vel<float>, g, dim3(256), 0, st, cs, tail);
 }
 
 void launch_pressure_bc(hipStream_t st, const CaseDev *cs, int ncase, int max_ring, int max_ng)
@@ -1918,7 +1932,7 @@ __global__ void k_tune_arm(const CaseDev *cs, int ncase, const Ctrl *ctrl0, cons
     if (k >= ncase) return;
     Ctrl *c = cs[k].ctrl;
     *c = saved[c - ctrl0];
-    if (!c->active || c->failed) return;
+    if (!c->active || c->failed || c->closed) return;
     c->ppe_done = 0;
     c->ppe_sweeps = 0;
 }

@@ -794,7 +794,7 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
                     // here: this one leaves its part of the result too)
                     whole = check;
                     if (solve && tl.y == 0 && threadIdx.x == 0) {
-                        ctw->ppe_done = 1;
+                        ctw->ppe_done = 2;
                         check_case(pa.ncase, false, false, bar);
                     }
                     break;

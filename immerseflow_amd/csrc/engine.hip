@@ -744,6 +744,31 @@ if_status Engine::check_barrier()
                             "the persistent form is now off");
 }
 
+// The tiles of an nx x ny array along a Hilbert curve.
+template <typename F> static void hilbert_order(int nx, int ny, F &&visit)
+{
+    int side = 1;
+    while (side < nx || side < ny) side *= 2;
+    for (long d = 0; d < (long)side * side; d++) {
+        int x = 0, y = 0;
+        long q = d;
+        for (int s = 1; s < side; s *= 2) {
+            const int rx = 1 & (int)(q / 2), ry = 1 & (int)(q ^ rx);
+            if (ry == 0) {
+                if (rx == 1) {
+                    x = s - 1 - x;
+                    y = s - 1 - y;
+                }
+                std::swap(x, y);
+            }
+            x += s * rx;
+            y += s * ry;
+            q /= 4;
+        }
+        if (x < nx && y < ny) visit(x, y);
+    }
+}
+
 if_status Engine::refresh()
 {
     g_valid_ = false;  // the captured launches point at the old tables
@@ -797,15 +822,32 @@ if_status Engine::refresh()
     any_moving_ = false;
     any_monitor_ = false;
     const int sty = sweep_ty;
+    // Launches of one stage: tiles along a Hilbert curve, so that those in
+    // flight on an XCD (64 of the 128 x 128 blocks) form a compact patch and
+    // share most of their halos in its L2.  (A persistent launch finds its
+    // neighbours by the row-major index.)
+    const auto sweep_tiles = [&](const Slot &s) {
+        const int wo = sweep_kind == 1 ? stream_out_cols(sweep_m) : sweep_kind >= 2 ? reg_out_cols(sweep_m) : 0;
+        return make_int2(wo > 0 ? (s.NX + wo - 1) / wo : s.ntx, (s.NY + sty - 1) / sty);
+    };
+    int nsw = 0;
+    for (int id : order_) {
+        const int2 t = sweep_tiles(*slots_[id]);
+        nsw += t.x * t.y;
+    }
+    const bool hilbert = sweep_kind >= 2 && !(use_persistent && pers_fits(pprec_, reg_waves(sweep_kind), sty, sweep_m,
+                                                                          nsw, wmode_));
     for (int k = 0; k < n; k++) {
         Slot &s = *slots_[order_[k]];
         s.dev.ppe_m = s.dev.ppe_solver == IF_PPE_RBSOR ? std::max(1, sweep_m) : 1;
         cs[k] = s.dev;
         for (int t = 0; t < s.ntx * s.nty; t++) tb.push_back(make_int2(k, t));
-        const int ntys = (s.NY + sty - 1) / sty;
-        const int wo = sweep_kind == 1 ? stream_out_cols(sweep_m) : sweep_kind >= 2 ? reg_out_cols(sweep_m) : 0;
-        const int ntxs = wo > 0 ? (s.NX + wo - 1) / wo : s.ntx;
-        for (int t = 0; t < ntxs * ntys; t++) tsw.push_back(make_int2(k, t));
+        const int2 nsw_k = sweep_tiles(s);
+        const int ntxs = nsw_k.x, ntys = nsw_k.y;
+        if (hilbert)
+            hilbert_order(ntxs, ntys, [&](int x, int y) { tsw.push_back(make_int2(k, y * ntxs + x)); });
+        else
+            for (int t = 0; t < ntxs * ntys; t++) tsw.push_back(make_int2(k, t));
         max_ng_ = std::max(max_ng_, s.gcap);
         max_ring_ = std::max(max_ring_, std::max(s.nx, s.ny));
         max_cells_ = std::max(max_cells_, s.nx * s.ny);

@@ -1932,7 +1932,7 @@ __global__ void k_tune_arm(const CaseDev *cs, int ncase, const Ctrl *ctrl0, cons
     if (k >= ncase) return;
     Ctrl *c = cs[k].ctrl;
     *c = saved[c - ctrl0];
-    if (!c->active || c->failed || c->closed) return;
+    if (!c->active || c->failed) return;
     c->ppe_done = 0;
     c->ppe_sweeps = 0;
 }

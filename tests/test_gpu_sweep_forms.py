@@ -113,3 +113,16 @@ def test_persistent_line_equals_launches(precision, nx, ny, check):
     assert out[0][:2] == out[1][:2]
     for f in FIELDS:
         assert np.array_equal(out[0][2][f], out[1][2][f]), f
+
+
+def test_autotune_times_open_cases():
+    """The autotuner times sweeps that run.  One is two dependent half-sweeps
+    with a block barrier each, which take over 100 ns between them; launches over
+    a closed case take a few us for 256 sweeps, 10 to 20 ns each."""
+    n = 256
+    xf = _faces(n, 8.0, 0.0)
+    with iff.Case(xf, xf.copy(), precision=iff.IF_MIXED, dt=0.002, re=100.0, ppe_itermax=320, check_every=160) as c:
+        c.step(1)
+        assert c.autotune()["sweep_ns"] * n * n > 50.0
+        st = c.step(1)
+        assert st["persistent_timeouts"] == 0 and st["failed"] == 0

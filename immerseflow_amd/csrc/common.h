@@ -199,6 +199,7 @@ struct CaseDev {
     GhostDev *gh;
     BodyDev *bodies;
     Ctrl *ctrl;
+    void *xb;                      // persistent red-black sweep: three strip buffers, each as the field
     double *part;                  // one partial per interior tile
     int *gcount;                   // ghost-compaction scratch (per 1024 cells)
     Monitor *mon;                  // null: no monitors

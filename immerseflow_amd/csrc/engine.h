@@ -147,6 +147,9 @@ private:
     double *d_vals_ = nullptr;     // the persistent solve's residuals, two per tile
     unsigned *d_flags_ = nullptr;  // its per-tile stage counters
     int cap_flags_ = 0;
+    char *d_xb_ = nullptr;         // its strip buffers (CaseDev::xb)
+    size_t cap_xb_ = 0, used_xb_ = 0;
+    bool pers_ready_ = false;      // the red-black launches are persistent
     // persistent line SOR: the resident line cases' blocks of rows, a launch
     // for each number of cells a lane holds; none if any case has no such form
     struct LineGroup {

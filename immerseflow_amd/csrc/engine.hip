@@ -59,6 +59,7 @@ Engine::~Engine()
     if (d_tickets_) hipFree(d_tickets_);
     if (d_flags_) hipFree(d_flags_);
     if (d_vals_) hipFree(d_vals_);
+    if (d_xb_) hipFree(d_xb_);
     if (d_line_blocks_) hipFree(d_line_blocks_);
     if (d_line_flags_) hipFree(d_line_flags_);
     if (d_tiles_base_) hipFree(d_tiles_base_);
@@ -835,12 +836,41 @@ if_status Engine::refresh()
         const int2 t = sweep_tiles(*slots_[id]);
         nsw += t.x * t.y;
     }
-    const bool hilbert = sweep_kind >= 2 && !(use_persistent && pers_fits(pprec_, reg_waves(sweep_kind), sty, sweep_m,
-                                                                          nsw, wmode_));
+    // persistent chunks: a register-tile shape with such a form in this
+    // precision whose tiles are all resident at once, and its strip buffers
+    pers_ready_ = use_persistent && sweep_kind >= 2 && nsw > 0 &&
+                  pers_fits(pprec_, reg_waves(sweep_kind), sty, sweep_m, nsw, wmode_);
+    std::vector<size_t> xb_off(n, 0);
+    used_xb_ = 0;
+    if (pers_ready_)
+        for (int k = 0; k < n; k++) {
+            const Slot &s = *slots_[order_[k]];
+            if (s.desc.ppe_solver != IF_PPE_RBSOR) continue;
+            // (column 1 on an aligned address, as in the fields: a column pair is
+            // one aligned store)
+            const size_t es = pprec_ == IF_FP64 ? 8 : 4;
+            xb_off[k] = used_xb_ + 256 - es;
+            used_xb_ += 256 + align256(3 * (size_t)s.P * s.ny * es);
+        }
+    if (used_xb_ > cap_xb_) {
+        if (d_xb_) hipFree(d_xb_);
+        d_xb_ = nullptr;
+        cap_xb_ = 0;
+        if (hipMalloc(&d_xb_, used_xb_) == hipSuccess) {
+            cap_xb_ = used_xb_;
+        } else {  // one launch per stage then
+            (void)hipGetLastError();
+            d_xb_ = nullptr;
+            used_xb_ = 0;
+            pers_ready_ = false;
+        }
+    }
+    const bool hilbert = sweep_kind >= 2 && !pers_ready_;
     for (int k = 0; k < n; k++) {
         Slot &s = *slots_[order_[k]];
         s.dev.ppe_m = s.dev.ppe_solver == IF_PPE_RBSOR ? std::max(1, sweep_m) : 1;
         cs[k] = s.dev;
+        cs[k].xb = d_xb_ ? d_xb_ + xb_off[k] : nullptr;
         for (int t = 0; t < s.ntx * s.nty; t++) tb.push_back(make_int2(k, t));
         const int2 nsw_k = sweep_tiles(s);
         const int ntxs = nsw_k.x, ntys = nsw_k.y;
@@ -924,6 +954,7 @@ if_status Engine::refresh()
 if_status Engine::zero_flags()
 {
     if (cap_flags_ > 0) IFF_HIP(hipMemsetAsync(d_flags_, 0, sizeof(unsigned) * cap_flags_, st_));
+    if (used_xb_ > 0) IFF_HIP(hipMemsetAsync(d_xb_, 0xff, used_xb_, st_));  // empty strips
     if (cap_line_ > 0) IFF_HIP(hipMemsetAsync(d_line_flags_, 0, sizeof(unsigned) * cap_line_, st_));
     return IF_OK;
 }
@@ -1007,10 +1038,7 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         launch_step_begin(st_, d_cases_, n);
         launch_source(st_, vprec_, d_cases_, d_tiles_base_, nt_base_);
 
-        // persistent chunk: a register-tile shape with a persistent form in
-        // this precision, and the grid fits on the device
-        bool pers = any_rb && use_persistent && sweep_kind >= 2 &&
-                    pers_fits(pprec_, reg_waves(sweep_kind), tiles_sweep_ty_, M, nt_sweep_, wmode_);
+        bool pers = any_rb && pers_ready_;
         if (any_rb) launch_sweeps = pers ? K : M;
         bool lpers = any_line && use_persistent && !line_groups_.empty();
         // FP64: chunks and their checks in one launch, up to kSolveSweeps
@@ -1314,8 +1342,7 @@ if_status Engine::autotune(if_tune_result *out)
         // error buffers and advances the stage counters of every tile alike.
         // FP64 shapes are timed per stage: an FP64 persistent launch's
         // second stage would overwrite the solve's current pressure.
-        const bool pc = pprec_ != IF_FP64 && c.kind >= 2 && use_persistent &&
-                        pers_fits(pprec_, reg_waves(c.kind), c.ty, c.m, nt_sweep_, wmode_);
+        const bool pc = pprec_ != IF_FP64 && pers_ready_;
         const int kp = 32 * c.m;
         const int s0 = pprec_ == IF_FP64 ? 0 : c.m;
         auto timed = [&]() {

@@ -2,6 +2,7 @@
 #include "sweep_reg.h"
 
 #include <functional>
+#include <iterator>
 
 namespace iff {
 
@@ -56,18 +57,19 @@ static void pers_one(hipStream_t st, const CaseDev *cs, const int2 *tiles, int n
 // the latency of its half-sweeps and of the exchange after each stage, not by
 // arithmetic: low tiles (few rows per wave) shorten the one, deep stages the
 // other, and the halo they recompute costs nothing on idle CUs; from about one
-// tile per CU on the recomputation counts.  Measured (us per sweep, uniform
+// one tile per CU on the recomputation counts.  Measured (us per sweep, uniform
 // n x n, one circle):
 //   FP32   n   64: 64 x 8 (one tile) 0.46, 16 x 12 0.54, 32 x 16 0.60
-//             256: 16 x 12 0.60, 32 x 16 0.66, 48 x 12 0.75, 64 x 8 0.85, 96 x 8 1.04
-//             611: 32 x 16 0.71 (200 tiles), 16 x 12 0.79 (312), 64 x 8 0.94
-//             800: 48 x 12 0.81 (170), 32 x 16 1.11 (325), 64 x 8 0.92
-//            1024: 64 x 8 0.96 (176), 48 x 12 1.12 (286), 96 x 8 1.12
-//            1948: 96 x 8 1.94 (441, two per CU); per stage 64 x 8 2.88
-//   stretched 2048 x 1024: 64 x 8 1.66 (352), 96 x 8 1.79 (242)
+//             256: 16 x 12 0.56, 32 x 16 0.60, 48 x 12 0.66, 64 x 8 0.86, 96 x 8 1.02
+//             611: 32 x 16 0.64 (200 tiles), 48 x 12 0.70, 16 x 12 0.80 (312), 64 x 8 0.94
+//             800: 48 x 12 0.72 (170), 64 x 8 0.94, 32 x 16 1.15 (325, per stage)
+//            1024: 64 x 8 0.97 (176), 48 x 12 1.12 (286), 96 x 8 1.12
+//            1400: 96 x 8 1.29 (225), 64 x 8 1.34 (330, two per CU)
+//            1948: 96 x 8 1.88 (441, two per CU); per stage 64 x 8 2.8
+//   stretched 2048 x 1024: 96 x 8 1.19 (242), 64 x 8 1.60 (352)
 //   FP64   n   64: 64 x 4 (one tile) 0.96, 16 x 12 1.06
-//             256: 16 x 12 1.10, 32 x 8 1.30, 48 x 4 1.78, 80 x 4 2.38
-//             800: 32 x 8 1.43 (225), 48 x 8 1.59, 64 x 8 1.81
+//             256: 16 x 12 1.05, 32 x 8 1.15, 48 x 8 1.57
+//             800: 32 x 8 1.27 (225), 48 x 8 1.65, 64 x 8 1.81
 //            1024: 48 x 8 1.80 (242), 64 x 8 1.92, 48 x 4 2.2
 //   stretched 2048 x 1024: only 80 x 4 fits, 2.9
 // False: none fits.
@@ -78,7 +80,7 @@ bool reg_auto_shape(int prec, int wt, const std::function<int(int, int, int *)> 
         bool single;        // only where every case is one tile
     };
     static const Shape s32[] = {{64, 8, 2, true}, {16, 12, 1, false}, {32, 16, 1, false}, {48, 12, 1, false},
-                                {64, 8, 2, false}, {96, 8, 2, false}};
+                                {64, 8, 1, false}, {96, 8, 1, false},  {64, 8, 2, false},  {96, 8, 2, false}};
     static const Shape s64[] = {{64, 4, 1, true}, {16, 12, 1, false}, {32, 8, 1, false}, {48, 8, 1, false},
                                 {64, 8, 1, false}, {80, 4, 1, false}};
     static int cus = -1;  // one device type per process
@@ -89,7 +91,10 @@ bool reg_auto_shape(int prec, int wt, const std::function<int(int, int, int *)> 
             return false;
         cus = n;
     }
-    for (const Shape &s : prec == IF_FP64 ? s64 : s32) {
+    const Shape *const list = prec == IF_FP64 ? s64 : s32;
+    const int count = (int)(prec == IF_FP64 ? std::size(s64) : std::size(s32));
+    for (int k = 0; k < count; k++) {
+        const Shape &s = list[k];
         int most = 0;  // tiles of the largest case
         const int nt = tiles(s.ty, s.m, &most);
         if ((s.single && most > 1) || nt > s.per_cu * cus || !pers_fits(prec, 16, s.ty, s.m, nt, wt)) continue;

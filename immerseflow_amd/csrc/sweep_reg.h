@@ -35,6 +35,7 @@
 #include "kernels.h"
 #include "sor.h"
 
+#include <type_traits>
 #include <utility>
 
 namespace iff {
@@ -178,17 +179,16 @@ __device__ __forceinline__ void fast_rows(ROW &&row, PUB &&publish)
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// Neighbour synchronisation of the persistent sweep.  Every tile has a
-// stage counter (flags[t], advanced by the number of stages per launch by
-// every tile, so all counters agree when a launch starts).  A block
-// publishes "stage l done" after its border strips are written, then waits
-// until the tiles of its case that its halo reaches have published the same stage.
-// Strips are written and halos read at device scope (sc1: write-through,
-// and loads that miss in the per-XCD L2), so no cache flush is needed; the
-// waits are bounded: past bar->timeout ticks of the 100 MHz real-time
-// counter bar->err is set, every later wait returns at once and every
-// block stops at its next stage boundary, so the kernel always ends; the
-// host checks err after the step.
+// Synchronisation of the persistent sweep.  Between stages a tile's border
+// strips go to its neighbours through strip buffers that the readers poll
+// (k_rbsor_reg); every tile has a stage counter (flags[t]), which counts the
+// stages over all launches, so that all counters of a case agree when a launch
+// starts; the FP64 solve's checks wait for them.  Strips are written and read
+// at device scope (sc1: write-through, and loads that miss in the per-XCD
+// L2), so no cache flush is needed.  All waits are bounded: past
+// bar->timeout ticks of the 100 MHz real-time counter bar->err is set, every
+// later wait ends soon and every block stops at its next stage boundary, so
+// the kernel always ends; the host checks err after the step.
 constexpr unsigned kRsrc3 = 0x00020000;              // buffer resource word 3 (gfx9)
 
 // wait_neighbours (sor.h) for all n tiles of a case, by all threads of the block (the
@@ -215,24 +215,28 @@ __device__ __forceinline__ bool wait_all(const unsigned *flags, int n, unsigned 
 }  // namespace
 
 // PERS: one launch runs the chunk's K sweeps as stages of M
-// sweeps.  The tile stays in registers; after each stage a block writes the
-// border strips (depth 2M) of its stored region, waits for its neighbouring
-// tiles to have written theirs, and reloads its halo ring from them.  Stage
-// L leaves its output where launch L of the chunked form does
-// (FP32 e[(L + 1) & 1], FP64 p[(ppe_base + L + 1) & 1]), the last stage of
-// a case the whole stored region, so
-// the checks read the same buffer either way.  A block is at most one
-// stage ahead of its neighbours, so the two buffers never hold data a
-// neighbour still needs when they are overwritten.
+// sweeps.  The tile stays in registers; after each stage a block sends the
+// border strips (depth 2M) of its stored region and takes its halo ring from its
+// neighbours' strips.  The last stage leaves the whole stored region where
+// launches of M sweeps leave it (FP32 e[n & 1], FP64 p[(ppe_base + n) & 1] after
+// n of them), so the checks read the same buffer either way.
 //
 // The second launch bound holds the FP32 per-stage 128 x 128 blocks (16
 // waves x 8 rows) at 8 waves per SIMD, i.e. 64 VGPRs and two blocks per CU:
 // left free, some of them take a few more registers and run at one block
 // per CU, a third slower.
 template <typename T, int M, int NW, int NRW, bool PERS, int WM>
-__global__ __launch_bounds__(64 * NW, (sizeof(T) == 4 && NW == 16 && (PERS ? WM == 1 || (WM == 0 && NRW <= 6) : NRW == 8 && WM != 2)) ? 8 : 1)
+constexpr bool two_per_cu = sizeof(T) == 4 && NW == 16 &&
+                            (PERS ? M <= 8 && (WM == 1 || (WM == 0 && NRW <= 6)) : NRW == 8 && WM != 2);
+
+template <typename T, int M, int NW, int NRW, bool PERS, int WM>
+__global__ __launch_bounds__(64 * NW, (two_per_cu<T, M, NW, NRW, PERS, WM>) ? 8 : 1)
 void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pad, int s, int K, PersArgs pa)
 {
+    // PERS: neighbours poll the strips themselves; where the registers for it
+    // are not there (two blocks per CU, FP64 from 5 rows a wave: spills cost
+    // up to 1.9 us per sweep), each tile's stage counter (flags) tells them
+    constexpr bool kPoll = NW == 16 && (sizeof(T) == 4 ? !two_per_cu<T, M, NW, NRW, PERS, WM> : NRW <= 4);
     constexpr int H = 2 * M;
     constexpr int TW = 128 - 2 * H;   // stored columns per tile
     constexpr int TY = NW * NRW - 2 * H;  // stored rows per tile
@@ -247,7 +251,6 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
     // 256 LDS cycles, where three rows of updates take about 160.)
     __shared__ T xch[2][NW + 2][2][64];
     const int t = tile_of_block(ntiles_pad);
-    const int nstage = (K + M - 1) / M;  // PERS: stages of a plain launch
     GridBar *const bar = pa.bar;
     unsigned *const flags = pa.flags;
     const bool solve = PERS && sizeof(T) == 8 && pa.nchunk > 0;
@@ -258,15 +261,10 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
             const Ctrl *cc = cr.ctrl;
             run = cr.ppe_solver == IF_PPE_RBSOR && cc->active && !cc->ppe_done && cr.ppe_itermax > cc->ppe_sweeps;
         }
-        if (!run) {  // whole workgroup: nobody waits on this tile, advance its counter
-            if (solve) {
-                if (t < ntiles && tiles[t].y == 0 && threadIdx.x == 0) {
-                    const Ctrl *cc = cs[tiles[t].x].ctrl;
-                    check_case(pa.ncase, false, cc->active && !cc->ad_done, bar);
-                }
-            } else if (t < ntiles && threadIdx.x == 0) {
-                const unsigned f0 = __hip_atomic_load(&flags[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&flags[t], f0 + (unsigned)nstage, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (!run) {  // whole workgroup, every tile of the case alike
+            if (solve && t < ntiles && tiles[t].y == 0 && threadIdx.x == 0) {
+                const Ctrl *cc = cs[tiles[t].x].ctrl;
+                check_case(pa.ncase, false, cc->active && !cc->ad_done, bar);
             }
             return;
         }
@@ -548,12 +546,13 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
     };
     // nst is even: the half-sweeps run in pairs whose colour order is fixed
     // per wave, so each loop body is straight-line code
-    auto pairs = [&]<bool UNI>(int n) {
+    auto pairs = [&]<bool UNI>(int n, auto &&after) {
         if (Z == 0)
             publish.template operator()<1>(0);
         else
             publish.template operator()<0>(0);
         __syncthreads();
+        after();
         if (Z == 0) {
             for (int h = 0; h < n; h += 2) {
                 half.template operator()<0, UNI>(h);
@@ -566,29 +565,26 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
             }
         }
     };
-    // n half-sweeps (n even)
-    auto sweeps = [&](int n) {
+    // n half-sweeps (n even); after() runs once every wave of the block is here
+    auto sweeps = [&](int n, auto &&after) {
         if constexpr (WM == 2) {
             if (uni)
-                pairs.template operator()<true>(n);
+                pairs.template operator()<true>(n, after);
             else
-                pairs.template operator()<false>(n);
+                pairs.template operator()<false>(n, after);
         } else {
-            pairs.template operator()<sizeof(T) == 4 && WM == 1>(n);
+            pairs.template operator()<sizeof(T) == 4 && WM == 1>(n, after);
         }
     };
     // store the stored region of the tile (rows H .. H+TY-1, columns H ..
-    // H+TW-1), or only its border strips of depth H (the halo of the
-    // neighbouring tiles)
-    auto store = [&](T *out, bool border) {
+    // H+TW-1)
+    auto store = [&](T *out) {
         if (lane >= H / 2 && lane < 64 - H / 2) {
-            const bool lb = lane < H || lane >= 64 - H;
 #pragma unroll
             for (int k = 0; k < NRW; k++) {
                 const int rr = w * NRW + k;
                 const int gj = jt0 + k;
                 if (rr < H || rr >= H + TY || gj > ny - 2) continue;
-                if (border && !lb && rr >= 2 * H && rr < TY) continue;
                 T *row = out + (size_t)gj * P;  // wave-uniform
                 if (sizeof(T) == 8 && ((smask >> k) & 1u)) {  // kept cells are not written
                     if (R.wa[k] != (T)0) GW(row)[ga] = R.pa[k];
@@ -615,7 +611,7 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
         constexpr int RY = (H + TY - 1) / TY, NB = 3 * (2 * RY + 1) - 1;
         static_assert(TW >= H && NB < 64, "halo reach");
         int nb = -1;
-        if (w == 0 && lane < NB) {
+        if (!kPoll && w == 0 && lane < NB) {
             const int d = lane < NB / 2 ? lane : lane + 1;  // without the centre
             const int qx = tx + d % 3 - 1, qy = ty + d / 3 - RY;
             if (qx >= 0 && qx < ntxs && qy >= 0 && qy < ntys) nb = t - tl.y + qy * ntxs + qx;
@@ -634,23 +630,27 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
             if (!st) m_halo |= 1u << k;
         }
         // Buffer offsets: the lane's column in the vector offset, the row
-        // (wave-uniform) in the scalar offset.  Stores are not masked: a lane
-        // that stores nothing has an offset past every field, which the
+        // (wave-uniform) in the scalar offset.  Accesses are not masked: a lane
+        // that stores or loads nothing has an offset past every field, which the
         // buffer's bounds check drops.  An exec mask and its branches per row
         // made a stage's stores and loads about 600 instructions a wave.
-        const int voff = ga * (int)sizeof(T), kDrop = 0x7fffff00;
-        const bool stl = lane >= H / 2 && lane < 64 - H / 2, side = lane < H || lane >= 64 - H;
-        const bool two = ga + 1 <= nx - 2;
-        const int vo_all = stl && two ? voff : kDrop;           // every stored column pair
-        const int vo_side = stl && two && side ? voff : kDrop;  // the left and right strips
-        // a last interior column without a partner (odd widths)
-        const int vo_one = stl && ga == nx - 2 ? voff : kDrop;
-        const bool one = __any(stl && ga == nx - 2);
-        // halo loads: a pair with a cell on the domain's ring loads that too
-        // (its value only ever meets a zero coefficient; in FP32 it is 0)
-        const bool ldl = ga >= 0 && ga <= nx - 2;
-        const bool ld_side = ldl && (lane < H / 2 || lane >= 64 - H / 2);
-        // the chunk's two buffers: stage l writes buffer (l + 1) & 1
+        constexpr int kDrop = 0x7fffff00;
+        const bool stl = lane >= H / 2 && lane < 64 - H / 2;  // stored lanes
+        // Offsets and lane masks are formed from an opaque copy of the column
+        // where they are used, and the rows' masks made opaque there: held over
+        // the sweeps they do not fit in the registers.
+        auto column = [&]() {
+            int q = ga;
+            asm volatile("" : "+v"(q));
+            return q;
+        };
+        auto opaque = [](unsigned &a, unsigned &b) {
+            asm volatile("" : "+v"(a), "+v"(b));
+            a = (unsigned)uniform((int)a);
+            b = (unsigned)uniform((int)b);
+        };
+        // the launch reads its first values from buf0 and leaves its result in
+        // one of the two
         void *buf0, *buf1;
         if constexpr (sizeof(T) == 8) {
             buf0 = c.p[ct->ppe_base & 1];
@@ -714,10 +714,17 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
             }
             return wave_max(m);
         };
-        // stage output at device scope: the border strips, or (the end of
-        // the case) the whole stored region
+        // output at device scope: the border strips, or (the end of the case) the
+        // whole stored region
         auto put = [&](const __amdgpu_buffer_rsrc_t ro, bool whole) __attribute__((always_inline)) {
+            const int q = column(), ln = (q - c0) >> 1;
+            const bool st = ln >= H / 2 && ln < 64 - H / 2;
+            const int vo_all = st && q + 1 <= nx - 2 ? q * (int)sizeof(T) : kDrop;
+            const int vo_side = ln < H || ln >= 64 - H ? vo_all : kDrop;
             const unsigned m_all = whole ? m_st : m_strip;
+            // a last interior column without a partner (odd widths)
+            const int vo_one = st && q == nx - 2 ? q * (int)sizeof(T) : kDrop;
+            const bool one = __any(st && q == nx - 2);
 #pragma unroll
             for (int k = 0; k < NRW; k++) {
                 const int srow = (jt0 + k) * P * (int)sizeof(T);  // uniform: scalar offset
@@ -749,16 +756,167 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
                 }
             }
         };
+        // The exchange by polling.  A stage's strips go to one of three buffers
+        // laid out as the field, stage g (counted over launches) to buffer
+        // g % 3, and a reader polls the cells themselves: a word of all ones,
+        // which no value has (kHole, a NaN that cap() maps to its neighbour),
+        // means not yet written.  So a stage costs a store, its way to the reader
+        // and the reader's load; with a counter behind the strips it is a round
+        // trip and two barriers more.  FP32 256^2 0.60 -> 0.56 us per sweep,
+        // 611^2 0.71 -> 0.64, stretched 2048 x 1024 1.32 -> 1.19; FP64 800^2
+        // 1.55 -> 1.27.
+        // Buffer (g + 1) % 3 is emptied during stage g: what it holds, stage
+        // g - 2, has been read, since the neighbours' stage g - 1, sent after
+        // that, has arrived in every wave of this block; and it is empty
+        // before stage g is sent, so a neighbour that has stage g finds
+        // it empty or stage g + 1 in it.
+        constexpr unsigned kHole = 0xffffffffu;
+        auto cap = [](unsigned x) { return x < kHole ? x : kHole - 1u; };
+        auto strip_buf = [&](unsigned g) {
+            return __builtin_amdgcn_make_buffer_rsrc(uniform_ptr((char *)c.xb + (size_t)(g % 3u) * (size_t)nrec), 0, nrec,
+                                                     kRsrc3);
+        };
+        auto send = [&](const __amdgpu_buffer_rsrc_t xo, auto empty) __attribute__((always_inline)) {
+            // the strips, in column pairs: every stored column in the top and
+            // bottom strips' rows, else the left and right strips' columns
+            unsigned ms = m_st, mp = m_strip;
+            opaque(ms, mp);
+            const int q = column(), ln = (q - c0) >> 1;
+            const bool on = q >= 1 && q <= nx - 2 && ln >= H / 2 && ln < 64 - H / 2;
+            const int vs_all = on ? q * (int)sizeof(T) : kDrop;
+            const int vs_side = on && (ln < H || ln >= 64 - H) ? q * (int)sizeof(T) : kDrop;
+#pragma unroll
+            for (int k = 0; k < NRW; k++) {
+                const int srow = (jt0 + k) * P * (int)sizeof(T);
+                if (!((ms >> k) & 1u)) continue;
+                const int vo = ((mp >> k) & 1u) ? vs_all : vs_side;
+                if constexpr (sizeof(T) == 4) {
+                    U2 v = {kHole, kHole};
+                    if constexpr (!decltype(empty)::value)
+                        v = U2{cap(__float_as_uint(R.pa[k])), __float_as_uint(R.pb[k])};
+                    __builtin_amdgcn_raw_buffer_store_b64(v, xo, vo, srow, kDev);
+                } else {  // (two atoms of 8 bytes)
+                    U4 v = {kHole, kHole, kHole, kHole};
+                    if constexpr (!decltype(empty)::value) {
+                        const U2 a = __builtin_bit_cast(U2, R.pa[k]), b = __builtin_bit_cast(U2, R.pb[k]);
+                        v = U4{a[0], cap(a[1]), b[0], cap(b[1])};
+                    }
+                    __builtin_amdgcn_raw_buffer_store_b128(v, xo, vo, srow, kDev);
+                }
+            }
+        };
+        using XV = std::conditional_t<sizeof(T) == 4, U2, U4>;
+        // this wave's part of the halo ring: the cells of the tile outside its
+        // stored region that lie in the domain's interior.  true: give up.
+        // Four rows at once, without branches: their loads are in flight
+        // together.  (A row that is not in the domain, and a lane that takes
+        // nothing, read past the buffer: 0.)
+        auto receive = [&](const __amdgpu_buffer_rsrc_t xi) __attribute__((always_inline)) {
+            constexpr int kGroup = NRW <= 6 ? NRW : 4;
+            unsigned long long t0 = 0;
+            for (unsigned tries = 1;; tries++) {
+                asm volatile("" ::: "memory");  // (load again)
+                bool hole = false;
+                unsigned mh = m_halo, ms = m_st;
+                opaque(mh, ms);
+                const int q = column(), ln = (q - c0) >> 1;
+                const bool h_all = q >= 1 && q <= nx - 2, h_side = h_all && (ln < H / 2 || ln >= 64 - H / 2);
+                const int vh_all = h_all ? q * (int)sizeof(T) : kDrop, vh_side = h_side ? q * (int)sizeof(T) : kDrop;
+#pragma unroll
+                for (int k0 = 0; k0 < NRW; k0 += kGroup) {
+                    XV x[kGroup];
+#pragma unroll
+                    for (int r = 0; r < kGroup && k0 + r < NRW; r++) {
+                        const int k = k0 + r, srow = max(jt0 + k, 0) * P * (int)sizeof(T);
+                        const int vo = (mh >> k) & 1u ? vh_all : (ms >> k) & 1u ? vh_side : kDrop;
+                        if constexpr (sizeof(T) == 4)
+                            x[r] = __builtin_amdgcn_raw_buffer_load_b64(xi, vo, srow, kDev);
+                        else
+                            x[r] = __builtin_amdgcn_raw_buffer_load_b128(xi, vo, srow, kDev);
+                    }
+#pragma unroll
+                    for (int r = 0; r < kGroup && k0 + r < NRW; r++) {
+                        const int k = k0 + r;
+                        const bool mine = (mh >> k) & 1u ? h_all : (ms >> k) & 1u && h_side;
+                        const V2 v = __builtin_bit_cast(V2, x[r]);
+                        if constexpr (sizeof(T) == 4) {
+                            hole = hole || x[r][0] == kHole;
+                            R.pa[k] = mine ? v[0] : R.pa[k];
+                            R.pb[k] = mine ? v[1] : R.pb[k];
+                        } else {  // kept cells stay 0
+                            hole = hole || x[r][1] == kHole || x[r][3] == kHole;
+                            R.pa[k] = mine ? (R.wa[k] != (T)0 ? v[0] : (T)0) : R.pa[k];
+                            R.pb[k] = mine ? (R.wb[k] != (T)0 ? v[1] : (T)0) : R.pb[k];
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (!__any(hole)) return false;
+                if (tries % 4 == 0 && __hip_atomic_load(&bar->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)
+                    return true;
+                const unsigned long long now = __builtin_amdgcn_s_memrealtime();
+                if (t0 == 0) t0 = now;
+                if (now - t0 > bar->timeout) {
+                    __hip_atomic_store(&bar->err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    return true;
+                }
+            }
+        };
+        // The same from the output of a stage whose counters have been seen.
+        // (A pair with a cell on the domain's ring loads that too: its value
+        // only ever meets a zero coefficient.)
+        auto reload = [&](const __amdgpu_buffer_rsrc_t ro) __attribute__((always_inline)) {
+            const int q = column(), ln = (q - c0) >> 1;
+            const bool ldl = q >= 0 && q <= nx - 2, ld_side = ldl && (ln < H / 2 || ln >= 64 - H / 2);
+            auto halo = [&](unsigned rows) {
+#pragma unroll
+                for (int k = 0; k < NRW; k++) {
+                    if (!((rows >> k) & 1u)) continue;
+                    const int srow = (jt0 + k) * P * (int)sizeof(T);
+                    V2 v;
+                    if constexpr (sizeof(T) == 4)
+                        v = __builtin_bit_cast(V2, __builtin_amdgcn_raw_buffer_load_b64(ro, q * 4, srow, kDev));
+                    else
+                        v = __builtin_bit_cast(V2, __builtin_amdgcn_raw_buffer_load_b128(ro, q * 8, srow, kDev));
+                    if constexpr (sizeof(T) == 8) {  // kept cells stay 0
+                        R.pa[k] = R.wa[k] != (T)0 ? v[0] : (T)0;
+                        R.pb[k] = R.wb[k] != (T)0 ? v[1] : (T)0;
+                    } else {
+                        R.pa[k] = v[0];
+                        R.pb[k] = v[1];
+                    }
+                }
+            };
+            if (ld_side) halo(m_st);
+            if (ldl) halo(m_halo);
+        };
+        __shared__ int stuck;  // a wave of the block has given up
+        if (threadIdx.x == 0) stuck = 0;
         __shared__ double red[sizeof(T) == 8 ? NW : 1];
         int done = 0, chunk = 0;      // sweeps and chunks behind the running chunk
         int kc = kexec, rest = kexec;  // sweeps of the running chunk, and what is left of them
         bool whole = false;
+        unsigned sent = 3u;  // bit q: stage g - 1 - q used its strip buffer (before the launch: maybe)
         int l = 0;
         for (;; l++) {
             int me = alone || rest < M ? rest : M;
             if (solve && !alone && rest == M) me = (M + 1) / 2;
-            sweeps(2 * me);
+            const unsigned g = f0 + (unsigned)l;
+            sweeps(2 * me, [&] {
+                if constexpr (kPoll)
+                    if (!alone && (sent & 2u)) send(strip_buf(g + 1u), std::true_type{});
+            });
             rest -= me;
+            // after a timed-out wait anywhere in the launch, stop sweeping: the
+            // fields in memory are finite, the step reports the failure and
+            // the solve resumes from the current pressure
+            if (kPoll && __builtin_amdgcn_readfirstlane(stuck)) {
+                if (solve && tl.y == 0 && threadIdx.x == 0) {
+                    ctw->ppe_done = 2;
+                    check_case(pa.ncase, false, false, bar);
+                }
+                break;
+            }
             const bool check = solve && rest == 0;
             const bool last = !solve && rest == 0;
             // (a plain launch leaves its output where launches of M sweeps do)
@@ -768,7 +926,16 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
                 if (lane == 0) red[w] = m;
                 __syncthreads();
             }
-            if (!alone || last) put(ro, last);
+            // at a check the tiles wait for each other all together anyway: the
+            // strips go with the counters
+            const bool poll = kPoll && !check;
+            sent = sent << 1 | (poll ? 1u : 0u);
+            if (kPoll && !last && poll && !alone) {
+                __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);  // (the emptied strips)
+                send(strip_buf(g), std::false_type{});
+            } else if (!alone || last) {
+                put(ro, last);
+            }
             if (last) break;
             if (check && threadIdx.x == 0) {
                 double m = red[0];
@@ -777,21 +944,18 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
                 __hip_atomic_store(&pa.vals[(size_t)(chunk & 1) * ntiles + t], m, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
             }
-            if (!alone) {
-                // publish stage l once every wave's stores are complete, wait
-                // for the neighbours' stage l (at a check: every tile's)
+            if (!alone && !poll) {
+                // the stage's counter, behind this block's stores; wait for the
+                // tiles the halo reaches, at a check for all tiles of the case
                 __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
                 __syncthreads();
                 if (threadIdx.x == 0)
-                    __hip_atomic_store(&flags[t], f0 + (unsigned)(l + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                // after a timed-out wait anywhere in the launch, stop sweeping:
-                // the fields keep finite values, the step reports the
-                // failure and the solve resumes from the current pressure
-                const bool bad = check ? wait_all(flags + (t - tl.y), ntxs * ntys, f0 + (unsigned)(l + 1), bar)
-                                       : w == 0 && wait_neighbours(flags, nb, f0 + (unsigned)(l + 1), bar);
+                    __hip_atomic_store(&flags[t], g + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const bool bad = check ? wait_all(flags + (t - tl.y), ntxs * ntys, g + 1u, bar)
+                                       : w == 0 && wait_neighbours(flags, nb, g + 1u, bar);
                 if (__builtin_amdgcn_readfirstlane(__syncthreads_or(bad))) {
-                    // (at a check other tiles may have seen every flag and end
-                    // here: this one leaves its part of the result too)
+                    // (at a check other tiles may have seen every counter and
+                    // end here: this one leaves its part of the result too)
                     whole = check;
                     if (solve && tl.y == 0 && threadIdx.x == 0) {
                         ctw->ppe_done = 2;
@@ -831,41 +995,23 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
                 if (alone) __syncthreads();  // red is read before the next chunk's maxima
             }
             if (alone) continue;
-            // halo ring: the cells of the tile outside its stored region
-            // that lie in the domain's interior (device-scope loads)
-            auto halo = [&](unsigned rows) {
-#pragma unroll
-                for (int k = 0; k < NRW; k++) {
-                    if (!((rows >> k) & 1u)) continue;
-                    const int srow = (jt0 + k) * P * (int)sizeof(T);
-                    V2 v;
-                    if constexpr (sizeof(T) == 4)
-                        v = __builtin_bit_cast(V2, __builtin_amdgcn_raw_buffer_load_b64(ro, voff, srow, kDev));
-                    else
-                        v = __builtin_bit_cast(V2, __builtin_amdgcn_raw_buffer_load_b128(ro, voff, srow, kDev));
-                    if constexpr (sizeof(T) == 8) {  // kept cells stay 0
-                        R.pa[k] = R.wa[k] != (T)0 ? v[0] : (T)0;
-                        R.pb[k] = R.wb[k] != (T)0 ? v[1] : (T)0;
-                    } else {
-                        R.pa[k] = v[0];
-                        R.pb[k] = v[1];
-                    }
-                }
-            };
-            if (ld_side) halo(m_st);
-            if (ldl) halo(m_halo);
+            if (poll) {
+                if constexpr (kPoll)
+                    if (receive(strip_buf(g))) stuck = 1;
+            } else {
+                reload(ro);
+            }
         }
-        if (solve) {  // (every stage has advanced the counter)
+        if (solve) {
             if (whole) put((l + 1) & 1 ? rs1 : rs0, true);
-            return;
+        } else if (!alone && threadIdx.x == 0) {
+            // (a case's counters agree when a launch starts)
+            __hip_atomic_store(&flags[t], f0 + (unsigned)(l + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        __syncthreads();
-        if (threadIdx.x == 0)
-            __hip_atomic_store(&flags[t], f0 + (unsigned)nstage, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return;
     }
-    sweeps(nst);
-    store(dst, false);
+    sweeps(nst, [] {});
+    store(dst);
 }
 
 }  // namespace iff

@@ -1353,17 +1353,20 @@ if_status Engine::autotune(if_tune_result *out)
                 sweep_launch(c, s0, 2 * c.m);
         };
         launch_tune_arm(st_, d_cases_, n, d_ctrl_, saved);
+        // (32 stages of a persistent launch are a long measurement by
+        // themselves: eight launches of each shape took 18 ms on 2048 x 1024)
+        const int reps = pc ? 2 : kReps;
         timed();  // warm-up
-        timed();
+        if (!pc) timed();
         (void)hipEventRecord(e0, st_);
-        for (int r = 0; r < kReps; r++) timed();
+        for (int r = 0; r < reps; r++) timed();
         (void)hipEventRecord(e1, st_);
         float ms = 0.f;
         if (!elapsed(&ms)) {
             rc = fail(IF_ERR_HIP, "autotune: timing failed");
             break;
         }
-        const double ns = 1e6 * (double)ms / (kReps * (double)(pc ? kp : c.m) * cells);
+        const double ns = 1e6 * (double)ms / (reps * (double)(pc ? kp : c.m) * cells);
         ncand++;
         if (ns < best_ns) {
             best_ns = ns;

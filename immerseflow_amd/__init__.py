@@ -276,10 +276,10 @@ class Case:
         """Poisson sweep kernel (0 LDS-tiled, 1 register-streaming, 2/3/4
         register-tile with 4/8/16 waves), tile or strip height, red-black
         sweeps per launch, sweeps per check.  Every kernel and shape gives
-        the same result.  Without a call the library uses 4/64/8 (mixed)
-        or, in FP64, 4/48, 4/64 or 4/80 with 4 sweeps as persistent
-        chunks (the smallest height that fits on the device) else 3/32/4, and
-        the case's check_every."""
+        the same result.  Without a call the shape follows the grids: a
+        persistent one that fits on the device (low tiles and deep stages for
+        small grids), else 4/88/10 or 4/64/8 (mixed), 3/32/4 (FP64), and the
+        case's check_every."""
         _check(_lib().if_case_tune(self._h, kernel, tile_y, sweeps_per_launch, check_every), "tune")
 
     def restart(self, u, v, p, uf=None, vf=None):

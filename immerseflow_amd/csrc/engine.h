@@ -67,15 +67,15 @@ public:
     Slot *slot(int k) { return (k >= 0 && k < (int)slots_.size()) ? slots_[k].get() : nullptr; }
 
     // Poisson sweep variant and check cadence (autotuned or user-set)
-    // (FP64 defaults; the constructor sets 4, 64, 8 for mixed precision)
+    // (until tuned refresh() sets the shape)
     int sweep_kind = 3;  // 0: LDS-tiled, 1: register-streaming, 2/3/4: register-tile (4/8/16 waves)
     int sweep_ty = 32, sweep_m = 4, check_k = 10;
-    bool shape_auto = true;  // FP64: the shape follows the resident set (refresh) until tuned
+    bool shape_auto = true;  // the shape follows the resident set (refresh) until tuned
     bool timing = false;
-    // replay each chunk of Poisson sweep launches from a captured hipGraph
+    // replay each chunk of several Poisson sweep launches from a captured hipGraph
     bool use_graphs = true;
-    // mixed precision, register-tile shapes: run each chunk as one
-    // persistent launch when all its blocks fit on the device at once
+    // run each chunk as one persistent launch (FP64: a solve) when the shape
+    // has that form and all blocks fit on the device at once
     bool use_persistent = true;
     double sweep_ms = 0.0;
     long long sweep_launches = 0;

@@ -252,28 +252,33 @@ if_status if_case_ghosts(if_case *c, int32_t *out, if_ghost *recs,
  * each direction and recomputes the rest).  Several red-black sweeps per launch is
  * temporal blocking; check_every is the number of sweeps between
  * convergence checks.  Results do not depend on the kernel, the tile
- * height or the sweeps per launch.  Defaults: kernel 4, 64 rows, 8 sweeps
- * (mixed); FP64 (until tuned): kernel 4, 4 sweeps as persistent chunks of
- * the smallest tile height of 48, 64 and 80 rows whose tiles fit on the
- * device in one launch, else kernel 3, 32 rows, 4 sweeps. */
+ * height or the sweeps per launch.  Until tuned, a case or batch runs kernel
+ * 4 in a shape that follows its grids: the first of a list of persistent
+ * shapes whose tiles fit on the device in one launch, low tiles with deep
+ * stages for small grids (mixed: 16 rows x 12 sweeps, 32 x 16, 48 x 12, 64 x 8,
+ * 96 x 8; FP64: 16 x 12, 32 x 8, 48 x 8, 64 x 8, 80 x 4; some of these shapes
+ * are the library's own and not accepted here); where none fits, launches of
+ * one stage: mixed 88 rows x 10 sweeps or 64 x 8, FP64 kernel 3, 32 x 4. */
 if_status if_case_tune(if_case *c, int kernel, int tile_y, int sweeps_per_launch,
                        int check_every);
 /* Launch mode of the Poisson sweeps (no counterpart in the reference,
  * whose PPESolver launches each Jacobi sweep from the host,
  * PPESolver.cu:172-189).  enable = 1 (the default): each chunk of
- * check_every sweeps is captured once into a hipGraph of kernel nodes and
- * replayed, recaptured when the resident set or the launch shape changes;
- * 0: the same kernels are launched one by one.  Results are identical. */
+ * check_every sweeps that takes several launches is captured once into a
+ * hipGraph of kernel nodes and replayed, recaptured when the resident set or
+ * the launch shape changes; 0: the same kernels are launched one by one.  Results are identical. */
 if_status if_case_graphs(if_case *c, int enable);
 /* Persistent Poisson chunks (no counterpart in the reference).  enable = 1
  * (the default): with a register-tile shape that has a persistent form
  * (mixed: 16 waves x 96/64 rows x 8 sweeps, 16 x 48 x 4, 8 x 32 x 8 and
- * 8 x 32 x 4; FP64: 16 x 80 x 4 and 16 x 48 x 4), when every block of the
- * launch can be resident on the device at once, each chunk of check_every
- * sweeps runs as one launch whose tiles stay in registers, in stages of
- * sweeps_per_launch sweeps separated by a halo exchange with the
- * neighbouring tiles; otherwise one launch per stage.  Results are
- * identical.  A neighbour wait that times out (20 ms; the blocks were not
+ * 8 x 32 x 4; FP64: 16 x 80/64/48 x 4 and 16 x 64/32 x 8; and the default
+ * shapes), when every block of the launch can be resident on the device at
+ * once, each chunk of check_every sweeps runs as one launch whose tiles
+ * stay in registers, in stages of sweeps_per_launch sweeps separated by a
+ * halo exchange with the neighbouring tiles (FP64: the convergence checks
+ * too, up to a whole solve in one launch); otherwise one launch per
+ * stage.  Line SOR cases of up to 512 interior columns run their chunks the
+ * same way.  Results are identical.  A neighbour wait that times out (20 ms; the blocks were not
  * all resident) ends that solve early with a finite pressure; the step then
  * turns the form off, solves again from that pressure with one launch per
  * stage, completes as usual (converged to the same stop level) and counts

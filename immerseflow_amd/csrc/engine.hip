@@ -25,7 +25,7 @@
 
 namespace iff {
 
-constexpr int kSolveSweeps = 4096;  // sweeps of a persistent FP64 solve launch
+constexpr int kSolveSweeps = 2048;  // sweeps of a persistent FP64 solve launch (a few ms: others share the device)
 constexpr int kTileY = kTileRows;  // base tiling (reductions, stencil passes)
 
 // viscous iterations enqueued when the last step tells nothing, and at a time
@@ -745,29 +745,33 @@ if_status Engine::check_barrier()
                             "the persistent form is now off");
 }
 
-// The tiles of an nx x ny array along a Hilbert curve.
+// The tiles of an nx x ny array along Hilbert curves: one in each square of
+// the shorter side, one square after the other.
 template <typename F> static void hilbert_order(int nx, int ny, F &&visit)
 {
     int side = 1;
-    while (side < nx || side < ny) side *= 2;
-    for (long d = 0; d < (long)side * side; d++) {
-        int x = 0, y = 0;
-        long q = d;
-        for (int s = 1; s < side; s *= 2) {
-            const int rx = 1 & (int)(q / 2), ry = 1 & (int)(q ^ rx);
-            if (ry == 0) {
-                if (rx == 1) {
-                    x = s - 1 - x;
-                    y = s - 1 - y;
+    while (side < std::min(nx, ny)) side *= 2;
+    auto curve = [&](int ox, int oy) {
+        for (int d = 0; d < side * side; d++) {
+            int x = 0, y = 0, q = d;
+            for (int s = 1; s < side; s *= 2) {
+                const int rx = 1 & (q / 2), ry = 1 & (q ^ rx);
+                if (ry == 0) {
+                    if (rx == 1) {
+                        x = s - 1 - x;
+                        y = s - 1 - y;
+                    }
+                    std::swap(x, y);
                 }
-                std::swap(x, y);
+                x += s * rx;
+                y += s * ry;
+                q /= 4;
             }
-            x += s * rx;
-            y += s * ry;
-            q /= 4;
+            if (ox + x < nx && oy + y < ny) visit(ox + x, oy + y);
         }
-        if (x < nx && y < ny) visit(x, y);
-    }
+    };
+    for (int oy = 0; oy < ny; oy += side)
+        for (int ox = 0; ox < nx; ox += side) curve(ox, oy);
 }
 
 if_status Engine::refresh()
@@ -842,7 +846,7 @@ if_status Engine::refresh()
                   pers_fits(pprec_, reg_waves(sweep_kind), sty, sweep_m, nsw, wmode_);
     std::vector<size_t> xb_off(n, 0);
     used_xb_ = 0;
-    if (pers_ready_)
+    if (pers_ready_ && pers_polls(pprec_, reg_waves(sweep_kind), sty, sweep_m, wmode_))
         for (int k = 0; k < n; k++) {
             const Slot &s = *slots_[order_[k]];
             if (s.desc.ppe_solver != IF_PPE_RBSOR) continue;
@@ -1500,6 +1504,10 @@ if_status Engine::get_field(int k, int which, double *out, size_t n)
     double *d = dense_scratch(s->dev, vprec_);
     launch_pack(st_, f.type, f.at, s->P, f.i0, f.j0, f.w, f.h, d);
     IFF_HIP(hipGetLastError());
+    // The caller's pages, meanwhile: a fresh buffer's are faulted in here by the
+    // CPU (large pages where there are any), not one by one when the copy pins
+    // them.
+    for (size_t b = 0; b < need * sizeof(double); b += 4096) ((volatile char *)out)[b] = 0;
     IFF_HIP(hipMemcpyAsync(out, d, need * sizeof(double), hipMemcpyDeviceToHost, st_));
     IFF_HIP(hipStreamSynchronize(st_));
     return IF_OK;

@@ -37,6 +37,7 @@ void launch_ppe_sweep_reg(hipStream_t st, int prec, int waves, int ty, int m, co
 // table changes.
 bool pers_fits(int prec, int waves, int ty, int m, int nt, int wt);
 int pers_blocks(int prec, int waves, int ty, int m, int wt);  // 0: no persistent form
+bool pers_polls(int prec, int waves, int ty, int m, int wt);  // it needs strip buffers (CaseDev::xb)
 // the default shape (kernel 4): tiles(tile_y, m, &most) counts the tiles of all
 // cases and of the largest one
 bool reg_auto_shape(int prec, int wt, const std::function<int(int, int, int *)> &tiles, int *ty, int *m);

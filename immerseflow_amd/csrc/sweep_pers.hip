@@ -121,6 +121,22 @@ int pers_blocks(int prec, int waves, int ty, int m, int wt)
     return 0;
 }
 
+bool pers_polls(int prec, int waves, int ty, int m, int wt)
+{
+#define IFF_PP(T_, W_, M_, TY_, NRW_)                                    \
+    if (waves == W_ && m == M_ && ty == TY_)                             \
+        return wt == 1                       ? polls<T_, M_, W_, NRW_, 1> \
+               : wt == 2 && sizeof(T_) == 4 ? polls<T_, M_, W_, NRW_, 2> \
+                                             : polls<T_, M_, W_, NRW_, 0>;
+    if (prec == IF_FP64) {
+        IFF_PERS_SHAPES64(IFF_PP)
+    } else {
+        IFF_PERS_SHAPES32(IFF_PP)
+    }
+#undef IFF_PP
+    return false;
+}
+
 bool pers_fits(int prec, int waves, int ty, int m, int nt, int wt)
 {
     const int pad = ((nt + 7) / 8) * 8;

@@ -229,14 +229,17 @@ template <typename T, int M, int NW, int NRW, bool PERS, int WM>
 constexpr bool two_per_cu = sizeof(T) == 4 && NW == 16 &&
                             (PERS ? M <= 8 && (WM == 1 || (WM == 0 && NRW <= 6)) : NRW == 8 && WM != 2);
 
+// PERS: neighbours poll the strips themselves; where the registers for it
+// are not there (two blocks per CU, FP64 from 5 rows a wave: spills cost up to
+// 1.9 us per sweep), each tile's stage counter (flags) tells them
+template <typename T, int M, int NW, int NRW, int WM>
+constexpr bool polls = NW == 16 && (sizeof(T) == 4 ? !two_per_cu<T, M, NW, NRW, true, WM> : NRW <= 4);
+
 template <typename T, int M, int NW, int NRW, bool PERS, int WM>
 __global__ __launch_bounds__(64 * NW, (two_per_cu<T, M, NW, NRW, PERS, WM>) ? 8 : 1)
 void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pad, int s, int K, PersArgs pa)
 {
-    // PERS: neighbours poll the strips themselves; where the registers for it
-    // are not there (two blocks per CU, FP64 from 5 rows a wave: spills cost
-    // up to 1.9 us per sweep), each tile's stage counter (flags) tells them
-    constexpr bool kPoll = NW == 16 && (sizeof(T) == 4 ? !two_per_cu<T, M, NW, NRW, PERS, WM> : NRW <= 4);
+    constexpr bool kPoll = PERS && polls<T, M, NW, NRW, WM>;
     constexpr int H = 2 * M;
     constexpr int TW = 128 - 2 * H;   // stored columns per tile
     constexpr int TY = NW * NRW - 2 * H;  // stored rows per tile

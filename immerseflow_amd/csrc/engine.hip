@@ -1061,6 +1061,7 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         // the host through the progress word.  One chunk is queued behind the
         // running one; the chunks behind the last case's end do nothing.
         const int nchunks = (max_ppe_ + K - 1) / K;
+        int ad_enq = 0;  // viscous iterations enqueued
         unsigned long long word = 0;
         // The step's end, per case and once (step_tail); where no monitor
         // samples it, enqueued behind the chunk that ended the last step's
@@ -1078,7 +1079,15 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
             const unsigned long long base = checks_;
             tail_in = false;
             if (entry_check) check(0);
+            // a case whose viscous loop is still open gets its iterations now: its
+            // solve would otherwise start when the others' had ended
+            auto ad_open = [&]() { return (word & kProgAdOpen) && ad_enq < max_ad_; };
             if (pers && solve) {
+                if (n > 1) {
+                    if_status r = wait_checks(base, 0, &word);
+                    if (r != IF_OK) return r;
+                    if (ad_open()) return IF_OK;
+                }
                 for (int u = 0; u < nchunks; u += nsolve) {
                     launch_ppe_sweep_pers(st_, pprec_, reg_waves(sweep_kind), tiles_sweep_ty_, M, d_cases_,
                                           d_tiles_sweep_, nt_sweep_, K,
@@ -1111,6 +1120,7 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
                     tail_in = expect;
                     return IF_OK;
                 }
+                if (ad_open()) return IF_OK;
             }
             return wait_checks(base, 0, &word);
         };
@@ -1121,7 +1131,7 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         // report it, and the passes from here on are enqueued again.
         // (Enqueueing the whole budget cost three launches for each of the 20
         // iterations of 25 that a step does not need: half of a 64^2 step.)
-        int ad_enq = 0, ad_next = ad_pred_ > 0 ? ad_pred_ : kAdFirst;
+        int ad_next = ad_pred_ > 0 ? ad_pred_ : kAdFirst;
         if (timing) launch_stamp_reset(st_, d_stamps_);
         do {
             for (int k = 0; k < ad_next && ad_enq < max_ad_; k++, ad_enq++) {

@@ -715,9 +715,9 @@ def line_sor_f2(iff, configs, a):
             t0 = time.perf_counter()
             st = c.step(steps)
             dt = time.perf_counter() - t0
-            ms, nsw = c.sweep_timing(reset=True)
+            ms, _ = c.sweep_timing(reset=True)
             c.close()
-            us = 1e3 * ms / max(1, nsw)
+            us = 1e3 * ms / max(1, st["total_ppe_sweeps"])
             r = dict(us_per_sweep=round(us, 2), mcell_sweeps_per_s=round(NX * NY / us, 1) if us > 0 else None)
             if cname == "c1":
                 r.update(ms_per_step=round(1e3 * dt / steps, 2), sweeps_last_step=st["ppe_sweeps"],

@@ -56,7 +56,7 @@ static void pers_one(hipStream_t st, const CaseDev *cs, const int2 *tiles, int n
 // device as one persistent launch, in this order.  A small grid is bound by
 // the latency of its half-sweeps and of the exchange after each stage, not by
 // arithmetic: low tiles (few rows per wave) shorten the one, deep stages the
-// other, and the halo they recompute costs nothing on idle CUs; from about one
+// other, and the halo they recompute costs nothing on idle CUs; from about
 // one tile per CU on the recomputation counts.  Measured (us per sweep, uniform
 // n x n, one circle):
 //   FP32   n   64: 64 x 8 (one tile) 0.46, 16 x 12 0.54, 32 x 16 0.60

@@ -34,6 +34,7 @@
 #include "common.h"
 #include "kernels.h"
 #include "sor.h"
+#include "stages.h"
 
 #include <type_traits>
 #include <utility>
@@ -812,8 +813,8 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
         // this wave's part of the halo ring: the cells of the tile outside its
         // stored region that lie in the domain's interior.  true: give up.
         // Four rows at once, without branches: their loads are in flight
-        // together.  (A row that is not in the domain, and a lane that takes
-        // nothing, read past the buffer: 0.)
+        // together.  (A lane that takes nothing, and every lane of a row outside
+        // the domain, has an offset past the field: 0.)
         auto receive = [&](const __amdgpu_buffer_rsrc_t xi) __attribute__((always_inline)) {
             constexpr int kGroup = NRW <= 6 ? NRW : 4;
             unsigned long long t0 = 0;
@@ -830,7 +831,7 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
                     XV x[kGroup];
 #pragma unroll
                     for (int r = 0; r < kGroup && k0 + r < NRW; r++) {
-                        const int k = k0 + r, srow = max(jt0 + k, 0) * P * (int)sizeof(T);
+                        const int k = k0 + r, srow = strip_row(jt0 + k, ny) * P * (int)sizeof(T);
                         const int vo = (mh >> k) & 1u ? vh_all : (ms >> k) & 1u ? vh_side : kDrop;
                         if constexpr (sizeof(T) == 4)
                             x[r] = __builtin_amdgcn_raw_buffer_load_b64(xi, vo, srow, kDev);

@@ -1,0 +1,38 @@
+"""The index rules of the persistent sweep's exchange (csrc/stages.h), compiled
+by the host compiler: the rows that its strip loads address."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "immerseflow_amd", "csrc")
+
+
+def _run(tmp_path, body):
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if not cxx:
+        pytest.skip("no host C++ compiler")
+    src, exe = tmp_path / "t.cpp", tmp_path / "t"
+    src.write_text('#include "stages.h"\n#include <cstdio>\n#include <initializer_list>\nusing namespace iff;\nint main() {\n' + body + "\nreturn 0;\n}\n")
+    subprocess.run([cxx, "-std=c++20", "-O1", "-Wall", "-Werror", "-I", CSRC, str(src), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_strip_rows_lie_in_the_field(tmp_path):
+    """Every row of every tile, for tile heights and halos around those in use
+    and grids from three rows up, addresses a row of the field, and a row of
+    the field addresses itself."""
+    _run(tmp_path, """
+    for (int ny = 3; ny < 700; ny++)
+        for (int ty : {16, 32, 48, 64, 80, 96})
+            for (int h : {8, 16, 24, 32})
+                for (int t = 0; t * ty < ny - 2; t++)
+                    for (int k = 0; k < ty + 2 * h; k++) {
+                        const int j = 1 + t * ty - h + k, row = strip_row(j, ny);
+                        if (row < 0 || row >= ny || (j >= 0 && j < ny && row != j)) {
+                            std::printf("ny %d row %d -> %d\\n", ny, j, row);
+                            return 1;
+                        }
+                    }""")

@@ -1101,7 +1101,9 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
                         return IF_OK;
                     }
                 }
-                return IF_OK;
+                // (no launch where no case may sweep: the entry check's word
+                // still tells of open viscous loops)
+                return wait_checks(base, 0, &word);
             }
             for (int u = 0; u < nchunks; u++) {
                 if (graph) {

@@ -1,0 +1,35 @@
+"""The step loop's bookkeeping: a step that returns has ended for every case,
+however many viscous iterations and sweeps its cases take or are allowed."""
+import numpy as np
+import pytest
+
+import immerseflow_amd as iff
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ("u", "v", "p", "uf", "vf")
+# a creeping flow: dt / (re dx^2) = 10, so that a viscous loop takes hundreds
+# of iterations
+SLOW = dict(dt=0.05, re=0.05, ad_tol=1e-6)
+
+
+def _faces(n):
+    return np.linspace(0.0, 20.0, n + 1)
+
+
+@pytest.mark.parametrize("precision", [iff.IF_FP64, iff.IF_MIXED])
+def test_step_without_sweeps_ends(require_gpu, precision):
+    """No Poisson sweep allowed, and more viscous iterations than a step
+    enqueues at first: the step still projects, as with one launch per stage."""
+    print("[gpu-test] no sweeps, long viscous loop", precision, flush=True)
+    out = []
+    for persistent in (True, False):
+        with iff.Case(_faces(64), _faces(48), precision=precision, bodies=[iff.circle(6.0, 10.0, 2.0)], ad_itermax=120,
+                      ppe_itermax=0, check_every=10, **SLOW) as c:
+            c.persistent(persistent)
+            st = [c.step(1) for _ in range(2)]
+            assert [s["ad_iters"] for s in st] == [120, 120]
+            out.append(([s["div_max"] for s in st], {f: c.get(f) for f in FIELDS}))
+    assert out[0][0] == out[1][0] and min(out[0][0]) > 0.0
+    for f in FIELDS:
+        assert np.array_equal(out[0][1][f], out[1][1][f]), f

@@ -1196,6 +1196,8 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         ad_pred_ = 0;
         int most = 0;
         for (int id : order_) {
+            if (all[id].active && !all[id].closed)
+                return fail(IF_ERR_HIP, "step: a case's loops had not ended at the step's end");
             ad_pred_ = std::max(ad_pred_, all[id].ad_iter + 1);
             most = std::max(most, all[id].ppe_sweeps);
         }

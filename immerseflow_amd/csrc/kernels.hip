@@ -1376,6 +1376,7 @@ __global__ void k_ppe_rearm(const CaseDev *cs, int ncase)
     if (k >= ncase) return;
     Ctrl *c = cs[k].ctrl;
     if (!c->active || c->failed || c->closed) return;
+    if (!c->ad_done) return;  // opens with the end of its viscous loop (k_ad_finish)
     c->ppe_done = 0;
     c->ppe_sweeps = 0;
 }

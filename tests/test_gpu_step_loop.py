@@ -33,3 +33,36 @@ def test_step_without_sweeps_ends(require_gpu, precision):
     assert out[0][0] == out[1][0] and min(out[0][0]) > 0.0
     for f in FIELDS:
         assert np.array_equal(out[0][1][f], out[1][1][f]), f
+
+
+def test_timeout_leaves_open_viscous_loops(require_gpu, monkeypatch):
+    """A neighbour wait of one case gives up (a limit of one tick, as in
+    test_gpu_timeout) while another case is still in its viscous loop and takes
+    more sweeps afterwards: both end their step, and the second one, a single
+    tile that waits for nobody, with the bits of per-stage launches."""
+    print("[gpu-test] time-out beside an open viscous loop", flush=True)
+    out = []
+    for persistent in (True, False):
+        if persistent:
+            monkeypatch.setenv("IFF_PERSISTENT_TIMEOUT_TICKS", "1")
+        else:
+            monkeypatch.delenv("IFF_PERSISTENT_TIMEOUT_TICKS")
+        b = iff.Batch(iff.IF_MIXED)
+        try:
+            b.tune(4, 64, 8, 40)
+            b.persistent(persistent)
+            wide = b.add(_faces(400), _faces(400), 3, dt=0.01, re=100.0, bodies=[iff.circle(6.0, 10.0, 0.5)],
+                         ppe_tol=1e-6, ppe_itermax=80)
+            slow = b.add(_faces(64), _faces(64), 3, bodies=[iff.circle(6.0, 10.0, 2.0)], ad_itermax=300, ppe_tol=1e-9,
+                         ppe_itermax=4000, **SLOW)
+            for k in range(2):
+                b.step(1)
+                assert [b.state(s)[:2] for s in (wide, slow)] == [(0, k + 1), (0, k + 1)]
+                assert b.state(slow)[2]["ad_iters"] == 300 and b.state(slow)[2]["ppe_sweeps"] > 80
+            assert b.state(wide)[2]["div_max"] < 1e300
+            out.append((b.state(slow)[2]["ppe_sweeps"], {f: b.get(slow, f) for f in FIELDS}))
+        finally:
+            b.close()
+    assert out[0][0] == out[1][0]
+    for f in FIELDS:
+        assert np.array_equal(out[0][1][f], out[1][1][f]), f

@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "common.h"
+#include "stages.h"
 
 namespace iff {
 
@@ -147,6 +148,7 @@ private:
     double *d_vals_ = nullptr;     // the persistent solve's residuals, two per tile
     unsigned *d_flags_ = nullptr;  // its per-tile stage counters
     int cap_flags_ = 0;
+    StageCount stages_;            // what they can have counted
     char *d_xb_ = nullptr;         // its strip buffers (CaseDev::xb)
     size_t cap_xb_ = 0, used_xb_ = 0;
     bool pers_ready_ = false;      // the red-black launches are persistent

@@ -854,7 +854,7 @@ if_status Engine::refresh()
             // one aligned store)
             const size_t es = pprec_ == IF_FP64 ? 8 : 4;
             xb_off[k] = used_xb_ + 256 - es;
-            used_xb_ += 256 + align256(3 * (size_t)s.P * s.ny * es);
+            used_xb_ += 256 + align256(kStripBufs * (size_t)s.P * s.ny * es);
         }
     if (used_xb_ > cap_xb_) {
         if (d_xb_) hipFree(d_xb_);
@@ -957,6 +957,7 @@ if_status Engine::refresh()
 // Every tile's and block's stage counter to 0.
 if_status Engine::zero_flags()
 {
+    stages_.used = 0;
     if (cap_flags_ > 0) IFF_HIP(hipMemsetAsync(d_flags_, 0, sizeof(unsigned) * cap_flags_, st_));
     if (used_xb_ > 0) IFF_HIP(hipMemsetAsync(d_xb_, 0xff, used_xb_, st_));  // empty strips
     if (cap_line_ > 0) IFF_HIP(hipMemsetAsync(d_line_flags_, 0, sizeof(unsigned) * cap_line_, st_));
@@ -1038,6 +1039,12 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         if (any_moving_) {
             if_status rc = update_moving();
             if (rc != IF_OK) return rc;
+        }
+        // (a stage is at least one sweep)
+        if ((pers_ready_ || !line_groups_.empty()) && stages_.wraps((unsigned long long)max_ppe_)) {
+            if_status rc = zero_flags();
+            if (rc != IF_OK) return rc;
+            stages_.used = (unsigned long long)max_ppe_;
         }
         launch_step_begin(st_, d_cases_, n);
         launch_source(st_, vprec_, d_cases_, d_tiles_base_, nt_base_);

@@ -762,14 +762,14 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
         };
         // The exchange by polling.  A stage's strips go to one of three buffers
         // laid out as the field, stage g (counted over launches) to buffer
-        // g % 3, and a reader polls the cells themselves: a word of all ones,
+        // strip_of(g), and a reader polls the cells themselves: a word of all ones,
         // which no value has (kHole, a NaN that cap() maps to its neighbour),
         // means not yet written.  So a stage costs a store, its way to the reader
         // and the reader's load; with a counter behind the strips it is a round
         // trip and two barriers more.  FP32 256^2 0.60 -> 0.56 us per sweep,
         // 611^2 0.71 -> 0.64, stretched 2048 x 1024 1.32 -> 1.19; FP64 800^2
         // 1.55 -> 1.27.
-        // Buffer (g + 1) % 3 is emptied during stage g: what it holds, stage
+        // Buffer strip_of(g + 1) is emptied during stage g: what it holds, stage
         // g - 2, has been read, since the neighbours' stage g - 1, sent after
         // that, has arrived in every wave of this block; and it is empty
         // before stage g is sent, so a neighbour that has stage g finds
@@ -777,7 +777,7 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
         constexpr unsigned kHole = 0xffffffffu;
         auto cap = [](unsigned x) { return x < kHole ? x : kHole - 1u; };
         auto strip_buf = [&](unsigned g) {
-            return __builtin_amdgcn_make_buffer_rsrc(uniform_ptr((char *)c.xb + (size_t)(g % 3u) * (size_t)nrec), 0, nrec,
+            return __builtin_amdgcn_make_buffer_rsrc(uniform_ptr((char *)c.xb + (size_t)strip_of(g) * (size_t)nrec), 0, nrec,
                                                      kRsrc3);
         };
         auto send = [&](const __amdgpu_buffer_rsrc_t xo, auto empty) __attribute__((always_inline)) {

@@ -66,3 +66,22 @@ def test_timeout_leaves_open_viscous_loops(require_gpu, monkeypatch):
     assert out[0][0] == out[1][0]
     for f in FIELDS:
         assert np.array_equal(out[0][1][f], out[1][1][f]), f
+
+
+@pytest.mark.parametrize("precision", [iff.IF_FP64, iff.IF_MIXED])
+def test_stage_counters_start_again(require_gpu, precision):
+    """With nearly 2^31 sweeps allowed a step, the stage counters of the
+    persistent sweep are zeroed before every third: the bits of per-stage
+    launches still."""
+    print("[gpu-test] stage counters zeroed between steps", precision, flush=True)
+    out = []
+    for persistent in (True, False):
+        with iff.Case(_faces(300), _faces(210), precision=precision, dt=0.01, re=100.0,
+                      bodies=[iff.circle(6.0, 10.0, 0.5)], ppe_tol=1e-5, ppe_itermax=2**31 - 5000, check_every=30) as c:
+            c.persistent(persistent)
+            st = [c.step(1) for _ in range(4)] + [c.step(5)]
+            assert all(s["persistent_timeouts"] == 0 and s["failed"] == 0 for s in st)
+            out.append(([s["total_ppe_sweeps"] for s in st], {f: c.get(f) for f in FIELDS}))
+    assert out[0][0] == out[1][0]
+    for f in FIELDS:
+        assert np.array_equal(out[0][1][f], out[1][1][f]), f

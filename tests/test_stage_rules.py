@@ -1,5 +1,6 @@
 """The index rules of the persistent sweep's exchange (csrc/stages.h), compiled
-by the host compiler: the rows that its strip loads address."""
+by the host compiler: the rows that its strip loads address, and the strip
+buffers that successive stages use."""
 import os
 import shutil
 import subprocess
@@ -36,3 +37,39 @@ def test_strip_rows_lie_in_the_field(tmp_path):
                             return 1;
                         }
                     }""")
+
+
+def test_stages_in_a_row_never_share_a_strip_buffer(tmp_path):
+    """Steps of random length over many times 2^32 stages, counted in 32 bits as
+    the tiles' counters are: three stages in a row use three buffers, and only
+    zeroed counters go back."""
+    _run(tmp_path, """
+    unsigned long long seed = 12345;
+    int zeroed = 0;
+    for (unsigned long long most : {1ull, 1000ull, 400000ull, 2147483647ull}) {
+        StageCount c;
+        unsigned counter = most < 1000000 ? 0xffffffffu - 100000u : 0;  // the tiles' counters
+        c.used = counter;
+        for (int step = 0; step < 200000; step++) {
+            seed = seed * 6364136223846793005ull + 1442695040888963407ull;
+            const unsigned n = (unsigned)(most - (seed >> 33) % (most / 8 + 1));  // this step's stages
+            if (c.wraps(most)) {
+                counter = 0;
+                zeroed++;
+            }
+            for (unsigned l = 0; l < (n < 64 ? n : 64); l++)
+                for (unsigned g : {counter + l, counter + n - 2 - l}) {
+                    const unsigned a = strip_of(g), b = strip_of(g + 1u), d = strip_of(g + 2u);
+                    if (n > l + 2 && (a == b || b == d || a == d)) {
+                        std::printf("stage %u: buffers %u %u %u\\n", g, a, b, d);
+                        return 1;
+                    }
+                }
+            counter += n;
+            if (counter > c.used) {
+                std::printf("%u stages, at most %llu expected\\n", counter, c.used);
+                return 1;
+            }
+        }
+    }
+    if (zeroed < 4) return 1;""")

@@ -1078,7 +1078,7 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         auto tail = [&]() {
             launch_pressure_bc(st_, d_cases_, n, max_ring_, max_ng_);
             launch_project(st_, vprec_, d_cases_, d_tiles_base_, nt_base_);
-            launch_ghost_vel(st_, vprec_, d_cases_, n, max_ng_, true);
+            launch_ghost_vel(st_, vprec_, d_cases_, n, max_ng_, GhostVel::tail);
             if (any_monitor_) launch_monitor(st_, vprec_, d_cases_, n, d_tiles_base_, nt_base_);
             launch_step_end(st_, d_cases_, n);
         };
@@ -1145,7 +1145,7 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
         do {
             for (int k = 0; k < ad_next && ad_enq < max_ad_; k++, ad_enq++) {
                 launch_ad_sweep(st_, vprec_, d_cases_, d_tiles_base_, nt_base_);
-                launch_ad_finish(st_, vprec_, d_cases_, n);
+                launch_ad_finish(st_, vprec_, d_cases_, n, max_ng_);
             }
             ad_next = kAdMore;
             // ---- P3: faces + RHS

@@ -9,8 +9,14 @@ namespace iff {
 void launch_step_begin(hipStream_t st, const CaseDev *cs, int ncase);
 void launch_source(hipStream_t st, int prec, const CaseDev *cs, const int2 *tiles, int nt);
 void launch_ad_sweep(hipStream_t st, int prec, const CaseDev *cs, const int2 *tiles, int nt);
-void launch_ad_finish(hipStream_t st, int prec, const CaseDev *cs, int ncase);
-void launch_ghost_vel(hipStream_t st, int prec, const CaseDev *cs, int ncase, int max_ng, bool tail = false);
+// ghost cells of the current velocity of every running case, of that of the
+// cases whose step ends (step_tail), or of the new viscous iterate
+enum class GhostVel { running, tail, iterate };
+void launch_ghost_vel(hipStream_t st, int prec, const CaseDev *cs, int ncase, int max_ng,
+                      GhostVel which = GhostVel::running);
+// the end of a viscous iteration: ghost cells (max_ng: of the case with most) and
+// the stopping rule
+void launch_ad_finish(hipStream_t st, int prec, const CaseDev *cs, int ncase, int max_ng);
 void launch_pressure_bc(hipStream_t st, const CaseDev *cs, int ncase, int max_ring, int max_ng);
 bool sweep_variant_ok(int ty, int m);
 void launch_ppe_sweep(hipStream_t st, int prec, int solver, int ty, int m, const CaseDev *cs,

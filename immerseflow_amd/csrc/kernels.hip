@@ -307,21 +307,32 @@ __device__ __forceinline__ void ghost_vel(const CaseDev &c, TS *u, TS *v, int g)
 }
 
 template <typename TS>
-__global__ __launch_bounds__(256) void k_ghost_vel(const CaseDev *cs, bool tail)
+__global__ __launch_bounds__(256) void k_ghost_vel(const CaseDev *cs, GhostVel which)
 {
     const CaseDev &c = cs[blockIdx.y];
     const Ctrl *ct = c.ctrl;
     const int g = blockIdx.x * 256 + threadIdx.x;
-    if (g >= ct->ng || !(tail ? step_tail(ct) : ct->active)) return;
-    ghost_vel(c, fld<TS>(c.u[ct->ad_base]), fld<TS>(c.v[ct->ad_base]), g);
+    if (g >= ct->ng || !(which == GhostVel::tail ? step_tail(ct) : ct->active)) return;
+    int buf = ct->ad_base;
+    if (which == GhostVel::iterate) {
+        if (ct->ad_done) return;
+        buf = 1 - buf;
+    }
+    ghost_vel(c, fld<TS>(c.u[buf]), fld<TS>(c.v[buf]), g);
 }
 
-// The end of a viscous iteration, one block per case: ghost cells of the new
-// iterate (twelve waves), and the stopping rule of ADSolver.cu:315 (the first
-// four, summing the partials in the fixed order).  One launch where the ghost
-// cells and the rule took two: at 64^2 an iteration's kernels last 2 us each,
-// and the launches between them bound the loop.
-constexpr int kAdFinish = 1024, kAdGhost0 = kAdFinish - 256;
+// The end of a viscous iteration, one block per case: the stopping rule of
+// ADSolver.cu:315 (four waves, summing the partials in the fixed order) and, in
+// a block of kAdFinish threads, the ghost cells of the new iterate (the other
+// twelve).  One launch where the ghost cells and the rule took two: at 64^2 an
+// iteration's kernels last 2 us each, and the launches between them bound the
+// loop.  Beyond kAdGhosts ghost cells in any case they go to a launch of their
+// own (launch_ad_finish): one block's twelve waves take about 9 us for every 768
+// of them.  Measured, ms a step of 25 iterations in one launch / in two: 256^2
+// with 320 ghost cells 0.57 / 0.60, 1024^2 with 448 1.12 / 1.14, 512^2 with 576
+// 0.70 / 0.69, 256^2 with 640 0.67 / 0.66, 1024^2 with 6,912 2.22 / 1.15, 4096^2
+// with 27,776 18.6 / 11.0.
+constexpr int kAdFinish = 1024, kAdGhost0 = kAdFinish - 256, kAdGhosts = 512;
 template <typename TS>
 __global__ __launch_bounds__(kAdFinish) void k_ad_finish(const CaseDev *cs, int ncase)
 {
@@ -1599,18 +1610,21 @@ void launch_ad_sweep(hipStream_t st, int prec, const CaseDev *cs, const int2 *ti
         hipLaunchKernelGGL(k_ad_sweep<float>, tile_grid(nt), dim3(256), 0, st, cs, tiles, nt, tile_pad(nt));
 }
 
-void launch_ad_finish(hipStream_t st, int prec, const CaseDev *cs, int ncase)
-{
-    if (prec == IF_FP64) hipLaunchKernelGGL(k_ad_finish<double>, dim3(ncase), dim3(kAdFinish), 0, st, cs, ncase);
-    else hipLaunchKernelGGL(k_ad_finish<float>, dim3(ncase), dim3(kAdFinish), 0, st, cs, ncase);
-}
-
-void launch_ghost_vel(hipStream_t st, int prec, const CaseDev *cs, int ncase, int max_ng, bool tail)
+void launch_ghost_vel(hipStream_t st, int prec, const CaseDev *cs, int ncase, int max_ng, GhostVel which)
 {
     if (max_ng <= 0) return;
     dim3 g((max_ng + 255) / 256, ncase);
-    if (prec == IF_FP64) hipLaunchKernelGGL(k_ghost_vel<double>, g, dim3(256), 0, st, cs, tail);
-    else hipLaunchKernelGGL(k_ghost_vel<float>, g, dim3(256), 0, st, cs, tail);
+    if (prec == IF_FP64) hipLaunchKernelGGL(k_ghost_vel<double>, g, dim3(256), 0, st, cs, which);
+    else hipLaunchKernelGGL(k_ghost_vel<float>, g, dim3(256), 0, st, cs, which);
+}
+
+void launch_ad_finish(hipStream_t st, int prec, const CaseDev *cs, int ncase, int max_ng)
+{
+    const bool apart = max_ng > kAdGhosts;
+    if (apart) launch_ghost_vel(st, prec, cs, ncase, max_ng, GhostVel::iterate);
+    const dim3 block(apart || max_ng <= 0 ? 256 : kAdFinish);
+    if (prec == IF_FP64) hipLaunchKernelGGL(k_ad_finish<double>, dim3(ncase), block, 0, st, cs, ncase);
+    else hipLaunchKernelGGL(k_ad_finish<float>, dim3(ncase), block, 0, st, cs, ncase);
 }
 
 void launch_pressure_bc(hipStream_t st, const CaseDev *cs, int ncase, int max_ring, int max_ng)

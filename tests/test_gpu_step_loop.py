@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import immerseflow_amd as iff
+import oracle_lib as O
 
 pytestmark = pytest.mark.gpu
 
@@ -85,3 +86,24 @@ def test_stage_counters_start_again(require_gpu, precision):
     assert out[0][0] == out[1][0]
     for f in FIELDS:
         assert np.array_equal(out[0][1][f], out[1][1][f]), f
+
+
+@pytest.mark.parametrize("nbody,apart", [(4, False), (9, True)])
+def test_ghost_cells_of_the_iterate(require_gpu, nbody, apart):
+    """The ghost cells of a viscous iterate, set beside the stopping rule or,
+    where a case has more than 512, in a launch of their own: the oracle's
+    fields (same expressions in FP64, other reduction orders: 1e-10 relative)."""
+    print("[gpu-test] ghost cells of the viscous iterate", nbody, flush=True)
+    xf, yf = np.linspace(0.0, 16.0, 161), np.linspace(0.0, 13.0, 131)
+    bodies = [iff.circle(3.0 + 4.5 * (k % 3), 2.5 + 4.0 * (k // 3), 1.4 + 0.01 * k) for k in range(nbody)]
+    prm = dict(dt=0.01, re=100.0, conv_factor=0.5, ubc=1.0, vbc=0.0, ad_itermax=25, ad_tol=1e-6, ppe_solver=1,
+               ppe_omega=1.8, ppe_itermax=200, ppe_tol=1e-9, check_every=10)
+    oc = O.PhysCase(xf, yf, [dict(b, c=b.get("cth", 1.0), s=b.get("sth", 0.0)) for b in bodies], prm)
+    with iff.Case(xf, yf, precision=iff.IF_FP64, bodies=bodies, **prm) as c:
+        assert c.ghosts()[2] == oc.ng and (oc.ng > 512) == apart
+        g, o = c.step(3), oc.step(3)[-1]
+        assert g["ad_iters"] == o[0] and g["ppe_sweeps"] == o[2]
+        for name in FIELDS:
+            ref = getattr(oc, name)
+            err = np.max(np.abs(c.get(name) - ref)) / max(1.0, np.max(np.abs(ref)))
+            assert err <= 1e-10, (name, err)

@@ -22,6 +22,7 @@
 #include "engine.h"
 #include "io.h"
 #include "kernels.h"
+#include "pages.h"
 
 namespace iff {
 
@@ -1532,7 +1533,7 @@ if_status Engine::get_field(int k, int which, double *out, size_t n)
     // The caller's pages, meanwhile: a fresh buffer's are faulted in here by the
     // CPU (large pages where there are any), not one by one when the copy pins
     // them.
-    for (size_t b = 0; b < need * sizeof(double); b += 4096) ((volatile char *)out)[b] = 0;
+    touch_pages(out, need * sizeof(double));
     IFF_HIP(hipMemcpyAsync(out, d, need * sizeof(double), hipMemcpyDeviceToHost, st_));
     IFF_HIP(hipStreamSynchronize(st_));
     return IF_OK;

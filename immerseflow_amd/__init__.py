@@ -339,8 +339,9 @@ class Case:
         _check(_lib().if_case_monitor_sample(self._h), "monitor")
 
     def autotune(self):
-        """Time every Poisson sweep launch shape on the current fields, keep
-        the fastest and choose the check interval (see if_case_autotune).
+        """Time the default and other Poisson sweep launch shapes on the
+        current fields, keep the fastest and choose the check interval (see
+        if_case_autotune).
         Returns the choice as a dict; the case's state is unchanged."""
         r = _abi.IfTuneResult()
         _check(_lib().if_case_autotune(self._h, C.byref(r)), "autotune")

@@ -1267,13 +1267,50 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
     return IF_OK;
 }
 
-// Launch-shape autotuner.  Times the candidate Poisson sweep shapes on the
-// running cases' current fields: each candidate runs a few launches that
-// read the solution and write only the solver's scratch buffers (FP64:
-// launch 0 of a chunk reads p[base] and writes p[base^1]; mixed: launch 1
-// reads e[1] and writes e[0]); the convergence check likewise writes only
-// scratch (the other p buffer, r32, tile partials).  The control blocks are
-// saved before and restored after, and reset to the saved copy before each
+// Where a field lies: its device array, the rectangle of it in the reference
+// layout, and its element type.
+struct FieldAt {
+    void *at;        // element (0, 0) of the pitched array
+    int i0, j0;      // the rectangle's first column and row
+    int w, h;        // its width and height
+    FieldType type;
+};
+
+static bool field_at(const Slot &s, const Ctrl &ct, int vprec, int which, FieldAt *f)
+{
+    const CaseDev &c = s.dev;
+    const FieldType v = vprec == IF_FP64 ? FieldType::f64 : FieldType::f32;
+    switch (which) {
+    case IF_FIELD_U: *f = {c.u[ct.ad_base], 0, 0, s.nx, s.ny, v}; return true;
+    case IF_FIELD_V: *f = {c.v[ct.ad_base], 0, 0, s.nx, s.ny, v}; return true;
+    case IF_FIELD_P: *f = {c.p[ct.ppe_base], 0, 0, s.nx, s.ny, FieldType::f64}; return true;
+    case IF_FIELD_UF: *f = {c.uf[0], 0, 1, s.nx - 1, s.ny - 2, FieldType::f64}; return true;
+    case IF_FIELD_VF: *f = {c.vf[0], 1, 0, s.nx - 2, s.ny - 1, FieldType::f64}; return true;
+    case IF_FIELD_IBLANK: *f = {c.flags, 0, 0, s.nx, s.ny, FieldType::iblank}; return true;
+    case IF_FIELD_FLAGS: *f = {c.flags, 0, 0, s.nx, s.ny, FieldType::flags}; return true;
+    }
+    return false;
+}
+
+// The case's scratch for a dense field: the convective sources' memory (they
+// are formed anew in every step), from the start of sx's allocation to the end
+// of sy's, at least 8 nx ny bytes in either velocity precision.
+static double *dense_scratch(const CaseDev &c, int vprec)
+{
+    const size_t es = vprec == IF_FP64 ? 8 : 4;
+    return (double *)((char *)c.sx - (256 / es - 1) * es);
+}
+
+// Launch-shape autotuner.  Times candidate Poisson sweep shapes, each in the
+// form it will run in, on the running cases' current fields: the shape that
+// the resident set has by default (refresh), the current one, and a fixed
+// list.  Mixed launches read the solution and write only the solver's scratch
+// buffers (launch 1 of a chunk reads e[1] and writes e[0]), as FP64 launches of
+// one stage do (launch 0 reads p[base] and writes p[base^1]) and the convergence
+// checks (the other p buffer, r32, tile partials).  An FP64 persistent launch
+// overwrites p[base] from its second stage on, so that is kept in the convective
+// sources' memory meanwhile (formed anew in every step).  The control blocks
+// are saved before and restored after, and reset to the saved copy before each
 // timed check (a check flips the case's buffer parity), so neither the
 // solution nor the loop state changes.
 if_status Engine::autotune(if_tune_result *out)
@@ -1320,8 +1357,8 @@ if_status Engine::autotune(if_tune_result *out)
     struct Shape {
         int kind, ty, m;
     };
-    // register tiles of 16, 8 and 4 waves at 8, 4 and 2 sweeps per launch,
-    // and the LDS-tiled kernel; shapes a precision lacks are skipped
+    // the list: register tiles of 16, 8 and 4 waves at 8, 4 and 2 sweeps per
+    // launch, and the LDS-tiled kernel; shapes a precision lacks are skipped
     static const Shape cands[] = {{4, 64, 8}, {4, 96, 8}, {4, 92, 9}, {4, 88, 10}, {4, 32, 8},
                                   {4, 48, 4}, {4, 64, 4}, {4, 80, 4}, {3, 32, 8}, {3, 48, 8},
                                   {3, 64, 8}, {3, 32, 4}, {3, 48, 4}, {3, 24, 2}, {2, 16, 4},
@@ -1341,39 +1378,40 @@ if_status Engine::autotune(if_tune_result *out)
     };
     const Shape keep{sweep_kind, sweep_ty, sweep_m};
     const bool keep_auto = shape_auto;
-    // each candidate is timed over its own tile table: refresh() must not
-    // replace the candidate's shape by the FP64 default while tuning
-    shape_auto = false;
-    Shape best = keep;
-    double best_ns = 1e300;
-    int ncand = 0;
-    for (const Shape &c : cands) {
-        if (c.kind >= 2 && !reg_variant_ok(pprec_, reg_waves(c.kind), c.ty, c.m)) continue;
-        sweep_kind = c.kind;
-        sweep_ty = c.ty;
-        sweep_m = c.m;
-        rc = refresh();
-        if (rc != IF_OK) break;
-        // the launch below covers exactly the candidate's tiles
-        {
-            const int wo = c.kind == 1 ? stream_out_cols(c.m) : c.kind >= 2 ? reg_out_cols(c.m) : 0;
-            int want = 0;
-            for (int id : order_) {
-                const Slot &sl = *slots_[id];
-                want += (wo > 0 ? (sl.NX + wo - 1) / wo : sl.ntx) * ((sl.NY + c.ty - 1) / c.ty);
-            }
-            if (want != nt_sweep_ || tiles_sweep_ty_ != c.ty) {
-                rc = fail(IF_ERR_STATE, "autotune: tile table does not match the candidate shape");
-                break;
-            }
+    auto same = [](const Shape &a, const Shape &b) { return a.kind == b.kind && a.ty == b.ty && a.m == b.m; };
+    // FP64: the current pressures to the cases' scratch, or back from it
+    auto pressures = [&](bool back) -> if_status {
+        for (int id : order_) {
+            const Slot &sl = *slots_[id];
+            FieldAt f;
+            (void)field_at(sl, ctl[id], vprec_, IF_FIELD_P, &f);
+            double *d = dense_scratch(sl.dev, vprec_);
+            if (back)
+                launch_unpack(st_, f.type, f.at, sl.P, f.i0, f.j0, f.w, f.h, d);
+            else
+                launch_pack(st_, f.type, f.at, sl.P, f.i0, f.j0, f.w, f.h, d);
         }
+        IFF_HIP(hipGetLastError());
+        return IF_OK;
+    };
+    if (pprec_ == IF_FP64) rc = pressures(false);
+    // one shape (after refresh(), over its own tile table): ns per cell and sweep
+    auto time_shape = [&](const Shape &c, double *ns) -> if_status {
+        // the launch below covers exactly the candidate's tiles
+        const int wo = c.kind == 1 ? stream_out_cols(c.m) : c.kind >= 2 ? reg_out_cols(c.m) : 0;
+        int want = 0;
+        for (int id : order_) {
+            const Slot &sl = *slots_[id];
+            want += (wo > 0 ? (sl.NX + wo - 1) / wo : sl.ntx) * ((sl.NY + c.ty - 1) / c.ty);
+        }
+        if (want != nt_sweep_ || tiles_sweep_ty_ != c.ty)
+            return fail(IF_ERR_STATE, "autotune: tile table does not match the candidate shape");
         // a shape that will run as persistent chunks is timed that way, over
-        // 32 stages (a typical check interval); it writes only the scratch
-        // error buffers and advances the stage counters of every tile alike.
-        // FP64 shapes are timed per stage: an FP64 persistent launch's
-        // second stage would overwrite the solve's current pressure.
-        const bool pc = pprec_ != IF_FP64 && pers_ready_;
-        const int kp = 32 * c.m;
+        // 32 stages (a typical check interval; FP64, two to three times as
+        // long a sweep: 96 sweeps); it advances the stage counters of every
+        // tile alike
+        const bool pc = pers_ready_;
+        const int kp = pprec_ == IF_FP64 ? 96 / c.m * c.m : 32 * c.m;
         const int s0 = pprec_ == IF_FP64 ? 0 : c.m;
         auto timed = [&]() {
             if (pc)
@@ -1392,23 +1430,52 @@ if_status Engine::autotune(if_tune_result *out)
         for (int r = 0; r < reps; r++) timed();
         (void)hipEventRecord(e1, st_);
         float ms = 0.f;
-        if (!elapsed(&ms)) {
-            rc = fail(IF_ERR_HIP, "autotune: timing failed");
-            break;
-        }
-        const double ns = 1e6 * (double)ms / (reps * (double)(pc ? kp : c.m) * cells);
-        ncand++;
-        if (ns < best_ns) {
+        if (!elapsed(&ms)) return fail(IF_ERR_HIP, "autotune: timing failed");
+        *ns = 1e6 * (double)ms / (reps * (double)(pc ? kp : c.m) * cells);
+        return IF_OK;
+    };
+    Shape best = keep, dflt = keep;
+    double best_ns = 1e300;
+    int ncand = 0;
+    // the default first.  Another shape has to beat it by more than such
+    // timings differ from run to run: the default goes on following the
+    // resident set, another one stays as it is
+    constexpr double kClear = 0.99;
+    if (rc == IF_OK) {
+        shape_auto = true;
+        rc = refresh();
+    }
+    if (rc == IF_OK) {
+        best = dflt = Shape{sweep_kind, sweep_ty, sweep_m};
+        rc = time_shape(dflt, &best_ns);
+    }
+    // refresh() must not replace a candidate's shape by the default
+    shape_auto = false;
+    auto candidate = [&](const Shape &c) {
+        sweep_kind = c.kind;
+        sweep_ty = c.ty;
+        sweep_m = c.m;
+        rc = refresh();
+        double ns = 0.0;
+        if (rc == IF_OK) rc = time_shape(c, &ns);
+        if (rc == IF_OK && ns < (same(best, dflt) ? kClear : 1.0) * best_ns) {
             best_ns = ns;
             best = c;
         }
+    };
+    if (rc == IF_OK && !same(keep, dflt)) candidate(keep);
+    for (const Shape &c : cands) {
+        if (rc != IF_OK) break;
+        if (c.kind >= 2 && !reg_variant_ok(pprec_, reg_waves(c.kind), c.ty, c.m)) continue;
+        ncand++;
+        if (!same(c, dflt) && !same(c, keep)) candidate(c);
     }
     double check_sweeps = 0.0;
     if (rc == IF_OK) {
         sweep_kind = best.kind;
         sweep_ty = best.ty;
         sweep_m = best.m;
-        shape_auto = false;
+        shape_auto = same(best, dflt);
         rc = refresh();
     }
     if (rc == IF_OK) {
@@ -1422,13 +1489,17 @@ if_status Engine::autotune(if_tune_result *out)
         if (!elapsed(&ms)) rc = fail(IF_ERR_HIP, "autotune: timing failed");
         else check_sweeps = 1e6 * (double)ms / kReps / (best_ns * cells);
     }
-    // restore the loop state
+    // restore the solution and the loop state
+    if (pprec_ == IF_FP64) {
+        const if_status back = pressures(true);
+        if (rc == IF_OK) rc = back;
+    }
     const bool restored =
         hipMemcpyAsync(d_ctrl_, saved, sizeof(Ctrl) * nall, hipMemcpyDeviceToDevice, st_) == hipSuccess &&
         hipStreamSynchronize(st_) == hipSuccess;
     cleanup();
     if (!restored) return fail(IF_ERR_HIP, "autotune: control-block restore failed");
-    if (rc == IF_OK && pprec_ != IF_FP64) rc = check_barrier();
+    if (rc == IF_OK) rc = check_barrier();
     if (rc != IF_OK) {
         sweep_kind = keep.kind;
         sweep_ty = keep.ty;
@@ -1446,7 +1517,7 @@ if_status Engine::autotune(if_tune_result *out)
         const double k = std::sqrt(2.0 * S * std::max(check_sweeps, 0.0));
         const int m = best.m;
         int K = (int)std::lround(k / m) * m;
-        K = std::max(std::max(4, m), std::min(1024, K));
+        K = std::max(std::max(4, m), std::min(1024 / m * m, K));
         check_k = K;
     }
     mark_dirty();
@@ -1474,40 +1545,6 @@ if_status Engine::slot_state(int k, int *state, int *steps_done, if_step_stats *
     if (steps_done) *steps_done = s->last.steps;
     if (st) *st = s->last;
     return IF_OK;
-}
-
-// Where a field lies: its device array, the rectangle of it in the reference
-// layout, and its element type.
-struct FieldAt {
-    void *at;        // element (0, 0) of the pitched array
-    int i0, j0;      // the rectangle's first column and row
-    int w, h;        // its width and height
-    FieldType type;
-};
-
-static bool field_at(const Slot &s, const Ctrl &ct, int vprec, int which, FieldAt *f)
-{
-    const CaseDev &c = s.dev;
-    const FieldType v = vprec == IF_FP64 ? FieldType::f64 : FieldType::f32;
-    switch (which) {
-    case IF_FIELD_U: *f = {c.u[ct.ad_base], 0, 0, s.nx, s.ny, v}; return true;
-    case IF_FIELD_V: *f = {c.v[ct.ad_base], 0, 0, s.nx, s.ny, v}; return true;
-    case IF_FIELD_P: *f = {c.p[ct.ppe_base], 0, 0, s.nx, s.ny, FieldType::f64}; return true;
-    case IF_FIELD_UF: *f = {c.uf[0], 0, 1, s.nx - 1, s.ny - 2, FieldType::f64}; return true;
-    case IF_FIELD_VF: *f = {c.vf[0], 1, 0, s.nx - 2, s.ny - 1, FieldType::f64}; return true;
-    case IF_FIELD_IBLANK: *f = {c.flags, 0, 0, s.nx, s.ny, FieldType::iblank}; return true;
-    case IF_FIELD_FLAGS: *f = {c.flags, 0, 0, s.nx, s.ny, FieldType::flags}; return true;
-    }
-    return false;
-}
-
-// The case's scratch for a dense field: the convective sources' memory (they
-// are formed anew in every step), from the start of sx's allocation to the end
-// of sy's, at least 8 nx ny bytes in either velocity precision.
-static double *dense_scratch(const CaseDev &c, int vprec)
-{
-    const size_t es = vprec == IF_FP64 ? 8 : 4;
-    return (double *)((char *)c.sx - (256 / es - 1) * es);
 }
 
 // Device field -> reference layout (double).  Packed on the device, so that

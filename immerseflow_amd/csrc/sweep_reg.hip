@@ -37,7 +37,10 @@ bool reg_variant_ok(int prec, int waves, int ty, int m)
         return (m == 4 && (ty == 48 || ty == 64 || ty == 80)) ||
                (m == 8 && (ty == 32 || ty == 64 || (ty == 96 && prec != IF_FP64))) ||
                (prec != IF_FP64 && ((m == 9 && ty == 92) || (m == 10 && ty == 88) || (m == 11 && ty == 84) ||
-                                    (m == 12 && ty == 80)));
+                                    (m == 12 && ty == 80))) ||
+               // the default's low tiles (reg_auto_shape)
+               (m == 12 && ty == 16) || (prec == IF_FP64 && m == 8 && ty == 48) ||
+               (prec != IF_FP64 && ((m == 16 && ty == 32) || (m == 12 && ty == 48)));
     return false;
 }
 
@@ -59,22 +62,22 @@ void launch_ppe_sweep_reg(hipStream_t st, int prec, int waves, int ty, int m, co
     IFF_RG(T, 8, 4, 32) IFF_RG(T, 8, 4, 48) IFF_RG(T, 8, 4, 64)                           \
     IFF_RG(T, 8, 8, 32) IFF_RG(T, 8, 8, 48) IFF_RG(T, 8, 8, 64)                           \
     IFF_RG(T, 16, 4, 48) IFF_RG(T, 16, 4, 64) IFF_RG(T, 16, 4, 80) IFF_RG(T, 16, 8, 32) IFF_RG(T, 16, 8, 64)
-    // (the default shapes' own come last in each list: they run per stage
-    // only after a neighbour wait timed out)
+    // (the default's low tiles come last in each list: without the persistent
+    // form, mostly after a neighbour wait timed out)
     if (prec == IF_FP64) {
         IFF_RG_ALL(double)
         IFF_RG(double, 16, 12, 16)
         IFF_RG(double, 16, 8, 48)
     } else {
         IFF_RG_ALL(float)
-        IFF_RG(float, 16, 12, 16)
-        IFF_RG(float, 16, 16, 32)
-        IFF_RG(float, 16, 12, 48)
         IFF_RG(float, 16, 8, 96)
         IFF_RG(float, 16, 9, 92)
         IFF_RG(float, 16, 10, 88)
         IFF_RG(float, 16, 11, 84)
         IFF_RG(float, 16, 12, 80)
+        IFF_RG(float, 16, 12, 16)
+        IFF_RG(float, 16, 16, 32)
+        IFF_RG(float, 16, 12, 48)
     }
 #undef IFF_RG_ALL
 #undef IFF_RG

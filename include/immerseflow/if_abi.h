@@ -171,7 +171,7 @@ typedef struct {
     double sweep_ns;        /* its time per interior cell-sweep (all running cases) */
     double check_sweeps;    /* one convergence check, in sweeps of that shape */
     int typical_sweeps;     /* sweeps per solve the check interval was chosen for (0: none yet) */
-    int candidates;         /* shapes timed */
+    int candidates;         /* shapes of the list that the precision has */
 } if_tune_result;
 
 typedef struct if_case if_case;
@@ -246,9 +246,10 @@ if_status if_case_ghosts(if_case *c, int32_t *out, if_ghost *recs,
  * registers), tile height 16/32/48 rows, 1, 2 or 4 sweeps per launch;
  * kernel 3: the same with eight wave64s per tile, tile height 24/40/56
  * (2 sweeps per launch), 32/48/64 (4) or 32/48/64 (8); kernel 4: sixteen
- * wave64s per tile, tile height 48/64/80 (4 sweeps per launch) or 32/64/96
- * (8), and in mixed precision only also 96 (8), 92 (9), 88 (10), 84 (11)
- * and 80 (12; the tile computes 128 x 128 cells, stores 128 - 4m of them in
+ * wave64s per tile, tile height 48/64/80 (4 sweeps per launch), 32/64 (8) or
+ * 16 (12), in FP64 also 48 (8), and in mixed precision also 96 (8), 92 (9),
+ * 88 (10), 84 (11), 48 and 80 (12) and 32 (16; the tiles of 80 rows and more
+ * compute 128 x 128 cells, store 128 - 4m of them in
  * each direction and recomputes the rest).  Several red-black sweeps per launch is
  * temporal blocking; check_every is the number of sweeps between
  * convergence checks.  Results do not depend on the kernel, the tile
@@ -256,9 +257,9 @@ if_status if_case_ghosts(if_case *c, int32_t *out, if_ghost *recs,
  * 4 in a shape that follows its grids: the first of a list of persistent
  * shapes whose tiles fit on the device in one launch, low tiles with deep
  * stages for small grids (mixed: 16 rows x 12 sweeps, 32 x 16, 48 x 12, 64 x 8,
- * 96 x 8; FP64: 16 x 12, 32 x 8, 48 x 8, 64 x 8, 80 x 4; some of these shapes
- * are the library's own and not accepted here); where none fits, launches of
- * one stage: mixed 88 rows x 10 sweeps or 64 x 8, FP64 kernel 3, 32 x 4. */
+ * 96 x 8; FP64: 16 x 12, 32 x 8, 48 x 8, 64 x 8, 80 x 4); where none fits,
+ * launches of one stage: mixed 88 rows x 10 sweeps or 64 x 8, FP64 kernel 3,
+ * 32 x 4. */
 if_status if_case_tune(if_case *c, int kernel, int tile_y, int sweeps_per_launch,
                        int check_every);
 /* Launch mode of the Poisson sweeps (no counterpart in the reference,
@@ -317,11 +318,13 @@ if_status if_case_monitor_sample(if_case *c);
  * overlap on one GPU share that array and race: serialise them. */
 if_status if_case_monitor_sample_noalloc(if_case *c);
 /* Autotuner (no counterpart in the reference, whose loop is fixed):
- * times every Poisson sweep launch shape of if_case_tune on the case's
- * current fields (a few launches each, on the solver's scratch buffers;
- * the solution and the loop state are left as they were; a shape that
- * would run as persistent chunks is timed as one) and keeps the
- * fastest.  The check interval is then chosen from the measured cost of a
+ * times the shape the case has by default, its current one and a list of
+ * sixteen others on the case's current fields (a few launches each; the
+ * solution and the loop state are left as they were; a shape that would
+ * run as persistent chunks is timed as one) and keeps the fastest.  Where the
+ * default is not beaten by more than 1 % it stays the default, and follows the
+ * resident set from then on; another shape stays as if set by if_case_tune.
+ * The check interval is then chosen from the measured cost of a
  * convergence check c (in sweeps) and the sweep count S of the last solve:
  * checking every K sweeps costs about S c / K checks plus K / 2 sweeps of
  * overshoot, least at K = sqrt(2 S c) (rounded to whole launches, 4..1024).

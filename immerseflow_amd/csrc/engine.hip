@@ -690,7 +690,8 @@ void Engine::enqueue_sweeps(int K, int M, bool any_rb, bool any_jac, bool any_li
 // topology (same kernels, same count) updates the instantiated graph in
 // place (hipGraphExecUpdate: new kernel arguments and launch sizes); only
 // a different topology destroys it and instantiates a new one.  The stream
-// is idle whenever this runs (every step ends with a synchronisation).
+// is idle whenever this runs: every step ends with a synchronisation, and the
+// time-out fallback within a step waits for it.
 if_status Engine::capture_sweeps(int K, int M, bool any_rb, bool any_jac, bool any_line, bool pers, bool lpers,
                             bool stamp)
 {
@@ -1186,6 +1187,9 @@ if_status Engine::step(int nsteps, int *finished, if_step_stats *agg)
                 launch_ppe_rearm(st_, d_cases_, n);
                 graph = use_graphs;
                 if (graph) {
+                    // (beside a Jacobi case the chunks are graph launches, and one
+                    // may be queued behind the check that was seen)
+                    IFF_HIP(hipStreamSynchronize(st_));
                     rc = capture_sweeps(K, M, any_rb, any_jac, any_line, false, false, timing);
                     if (rc != IF_OK) return rc;
                 }

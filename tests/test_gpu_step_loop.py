@@ -107,3 +107,28 @@ def test_ghost_cells_of_the_iterate(require_gpu, nbody, apart):
             ref = getattr(oc, name)
             err = np.max(np.abs(c.get(name) - ref)) / max(1.0, np.max(np.abs(ref)))
             assert err <= 1e-10, (name, err)
+
+
+def test_timeout_captures_its_chunk_again(require_gpu, monkeypatch):
+    """Beside a Jacobi case a chunk is several launches, replayed from a graph
+    that holds the persistent one.  A forced time-out captures it anew within the
+    step: the Jacobi case, which waits for nobody, is solved again from its start
+    and ends like the others at its stop level, and later steps replay the new
+    graph."""
+    print("[gpu-test] time-out with a captured chunk", flush=True)
+    monkeypatch.setenv("IFF_PERSISTENT_TIMEOUT_TICKS", "1")
+    b = iff.Batch(iff.IF_MIXED)
+    try:
+        b.tune(4, 64, 8, 40)
+        wide = b.add(_faces(400), _faces(400), 9, dt=0.01, re=100.0, bodies=[iff.circle(6.0, 10.0, 0.5)],
+                     ppe_tol=1e-5, ppe_itermax=20000)
+        jac = b.add(_faces(64), _faces(64), 9, dt=0.01, re=100.0, bodies=[iff.circle(6.0, 10.0, 2.0)],
+                    ppe_solver=iff.IF_PPE_JACOBI, ppe_omega=1.0, ppe_tol=1e-4, ppe_itermax=40000)
+        for k in range(6):
+            b.step(1)
+            for s, tol in ((wide, 1e-5), (jac, 1e-4)):
+                state, steps, st = b.state(s)
+                assert (state, steps) == (0, k + 1) and st["failed"] == 0
+                assert st["ppe_res"] <= tol and st["ppe_sweeps"] > 0 and st["div_max"] <= 1.01 * tol
+    finally:
+        b.close()

@@ -180,7 +180,7 @@ struct CaseDev {
     double *uf[2], *vf[2];         // face velocities: [0] = U^n, [1] = U*
     double *p[2], *rhs;
     float *e[2], *r32;             // mixed Poisson error / residual
-    float *w32;                    // mixed: each cell's FP32 SOR weight om / sa (0: not updated), formed once per step
+    float *w32;                    // mixed: each cell's FP32 SOR weight om / sa (0: not updated; k_weights32)
     float *wtab;                   // mixed on a grid whose FP32 coefficients are each one value: the SOR
                                    // weight of each of the 64 patterns of flag bits 0-5; null: per-cell
                                    // weights (w32)

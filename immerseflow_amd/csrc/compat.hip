@@ -271,7 +271,10 @@ __global__ void kc_pbc(int nx, int ny, double *p)
 constexpr int kOneCells = 8192;       // 16 waves x 512 cells
 constexpr int kOneReg = 4096;         // 8 waves, 256 registers a lane
 constexpr int kOneQ = 8;              // cells per lane
-constexpr int kOneIters = 16384;      // Poisson iterations per launch: bounds a launch to about 10 ms
+// iterations per launch at most: a Poisson launch lasts up to 18 ms at 52 x 52
+// cells and 45 ms at 90 x 91; an ADsolver call is one launch, 6.2 and 24 us an
+// iteration (calls that allow more iterations than this run launch by launch)
+constexpr int kOneIters = 16384;
 constexpr size_t kOneLds = 160 * 1024;
 
 // Lane l's value plus that of lane l ^ h for h = 32, 16, ..: in lane 0 the
@@ -353,9 +356,11 @@ constexpr int kOneStride = kOneReg + 1;
 // stores p_k from registers.  Everything a cell needs is in registers (8
 // waves, 256 registers a lane) and the loop has no branch per cell: a ring
 // cell, or one past the end, has zero coefficients, reads an interior cell's
-// neighbours and stores to a spare cell.  Bound by its FP64 instructions (17
-// per cell): the deck's 14,755 iterations on 52 x 52 cells take 16.0 ms (312
-// launch by launch, 27.8 with a branch per cell).
+// neighbours and stores to a spare cell.  The deck's 14,807 iterations on 52 x
+// 52 cells take 16.1 ms (312 launch by launch, 27.8 with a branch per cell): of an
+// iteration's 2,600 cycles the FP64 instructions (17 per cell) are 1,090 on the
+// SIMDs that hold two of the six waves, the rest is the chain of the fold, its
+// LDS write, the barrier and the second fold.
 __global__ __launch_bounds__(512) void kc_ppe_one(int nx, int ny, const double *vx, const double *vy, double *p,
                                                   int iter0, int itermax, int most, double tol, double *out)
 {

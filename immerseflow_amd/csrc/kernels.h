@@ -67,7 +67,7 @@ void launch_line_pers(hipStream_t st, int prec, int B, const CaseDev *cs, const 
 void launch_ppe_check(hipStream_t st, int prec, const CaseDev *cs, int ncase, const int2 *tiles,
                       int nt, int K, GridBar *bar);
 void launch_ppe_rearm(hipStream_t st, const CaseDev *cs, int ncase);
-// zebra line SOR: the per-step factors (pivots, c', 1/m) of every line
+// zebra line SOR: the factors (pivots, c', 1/m) of every line
 // case, then one sweep (both colours) at chunk position s
 void launch_line_factor(hipStream_t st, int prec, const CaseDev *cs, int ncase, int max_ny);
 void launch_weights32(hipStream_t st, const CaseDev *cs, int ncase, int max_n);

@@ -773,13 +773,12 @@ __global__ __launch_bounds__(256) void k_jacobi(const CaseDev *cs, const int2 *t
 // the separators' Schur complement is solved by cyclic reduction across
 // the lanes (shuffles), and each segment adds its separators' share.  The
 // factors depend on the flags and the metric only: k_line_factor forms
-// them once per step, in the segment layout [plane][t][lane] that a
-// lane-per-segment loop reads coalesced.  The sweep kernel stages the
+// them once for a resident set (every step with moving bodies), in the
+// segment layout [plane][t][lane] that a lane-per-segment loop reads coalesced.  The sweep kernel stages the
 // row's right side into LDS in that layout (coalesced row loads, a
 // transposing store), runs the lanes' recurrences there, and relaxes and
 // stores the row with coalesced accesses.
-// The factors of every interior row of every line-solve case (once per
-// step): lane k forms segment k's pivots r = 1/den, -l r, -u r and spikes
+// The factors of every interior row of every line-solve case: lane k forms segment k's pivots r = 1/den, -l r, -u r and spikes
 // h, q; lanes 0..m-1 (m = S - 1) the separators' -l, -u and the cyclic
 // reduction's multipliers and final reciprocals.  Operation for operation
 // the oracle's line_factor_row.
@@ -1394,8 +1393,9 @@ __global__ void k_ppe_rearm(const CaseDev *cs, int ncase)
 
 // The FP32 red-black SOR weight of every interior cell, om / sa over the
 // open faces (sor_weight, the expression every FP32 sweep kernel uses), 0
-// for a cell the sweep keeps (not fluid, or no open face).  Once per step,
-// after the flags are final: the register-tile kernel loads it instead of
+// for a cell the sweep keeps (not fluid, or no open face).  Once for a
+// resident set (every step with moving bodies), after the flags are final: the
+// register-tile kernel loads it instead of
 // forming it from the flags on every launch.  One block per row.  On a grid
 // whose coefficients are one value per axis (wtab) the weight depends on
 // the flags alone: the first block also writes K = w ax of each pattern of

@@ -338,7 +338,8 @@ void k_rbsor_reg(const CaseDev *cs, const int2 *tiles, int ntiles, int ntiles_pa
     //      batch mixing uniform and stretched grids).
     RegTile<T, NRW> R;
     int lf[NRW];  // FP64: flags, slot a in bits 0-7, slot b in bits 8-15
-    // FP32: the cells' weights om / sa, formed once per step (k_weights32),
+    // FP32: the cells' weights om / sa (k_weights32: once for a resident set,
+    // every step with moving bodies),
     // or on a grid with one value per coefficient the weight of the cell's
     // flag pattern: lane q holds the table's entry q, and each cell reads
     // its entry across the wave (ds_bpermute)

@@ -348,7 +348,10 @@ if_status if_case_byte_model(if_case *c, double *sweep_bytes_per_cell,
  * Many independent cases advanced together: every kernel launch covers the
  * tiles of all resident cases; per-case device flags end each case's
  * iterations independently; per-case reductions run in a fixed order, so a
- * case's result does not depend on what else is resident. */
+ * case's result does not depend on what else is resident.  hbm_budget bounds
+ * the sum of the cases' footprints (0: no bound); the library's own tables and
+ * the exchange buffers of persistent launches come on top (at most about 35 MB,
+ * whatever the cases). */
 if_status if_batch_create(int precision, size_t hbm_budget, if_batch **out);
 void if_batch_destroy(if_batch *b);
 /* Admit a case that should run nsteps steps; IF_ERR_BUDGET when its

@@ -322,8 +322,9 @@ if_status if_case_monitor_sample_noalloc(if_case *c);
  * sixteen others on the case's current fields (a few launches each; the
  * solution and the loop state are left as they were; a shape that would
  * run as persistent chunks is timed as one) and keeps the fastest.  Where the
- * default is not beaten by more than 1 % it stays the default, and follows the
- * resident set from then on; another shape stays as if set by if_case_tune.
+ * default is not beaten (a persistent one: by more than 1 %) it stays the
+ * default, and follows the resident set from then on; another shape stays as if
+ * set by if_case_tune.
  * The check interval is then chosen from the measured cost of a
  * convergence check c (in sweeps) and the sweep count S of the last solve:
  * checking every K sweeps costs about S c / K checks plus K / 2 sweeps of

@@ -42,8 +42,8 @@ static void pers_one(hipStream_t st, const CaseDev *cs, const int2 *tiles, int n
 }
 
 // the shapes with a persistent form: (waves, sweeps per stage, tile_y,
-// rows per wave), FP32 and FP64; the last ones of each are the default
-// shapes' own (reg_auto_shape)
+// rows per wave), FP32 and FP64; the last ones of each only for the
+// default's low tiles (reg_auto_shape)
 #define IFF_PERS_SHAPES32(X)                                                                                \
     X(float, 16, 8, 96, 8) X(float, 16, 8, 64, 6) X(float, 16, 4, 48, 4) X(float, 8, 8, 32, 8) X(float, 8, 4, 32, 6) \
     X(float, 16, 12, 16, 4) X(float, 16, 16, 32, 6) X(float, 16, 12, 48, 6)
